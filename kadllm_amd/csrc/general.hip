@@ -10,9 +10,9 @@
 // of the reference's torch path in fp32: the per-token recurrence of
 // ops.py:152-158 and one softmax over the prefix and causal suffix keys
 // (equal to the two-partition LSE merge of ops.py:229-249,340).
-//
-// Both are one wave per unit of work; neither is meant for the headline
-// shapes, which the specialised kernels serve.
+
+#include <type_traits>
+#include <utility>
 
 #include "kad_common.h"
 
@@ -31,100 +31,254 @@ __device__ __forceinline__ void store_from_float(void* p, int64_t i, int dtype, 
 __device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 // ---------------------------------------------------------------------------
-// Gated delta recurrence, one wave per (sequence n, value head hv, 64 value
-// columns).  The columns of the state evolve independently under
+// Gated delta recurrence.  The value columns of the state evolve independently under
 //   S <- S e^{g_t};  u = beta_t (v_t - S^T k_t);  S <- S + k_t u^T;  o_t = S^T q_t
-// so lane j keeps column v0 + j of S (K values) in registers for all T tokens.
-// q and k of each token are L2-normalised in fp32 as the reference does
-// (q / sqrt(sum q^2 + 1e-6) * scale, ops.py:147-148) and shared through LDS.
-template <int KMAX>
-__global__ __launch_bounds__(64) void gdn_recurrent_kernel(
-    const void* __restrict__ q, const void* __restrict__ k, const void* __restrict__ v,
-    int64_t ld_qk, int64_t ld_v, int qkv_dtype, const void* __restrict__ gdecay,
+// A column is held by 16 consecutive lanes (K / 16 values each, in registers
+// for all T tokens), a workgroup of 4 waves holds 16 columns of one
+// (sequence, value head).  A token is one dependent step, so what bounds the
+// kernel is the step's length: both dot products (with k, and with q on the
+// state before the update, o_t = e^{g} S^T q + (k.q) u) are reduced together
+// on DPP permutes within the 16-lane row, and everything that needs no state
+// -- the L2 norms (q / sqrt(sum q^2 + 1e-6) * scale, ops.py:147-148), k.q,
+// e^g -- is computed for kTile tokens at a time by all lanes, while the next
+// tile's loads are in flight.  16 lanes a column give one wave per SIMD at
+// 2 sequences x 16 heads x 128 columns, where one lane a column left 64 waves
+// (777 fp32 tokens there: 5,970 -> 144 us, 0.19 us a token).
+constexpr int kTile = 16;   // tokens staged at a time, one per 16-lane row
+constexpr int kCols = 16;   // state columns per workgroup
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_row(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL,
+                                                               0xF, 0xF, true));
+}
+// sum over the 16 lanes of a row, in all of them
+__device__ __forceinline__ float row16_sum(float x) {
+  x += dpp_row<0xB1>(x);   // quad_perm [1, 0, 3, 2]
+  x += dpp_row<0x4E>(x);   // quad_perm [2, 3, 0, 1]
+  x += dpp_row<0x141>(x);  // row_half_mirror
+  x += dpp_row<0x140>(x);  // row_mirror
+  return x;
+}
+
+// f(0) .. f(15) with the index a compile-time constant
+template <typename F, int... I>
+__device__ __forceinline__ void unroll16_at(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <typename F>
+__device__ __forceinline__ void unroll16(F&& f) {
+  unroll16_at(f, std::make_integer_sequence<int, 16>{});
+}
+
+// KV values of a column per lane (K <= 16 KV); lane p of a column owns the
+// rows c * 16 VW + p VW + e (VW = min(KV, 4)), so that a row of k or q is read
+// from LDS as consecutive 16-byte words.
+template <typename TIN, int KV>
+__global__ __launch_bounds__(256) void gdn_recurrent_kernel(
+    const TIN* __restrict__ q, const TIN* __restrict__ k, const TIN* __restrict__ v,
+    int64_t ld_qk, int64_t ld_v, const void* __restrict__ gdecay,
     int gate_dtype, const void* __restrict__ beta, int beta_dtype, int64_t ld_gate,
-    const void* __restrict__ init, int state_dtype, int beams_per_state, void* __restrict__ out,
+    const void* __restrict__ init, int state_dtype, int beams_per_state, TIN* __restrict__ out,
     int64_t ld_out, float* __restrict__ final_state, int T, int H, int HV, int K, int V,
-    float scale, int nvt) {
-  __shared__ float qs[KMAX], ks[KMAX];
-  const int lane = threadIdx.x;
-  const int64_t bid = blockIdx.x;
-  const int vt = (int)(bid % nvt);
-  const int64_t nh = bid / nvt;
+    float scale, int nvt, int wide) {
+  constexpr int VW = KV < 4 ? KV : 4, NC = KV / VW, KP = 16 * KV;
+  constexpr int kQK = kTile * KP;   // floats of a tile's k (or q) rows
+  constexpr int kStage = 2 * kQK > KP * (kCols + 1) ? 2 * kQK : KP * (kCols + 1);
+  typedef float vec_t __attribute__((ext_vector_type(VW)));
+  // two tiles of [k | q] rows; the state passes through the first on its way
+  // in and out (coalesced rows of 16 columns)
+  __shared__ __attribute__((aligned(16))) float rows[2][kStage];
+  __shared__ __attribute__((aligned(16))) float scal[2][kTile][4];  // e^g, beta, k.q
+  __shared__ float vs[2][kTile][kCols + 1], os[2][kTile][kCols + 1];
+  const int tid = threadIdx.x, p = tid & 15, g16 = tid >> 4;
+  const int vt = (int)(blockIdx.x % (unsigned)nvt);
+  const int64_t nh = blockIdx.x / (unsigned)nvt;
   const int hv = (int)(nh % HV);
   const int64_t n = nh / HV;
   const int h = hv / (HV / H);
-  const int j = vt * 64 + lane;
-  const bool active = j < V;
+  const int v0 = vt * kCols, ncol = min(kCols, V - v0);
 
-  float s[KMAX];
-  const int64_t sbase = init ? (((n / beams_per_state) * HV + hv) * (int64_t)K) * V : 0;
+  float s[KV];
+  const int64_t sbase =
+      init ? (((n / beams_per_state) * HV + hv) * (int64_t)K) * V + v0 : 0;
 #pragma unroll
-  for (int i = 0; i < KMAX; ++i)
-    s[i] = (init && active && i < K) ? load_as_float(init, sbase + (int64_t)i * V + j, state_dtype)
-                                     : 0.f;
-
-  for (int t = 0; t < T; ++t) {
-    const int64_t row = n * T + t;
-    float sq = 0.f, sk = 0.f;
-    for (int i = lane; i < K; i += 64) {
-      const float a = load_as_float(q, row * ld_qk + (int64_t)h * K + i, qkv_dtype);
-      const float b = load_as_float(k, row * ld_qk + (int64_t)h * K + i, qkv_dtype);
-      qs[i] = a;
-      ks[i] = b;
-      sq += a * a;
-      sk += b * b;
-    }
-    sq = wave_sum(sq);
-    sk = wave_sum(sk);
-    const float dq = sqrtf(sq + 1e-6f), dk = sqrtf(sk + 1e-6f);
-    for (int i = lane; i < K; i += 64) {
-      qs[i] = qs[i] / dq * scale;
-      ks[i] = ks[i] / dk;
+  for (int i = 0; i < KV; ++i) s[i] = 0.f;
+  if (init) {
+    for (int r = g16; r < K; r += 16)
+      rows[0][r * (kCols + 1) + p] =
+          p < ncol ? load_as_float(init, sbase + (int64_t)r * V + p, state_dtype) : 0.f;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < KV; ++i) {
+      const int r = (i / VW) * 16 * VW + p * VW + i % VW;
+      if (r < K) s[i] = rows[0][r * (kCols + 1) + g16];
     }
     __syncthreads();
-    const float decay = expf(load_as_float(gdecay, row * ld_gate + hv, gate_dtype));
-    const float bt = load_as_float(beta, row * ld_gate + hv, beta_dtype);
-    const float vj = active ? load_as_float(v, row * ld_v + (int64_t)hv * V + j, qkv_dtype) : 0.f;
-    float recall = 0.f;
-#pragma unroll
-    for (int i = 0; i < KMAX; ++i) {
-      if (i < K) {
-        s[i] *= decay;
-        recall += s[i] * ks[i];
-      }
-    }
-    const float u = bt * (vj - recall);
-    float o = 0.f;
-#pragma unroll
-    for (int i = 0; i < KMAX; ++i) {
-      if (i < K) {
-        s[i] += ks[i] * u;
-        o += s[i] * qs[i];
-      }
-    }
-    if (active) store_from_float(out, row * ld_out + (int64_t)hv * V + j, qkv_dtype, o);
-    __syncthreads();  // qs/ks are rewritten by the next token
   }
-  if (final_state && active) {
-    float* f = final_state + ((n * HV + hv) * (int64_t)K) * V + j;
+
+  // this thread's share of a tile: KV elements of token g16's q and k rows,
+  // column p of its v row, and its gates (every lane of the row loads them)
+  TIN rq[KV], rk[KV], rv;
+  float rg, rb;
+  const TIN* qh = q + (int64_t)h * K;
+  const TIN* kh = k + (int64_t)h * K;
+  const TIN* vh = v + (int64_t)hv * V + v0;
+  auto fetch = [&](int t0) {
+    const int64_t row = n * T + min(t0 + g16, T - 1);  // rows past the end are not used
+    if (wide) {
+      typedef TIN raw_t __attribute__((ext_vector_type(VW)));
 #pragma unroll
-    for (int i = 0; i < KMAX; ++i)
-      if (i < K) f[(int64_t)i * V] = s[i];
+      for (int c = 0; c < NC; ++c) {
+        const raw_t a = *(const raw_t*)(qh + row * ld_qk + c * 16 * VW + p * VW);
+        const raw_t b = *(const raw_t*)(kh + row * ld_qk + c * 16 * VW + p * VW);
+#pragma unroll
+        for (int e = 0; e < VW; ++e) {
+          rq[c * VW + e] = a[e];
+          rk[c * VW + e] = b[e];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < KV; ++i) {
+        const int r = (i / VW) * 16 * VW + p * VW + i % VW;
+        rq[i] = r < K ? qh[row * ld_qk + r] : TIN(0);
+        rk[i] = r < K ? kh[row * ld_qk + r] : TIN(0);
+      }
+    }
+    rv = p < ncol ? vh[row * ld_v + p] : TIN(0);
+    rg = load_as_float(gdecay, row * ld_gate + hv, gate_dtype);
+    rb = load_as_float(beta, row * ld_gate + hv, beta_dtype);
+  };
+  auto stash = [&](int buf) {
+    float fq[KV], fk[KV], sq = 0.f, sk = 0.f;
+#pragma unroll
+    for (int i = 0; i < KV; ++i) {
+      fq[i] = Elem<TIN>::to_f(rq[i]);
+      fk[i] = Elem<TIN>::to_f(rk[i]);
+      sq += fq[i] * fq[i];
+      sk += fk[i] * fk[i];
+    }
+    const float dq = sqrtf(row16_sum(sq) + 1e-6f), dk = sqrtf(row16_sum(sk) + 1e-6f);
+    float kq = 0.f;
+#pragma unroll
+    for (int i = 0; i < KV; ++i) {
+      fq[i] = fq[i] / dq * scale;
+      fk[i] = fk[i] / dk;
+      kq += fk[i] * fq[i];
+    }
+    kq = row16_sum(kq);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      vec_t a, b;
+#pragma unroll
+      for (int e = 0; e < VW; ++e) {
+        a[e] = fk[c * VW + e];
+        b[e] = fq[c * VW + e];
+      }
+      const int at = g16 * KP + c * 16 * VW + p * VW;
+      *(vec_t*)&rows[buf][at] = a;
+      *(vec_t*)&rows[buf][kQK + at] = b;
+    }
+    vs[buf][g16][p] = Elem<TIN>::to_f(rv);
+    if (p == 0) {
+      scal[buf][g16][0] = expf(rg);
+      scal[buf][g16][1] = rb;
+      scal[buf][g16][2] = kq;
+    }
+  };
+
+  fetch(0);
+  stash(0);
+  __syncthreads();
+  const int ntiles = (T + kTile - 1) / kTile;
+  for (int tile = 0; tile < ntiles; ++tile) {
+    const int buf = tile & 1, t0 = tile * kTile, nt = min(kTile, T - t0);
+    if (tile + 1 < ntiles) fetch(t0 + kTile);
+    // lane p of a column's row keeps token p's v and gates; a token's values
+    // reach the row's other lanes by a DPP row broadcast
+    const float tv = vs[buf][p][g16];
+    const float4 tg = *(const float4*)scal[buf][p];
+    vec_t kv[NC], qv[NC];
+    auto load = [&](int t, vec_t (&kr)[NC], vec_t (&qr)[NC]) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int at = t * KP + c * 16 * VW + p * VW;
+        kr[c] = *(const vec_t*)&rows[buf][at];
+        qr[c] = *(const vec_t*)&rows[buf][kQK + at];
+      }
+    };
+    load(0, kv, qv);
+    float ot = 0.f;  // token p's output
+    auto step = [&](auto tc) {
+      constexpr int t = decltype(tc)::value;
+      vec_t kn[NC], qn[NC];
+      load(t + 1 < kTile ? t + 1 : t, kn, qn);
+      const float decay = dpp_row<0x150 + t>(tg.x), bt = dpp_row<0x150 + t>(tg.y);
+      const float kq = dpp_row<0x150 + t>(tg.z), vj = dpp_row<0x150 + t>(tv);
+      float dk[2] = {0.f, 0.f}, dq[2] = {0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < KV; ++i) {
+        dk[i & 1] = fmaf(s[i], kv[i / VW][i % VW], dk[i & 1]);
+        dq[i & 1] = fmaf(s[i], qv[i / VW][i % VW], dq[i & 1]);
+      }
+      const float rk = row16_sum(dk[0] + dk[1]), rq = row16_sum(dq[0] + dq[1]);
+      const float u = bt * (vj - decay * rk);
+#pragma unroll
+      for (int i = 0; i < KV; ++i) s[i] = fmaf(kv[i / VW][i % VW], u, s[i] * decay);
+      const float o = fmaf(kq, u, decay * rq);
+      ot = p == t ? o : ot;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        kv[c] = kn[c];
+        qv[c] = qn[c];
+      }
+    };
+    // whole tiles without a branch between tokens, which would hold the next
+    // token's LDS reads back until it
+    if (nt == kTile)
+      unroll16(step);
+    else
+      unroll16([&](auto tc) {
+        if (decltype(tc)::value < nt) step(tc);
+      });
+    os[buf][p][g16] = ot;
+    if (tile + 1 < ntiles) stash(buf ^ 1);
+    __syncthreads();
+    if (g16 < nt && p < ncol)
+      out[(n * T + t0 + g16) * ld_out + (int64_t)hv * V + v0 + p] =
+          Elem<TIN>::from_f(os[buf][g16][p]);
+  }
+  if (final_state) {
+#pragma unroll
+    for (int i = 0; i < KV; ++i) {
+      const int r = (i / VW) * 16 * VW + p * VW + i % VW;
+      rows[0][r * (kCols + 1) + g16] = s[i];
+    }
+    __syncthreads();
+    float* f = final_state + ((n * HV + hv) * (int64_t)K) * V + v0;
+    if (p < ncol)
+      for (int r = g16; r < K; r += 16) f[(int64_t)r * V + p] = rows[0][r * (kCols + 1) + p];
   }
 }
 
-template <int KMAX>
+template <typename TIN, int KV>
 int launch_recurrent(const void* q, const void* k, const void* v, int64_t ld_qk, int64_t ld_v,
-                     int qkv_dtype, const void* g, int gate_dtype, const void* beta,
-                     int beta_dtype, int64_t ld_gate, const void* init, int state_dtype,
-                     int bps, void* out, int64_t ld_out, float* fin, int N, int T, int H, int HV,
-                     int K, int V, float scale, hipStream_t s) {
-  const int nvt = (V + 63) / 64;
+                     const void* g, int gate_dtype, const void* beta, int beta_dtype,
+                     int64_t ld_gate, const void* init, int state_dtype, int bps, void* out,
+                     int64_t ld_out, float* fin, int N, int T, int H, int HV, int K, int V,
+                     float scale, hipStream_t s) {
+  const int nvt = (V + kCols - 1) / kCols;
   const int64_t blocks = (int64_t)N * HV * nvt;
   if (blocks > 0x7fffffffLL) KAD_UNSUPPORTED("too many (sequence, head) pairs for one launch");
-  hipLaunchKernelGGL((gdn_recurrent_kernel<KMAX>), dim3((unsigned)blocks), dim3(64), 0, s, q, k,
-                     v, ld_qk, ld_v, qkv_dtype, g, gate_dtype, beta, beta_dtype, ld_gate, init,
-                     state_dtype, bps, out, ld_out, fin, T, H, HV, K, V, scale, nvt);
+  // whole vectors of min(KV, 4) elements: full, aligned rows
+  constexpr int VW = KV < 4 ? KV : 4;
+  const int wide = K == 16 * KV && ld_qk % VW == 0 && ((uintptr_t)q % (VW * sizeof(TIN))) == 0 &&
+                   ((uintptr_t)k % (VW * sizeof(TIN))) == 0;
+  hipLaunchKernelGGL((gdn_recurrent_kernel<TIN, KV>), dim3((unsigned)blocks), dim3(256), 0, s,
+                     (const TIN*)q, (const TIN*)k, (const TIN*)v, ld_qk, ld_v, g, gate_dtype,
+                     beta, beta_dtype, ld_gate, init, state_dtype, bps, (TIN*)out, ld_out, fin, T,
+                     H, HV, K, V, scale, nvt, wide);
   return kad_launch_status("gdn_recurrent_kernel");
 }
 
@@ -268,16 +422,22 @@ extern "C" int kad_gdn_recurrent(const void* q, const void* k, const void* v, in
               "unknown state dtype code %d", state_dtype);
   const int bps = initial_state ? beams_per_state : 1;
   hipStream_t s = (hipStream_t)stream;
-#define KAD_REC(KM)                                                                           \
-  if (K <= KM)                                                                                \
-    return launch_recurrent<KM>(q, k, v, ld_qk, ld_v, qkv_dtype, log_decay, gate_dtype, beta, \
-                                beta_dtype, ld_gate, initial_state, state_dtype, bps, out,    \
-                                ld_out, final_state, N, T, H, HV, K, V, scale, s);
+#define KAD_REC_T(TIN, KV)                                                                      \
+  return launch_recurrent<TIN, KV>(q, k, v, ld_qk, ld_v, log_decay, gate_dtype, beta,         \
+                                   beta_dtype, ld_gate, initial_state, state_dtype, bps, out, \
+                                   ld_out, final_state, N, T, H, HV, K, V, scale, s);
+#define KAD_REC(KV)                                                  \
+  if (K <= 16 * KV) {                                                \
+    if (qkv_dtype == KAD_DTYPE_F32) KAD_REC_T(float, KV)             \
+    if (qkv_dtype == KAD_DTYPE_BF16) KAD_REC_T(bf16_t, KV)           \
+    KAD_REC_T(_Float16, KV)                                          \
+  }
+  KAD_REC(1)
+  KAD_REC(2)
+  KAD_REC(4)
+  KAD_REC(8)
   KAD_REC(16)
-  KAD_REC(32)
-  KAD_REC(64)
-  KAD_REC(128)
-  KAD_REC(256)
+#undef KAD_REC_T
 #undef KAD_REC
   KAD_UNSUPPORTED("gated delta recurrence supports key dims <= 256, got %d", K);
 }

@@ -57,6 +57,28 @@ def test_gated_delta_final_state_general(device, dtype, K, V):
         assert_close_rel(go, eo, rtol=1e-2, atol_frac=4e-3, name="gdn final")
 
 
+@pytest.mark.parametrize("T", [1, 16, 17, 33])
+@pytest.mark.parametrize("K,V,offset", [(1, 1, 0), (16, 17, 0), (33, 16, 0), (64, 15, 1),
+                                        (128, 33, 0), (128, 16, 1), (256, 18, 0), (200, 5, 0)])
+def test_gated_delta_recurrence_tile_edges(device, T, K, V, offset):
+    """Tokens around the kernel's 16-token tiles, columns around its 16-column
+    groups, key dims at and between its 16-lane splits, and rows that are not
+    16-byte aligned (``offset`` elements into their storage).  fp32 sums of at
+    most 256 terms over 33 steps of a contracting state: 2e-5 absolute."""
+    q, k, v, g, beta, S = gdn_inputs(2, 1, T, 1, 2, K, V, dtype=torch.float32, seed=T + K)
+    eo, ef = ops_ref.gated_delta(q.double(), k.double(), v.double(), g.double(), beta.double(),
+                                 S.double(), return_final_state=True, compute=torch.float64)
+
+    def shifted(t):
+        d = torch.empty(t.numel() + offset, dtype=t.dtype, device=device)[offset:].view(t.shape)
+        return d.copy_(t)
+
+    go, gf = ops.gated_delta(*map(shifted, (q, k, v)), *_on(device, g, beta, S),
+                             return_final_state=True)
+    torch.testing.assert_close(go.double().cpu(), eo, atol=2e-5, rtol=1e-4)
+    torch.testing.assert_close(gf.double().cpu(), ef.double(), atol=2e-5, rtol=1e-4)
+
+
 def _attn_inputs(B, W, T, H, HK, L, D, dtype, seed, Tk=None):
     g = torch.Generator().manual_seed(seed)
     Tk = T if Tk is None else Tk
