@@ -283,14 +283,34 @@ int launch_recurrent(const void* q, const void* k, const void* v, int64_t ld_qk,
 }
 
 // ---------------------------------------------------------------------------
-// Prefix + causal-suffix attention, one wave per query row (n, t, h).  Keys
-// are visited in tiles of 64: lane j scores key j of the tile (the request's
-// prefix keys first, then the beam's own suffix keys up to the query's
-// position), an online softmax folds each tile in, and lane l accumulates
-// output dims l, l + 64, ...  Masked prefix keys are skipped; a row with no
-// visible key gives zeros (ops.py:229-240).  The output is rounded to the
-// tensor dtype, then multiplied by the rounded sigmoid of the gate when one is
-// given (src/kadllm/adapters/qwen3_5.py:199-201).
+// Prefix + causal-suffix attention in fp32 on v_mfma_f32_16x16x4_f32.
+//
+// The rows (beam, token, query head of the key head's group) of one key head
+// read the same prefix keys, so a workgroup takes 16 of them as the N
+// dimension of S^T = K Q^T and its 4 waves take every fourth step of 16 keys:
+// the request's prefix keys, then the suffix.  Suffixes of up to 8 tokens go
+// one token a step, its 16 keys the tile's beams (a row sees its own); longer
+// ones, whole prompts among them, keep to one beam per tile and go 16 tokens a
+// step.  Either way a row's keys come in steps that do not depend on which
+// rows share its tile or on how many tokens follow, nor do its bits.  Each wave folds
+// its steps with an online softmax into O^T = V^T P^T -- the accumulator of
+// S^T is P^T's operand as it stands -- and the four partial results merge
+// through LDS.  Splitting the keys over the waves rather than the rows fills
+// the chip with 16-row groups: 4 requests x 2 key heads x 512 rows are 256
+// workgroups.  Matrix rate bounds it (a step is 2 x 64 MFMAs of 32 cycles at
+// head dim 256, against 32 KB of K and V from L2 that arrive meanwhile: V
+// during S, the next K during O); 4 requests x 64 beams x 2 tokens, 500 fp32
+// keys: 1,100 us as one wave per row, 44 us here.
+//
+// Masked prefix keys have weight 0 and their V is not read as a number; a row
+// with no visible key gives zeros (ops.py:229-240).  The output is rounded to
+// the tensor dtype, then multiplied by the rounded sigmoid of the gate when
+// one is given (src/kadllm/adapters/qwen3_5.py:199-201).
+//
+// A product with weight 0 is not left out of an MFMA, so an infinite or NaN V
+// entry that a row must not see would reach it.  Rows whose result is not
+// finite are therefore computed again one by one (attention_row), skipping
+// the keys of weight 0.
 struct AttnArgs {
   const void *q, *pk, *pv, *sk, *sv, *gate;
   const uint8_t* mask;
@@ -300,101 +320,338 @@ struct AttnArgs {
   int64_t ssk_n, ssk_t, ssk_h, ssv_n, ssv_t, ssv_h;
   int64_t sg_n, sg_t, sg_h;
   int64_t so_n, so_t, so_h;
-  int W, Tq, Tk, H, HK, L, D, dtype;
+  int W, Tq, Tk, H, HK, L, D;
+  int by_token;      // suffix order, see attention_general_kernel
+  int beams;         // beams that share a group of rows: W, or 1
+  int rows, tiles;   // rows of a group, and its 16-row tiles
   float scale;
 };
 
-template <int DMAX>
-__global__ __launch_bounds__(64) void attention_general_kernel(AttnArgs a) {
-  constexpr int R = DMAX / 64;  // output dims per lane
-  __shared__ float qv[DMAX];
-  __shared__ float ps[64];
-  const int lane = threadIdx.x;
-  const int64_t rid = blockIdx.x;
-  const int h = (int)(rid % a.H);
-  const int t = (int)((rid / a.H) % a.Tq);
-  const int64_t n = rid / ((int64_t)a.H * a.Tq);
+template <typename TIN>
+__device__ __forceinline__ void attention_store(const AttnArgs& a, int64_t n, int t, int h, int d,
+                                                float y) {
+  y = round_to_dtype(y, Elem<TIN>::code);
+  if (a.gate) {
+    const float g = Elem<TIN>::to_f(((const TIN*)a.gate)[n * a.sg_n + (int64_t)t * a.sg_t +
+                                                         (int64_t)h * a.sg_h + d]);
+    y = y * round_to_dtype(sigmoid_exact(g), Elem<TIN>::code);
+  }
+  ((TIN*)a.out)[n * a.so_n + (int64_t)t * a.so_t + (int64_t)h * a.so_h + d] =
+      Elem<TIN>::from_f(y);
+}
+
+// one row by one wave: lane j scores key j of a tile of 64, lane l
+// accumulates output dims l, l + 64, ...; buf: DMAX + 64 floats of LDS of the
+// wave's own
+template <typename TIN, int DMAX>
+__device__ void attention_row(const AttnArgs& a, float* buf, int64_t n, int t, int h) {
+  constexpr int R = DMAX / 64;
+  float *qv = buf, *ps = buf + DMAX;
+  const int lane = threadIdx.x & 63;
   const int64_t b = n / a.W;
   const int hk = h / (a.H / a.HK);
-  const int tpos = t + (a.Tk - a.Tq);  // suffix position of this query
-  const int nkeys = a.L + tpos + 1;
-  const int dt = a.dtype;
-
+  const int nkeys = a.L + t + (a.Tk - a.Tq) + 1;
+  // LDS of one wave is read and written in program order
+  auto fence = [] { asm volatile("" ::: "memory"); };
+  fence();
   for (int d = lane; d < a.D; d += 64)
-    qv[d] = load_as_float(a.q, n * a.sq_n + (int64_t)t * a.sq_t + (int64_t)h * a.sq_h + d, dt);
-  __syncthreads();
-
-  // element offset of key `key`'s K row and V row
-  auto krow = [&](int key, const void*& base) -> int64_t {
-    if (key < a.L) {
-      base = a.pk;
-      return b * a.sp_b + (int64_t)key * a.sp_l + (int64_t)hk * a.sp_h;
-    }
-    base = a.sk;
-    return n * a.ssk_n + (int64_t)(key - a.L) * a.ssk_t + (int64_t)hk * a.ssk_h;
+    qv[d] = Elem<TIN>::to_f(
+        ((const TIN*)a.q)[n * a.sq_n + (int64_t)t * a.sq_t + (int64_t)h * a.sq_h + d]);
+  fence();
+  auto krow = [&](int key) {
+    return key < a.L ? (const TIN*)a.pk + b * a.sp_b + (int64_t)key * a.sp_l + (int64_t)hk * a.sp_h
+                     : (const TIN*)a.sk + n * a.ssk_n + (int64_t)(key - a.L) * a.ssk_t +
+                           (int64_t)hk * a.ssk_h;
   };
-  auto vrow = [&](int key, const void*& base) -> int64_t {
-    if (key < a.L) {
-      base = a.pv;
-      return b * a.sp_b + (int64_t)key * a.sp_l + (int64_t)hk * a.sp_h;
-    }
-    base = a.sv;
-    return n * a.ssv_n + (int64_t)(key - a.L) * a.ssv_t + (int64_t)hk * a.ssv_h;
+  auto vrow = [&](int key) {
+    return key < a.L ? (const TIN*)a.pv + b * a.sp_b + (int64_t)key * a.sp_l + (int64_t)hk * a.sp_h
+                     : (const TIN*)a.sv + n * a.ssv_n + (int64_t)(key - a.L) * a.ssv_t +
+                           (int64_t)hk * a.ssv_h;
   };
-
   float m = -INFINITY, l = 0.f;
   float o[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) o[r] = 0.f;
-
   for (int k0 = 0; k0 < nkeys; k0 += 64) {
     const int key = k0 + lane;
     float sc = -INFINITY;
     if (key < nkeys && !(key < a.L && a.mask && a.mask[b * a.L + key] == 0)) {
-      const void* base;
-      const int64_t off = krow(key, base);
+      const TIN* kp = krow(key);
       float acc = 0.f;
-      for (int d = 0; d < a.D; ++d) acc += qv[d] * load_as_float(base, off + d, dt);
+      for (int d = 0; d < a.D; ++d) acc += qv[d] * Elem<TIN>::to_f(kp[d]);
       sc = acc * a.scale;
     }
-    const float mt = wave_max(sc);
-    const float mn = fmaxf(m, mt);
+    const float mn = fmaxf(m, wave_max(sc));
     if (mn == -INFINITY) continue;  // nothing visible yet (masked keys only)
     const float p = sc == -INFINITY ? 0.f : expf(sc - mn);
     const float alpha = m == -INFINITY ? 0.f : expf(m - mn);
     l = l * alpha + wave_sum(p);
     m = mn;
+    fence();
     ps[lane] = p;
-    __syncthreads();
+    fence();
 #pragma unroll
     for (int r = 0; r < R; ++r) o[r] *= alpha;
     const int nk = min(64, nkeys - k0);
     for (int jj = 0; jj < nk; ++jj) {
       const float pj = ps[jj];
       if (pj == 0.f) continue;
-      const void* base;
-      const int64_t off = vrow(k0 + jj, base);
+      const TIN* vp = vrow(k0 + jj);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int d = lane + 64 * r;
-        if (d < a.D) o[r] += pj * load_as_float(base, off + d, dt);
+        if (d < a.D) o[r] += pj * Elem<TIN>::to_f(vp[d]);
       }
     }
-    __syncthreads();
   }
-  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  const float inv = l > 0.f ? 1.0f / l : (l == 0.f ? 0.f : l);  // a NaN sum stays one
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int d = lane + 64 * r;
-    if (d >= a.D) continue;
-    float y = round_to_dtype(o[r] * inv, dt);
-    if (a.gate) {
-      const float g = load_as_float(
-          a.gate, n * a.sg_n + (int64_t)t * a.sg_t + (int64_t)h * a.sg_h + d, dt);
-      y = round_to_dtype(y * round_to_dtype(sigmoid_exact(g), dt), dt);
-    }
-    store_from_float(a.out, n * a.so_n + (int64_t)t * a.so_t + (int64_t)h * a.so_h + d, dt, y);
+    if (d < a.D) attention_store<TIN>(a, n, t, h, d, o[r] * inv);
   }
+}
+
+// x combined with lane ^ 16's, as max_xor32
+__device__ __forceinline__ float max_xor16(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// FULL: head dim DMAX, every row 4-element aligned (whole-vector loads);
+// otherwise elements one by one, zero past the head dim
+template <typename TIN, int DMAX, bool FULL>
+__global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
+  constexpr int NQ = DMAX / 16;   // 16-dim pieces of a row
+  constexpr int NV = DMAX / 64;   // 64-dim pieces
+  constexpr int LDO = DMAX + 4;   // LDS row of a partial output
+  typedef TIN raw4 __attribute__((ext_vector_type(4)));
+  __shared__ __attribute__((aligned(16))) float po[4][16 * LDO];
+  __shared__ float pm[4][16], pl[4][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int c = lane & 15, j = lane >> 4;
+  const int G = a.H / a.HK;
+  const int lid = xcd_logical_id(blockIdx.x, gridDim.x);
+  const int tile = lid % a.tiles;
+  const int hk = (lid / a.tiles) % a.HK;
+  const int64_t n0 = (int64_t)(lid / a.tiles / a.HK) * a.beams;  // the group's first beam
+  const int64_t b = n0 / a.W;
+  const int r0 = tile * 16, r1 = min(r0 + 15, a.rows - 1);
+  const int w_lo = r0 / (a.Tq * G), w_hi = r1 / (a.Tq * G);
+  // this lane's query row (rows past the end repeat the last one)
+  const int row = min(r0 + c, a.rows - 1);
+  const int qw = row / (a.Tq * G), qt = row / G % a.Tq, qh = hk * G + row % G;
+  const int qpos = qt + (a.Tk - a.Tq);  // its suffix position
+  // suffix tokens that some row of the tile sees
+  const int nsuf = w_lo == w_hi ? (r1 / G % a.Tq) + (a.Tk - a.Tq) + 1 : a.Tk;
+  const int psteps = (a.L + 15) / 16;
+  const int steps = psteps + (a.by_token ? nsuf : (nsuf + 15) / 16);
+
+  auto load4 = [&](const TIN* p, int d) -> raw4 {
+    if constexpr (FULL) {
+      return *(const raw4*)(p + d);
+    } else {
+      raw4 r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = d + e < a.D ? p[d + e] : TIN(0);
+      return r;
+    }
+  };
+  // key i of step s; past the end the last one
+  auto kv_row = [&](bool value, int s, int i) -> const TIN* {
+    if (s < psteps) {
+      const int key = min(s * 16 + i, a.L - 1);
+      return (const TIN*)(value ? a.pv : a.pk) + b * a.sp_b + (int64_t)key * a.sp_l +
+             (int64_t)hk * a.sp_h;
+    }
+    const int64_t n = n0 + (a.by_token ? min(w_lo + i, w_hi) : w_lo);
+    const int64_t t = a.by_token ? s - psteps : min((s - psteps) * 16 + i, nsuf - 1);
+    return value ? (const TIN*)a.sv + n * a.ssv_n + t * a.ssv_t + (int64_t)hk * a.ssv_h
+                 : (const TIN*)a.sk + n * a.ssk_n + t * a.ssk_t + (int64_t)hk * a.ssk_h;
+  };
+
+  // v_mfma_f32_16x16x4_f32: lane l holds A[l%16][l/16] and B[l/16][l%16],
+  // accumulator element r of lane l is C[(l/16)*4 + r][l%16].  The dims of a
+  // 16-dim piece i meet in the order 16 i + 4 j + e (step e), so that a lane
+  // reads its share of a row as 4-element vectors.
+  float qf[NQ][4];
+  {
+    const TIN* qp = (const TIN*)a.q + (n0 + qw) * a.sq_n + (int64_t)qt * a.sq_t +
+                    (int64_t)qh * a.sq_h;
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const raw4 r = load4(qp, 16 * i + 4 * j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qf[i][e] = Elem<TIN>::to_f(r[e]);
+    }
+  }
+  raw4 kf[NQ], vf[4][NV];
+  auto load_k = [&](int s) {
+    const TIN* p = kv_row(false, s, c);
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) kf[i] = load4(p, 16 * i + 4 * j);
+  };
+  f32x4 o[NV * 4];
+#pragma unroll
+  for (int i = 0; i < NV * 4; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;  // l: this lane's share of the row's sum
+
+  if (wave < steps) load_k(wave);
+  for (int s = wave; s < steps; s += 4) {
+    // V of key 4 j + r, dims 64 i + 4 c + e
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const TIN* p = kv_row(true, s, 4 * j + r);
+#pragma unroll
+      for (int i = 0; i < NV; ++i) vf[r][i] = load4(p, 64 * i + 4 * c);
+    }
+    // which of this lane's 4 keys its row sees; hidden: nobody does
+    bool seen[4], hidden[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (s < psteps) {
+        const int key = s * 16 + 4 * j + r;
+        seen[r] = key < a.L && !(a.mask && a.mask[b * a.L + key] == 0);
+        hidden[r] = !seen[r];
+      } else if (a.by_token) {
+        const int w = w_lo + 4 * j + r;
+        seen[r] = w == qw && s - psteps <= qpos;
+        hidden[r] = w > w_hi;
+      } else {
+        const int t = (s - psteps) * 16 + 4 * j + r;
+        seen[r] = t <= qpos;
+        hidden[r] = t >= nsuf;
+      }
+    }
+    f32x4 acc[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NQ; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(Elem<TIN>::to_f(kf[i][e]), qf[i][e], acc[e],
+                                                      0, 0, 0);
+    if (s + 4 < steps) load_k(s + 4);
+    float sc[4], mt = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float x = ((acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r])) * a.scale;
+      sc[r] = seen[r] ? x : -INFINITY;
+      mt = fmaxf(mt, sc[r]);
+    }
+    mt = max_xor32(max_xor16(mt));
+    const float mn = fmaxf(m, mt);
+    // rows that see a larger score: scale what they have
+    if (__any(mn != m)) {
+      const float alpha = mn == m ? 1.f : (m == -INFINITY ? 0.f : expf(m - mn));
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < NV * 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[i][r] *= alpha;
+      m = mn;
+    }
+    float p[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      p[r] = sc[r] == -INFINITY ? 0.f : expf(sc[r] - m);
+      l += p[r];
+    }
+    if (__any(hidden[0] | hidden[1] | hidden[2] | hidden[3])) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (hidden[r])
+#pragma unroll
+          for (int i = 0; i < NV; ++i) vf[r][i] = raw4{TIN(0), TIN(0), TIN(0), TIN(0)};
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          o[i * 4 + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(Elem<TIN>::to_f(vf[r][i][e]), p[r],
+                                                              o[i * 4 + e], 0, 0, 0);
+  }
+  // o[4 i + e][r] is dim 64 i + 4 (4 j + r) + e of row c
+  l = add_xor32(add_xor16(l));
+  if (lane < 16) {
+    pm[wave][lane] = m;
+    pl[wave][lane] = l;
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *(f32x4*)&po[wave][c * LDO + 64 * i + 16 * j + 4 * r] =
+          f32x4{o[4 * i][r], o[4 * i + 1][r], o[4 * i + 2][r], o[4 * i + 3][r]};
+  __syncthreads();
+
+  // merge: thread -> row tid / 16, dims 64 i + 4 (tid % 16) + e
+  const int mr = tid >> 4, md = (tid & 15) * 4;
+  float M = -INFINITY, wgt[4], sum = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) M = fmaxf(M, pm[w][mr]);
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    wgt[w] = pm[w][mr] == -INFINITY ? 0.f : expf(pm[w][mr] - M);
+    // a wave that saw only NaN scores has no maximum but a NaN sum
+    sum += pl[w][mr] != pl[w][mr] ? pl[w][mr] : pl[w][mr] * wgt[w];
+  }
+  const float inv = sum > 0.f ? 1.0f / sum : (sum == 0.f ? 0.f : sum);
+  const int orow = min(r0 + mr, a.rows - 1);
+  const int64_t on = n0 + orow / (a.Tq * G);
+  const int ot = orow / G % a.Tq, oh = hk * G + orow % G;
+  bool finite = true;
+  f32x4 y[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    y[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) y[i] += *(const f32x4*)&po[w][mr * LDO + 64 * i + md] * wgt[w];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      y[i][e] *= inv;
+      finite = finite && fabsf(y[i][e]) < INFINITY;
+    }
+  }
+  if (__syncthreads_or(!finite)) {
+    for (int r = r0 + wave; r <= r1; r += 4)
+      attention_row<TIN, DMAX>(a, po[wave], n0 + r / (a.Tq * G), r / G % a.Tq, hk * G + r % G);
+    return;
+  }
+  if (r0 + mr < a.rows)
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (64 * i + md + e < a.D) attention_store<TIN>(a, on, ot, oh, 64 * i + md + e, y[i][e]);
+}
+
+template <typename TIN, int DMAX>
+int launch_attention(const AttnArgs& a, unsigned blocks, hipStream_t s) {
+  const int64_t strides[] = {a.sq_n, a.sq_t, a.sq_h, a.sp_b, a.sp_l, a.sp_h, a.ssk_n,
+                             a.ssk_t, a.ssk_h, a.ssv_n, a.ssv_t, a.ssv_h};
+  bool full = a.D == DMAX;
+  for (int64_t x : strides) full = full && x % 4 == 0;
+  for (const void* p : {a.q, a.pk, a.pv, a.sk, a.sv})
+    full = full && ((uintptr_t)p % (4 * sizeof(TIN))) == 0;
+  if (full)
+    hipLaunchKernelGGL((attention_general_kernel<TIN, DMAX, true>), dim3(blocks), dim3(256), 0, s,
+                       a);
+  else
+    hipLaunchKernelGGL((attention_general_kernel<TIN, DMAX, false>), dim3(blocks), dim3(256), 0, s,
+                       a);
+  return kad_launch_status("attention_general_kernel");
+}
+
+template <typename TIN>
+int launch_attention_dim(const AttnArgs& a, unsigned blocks, hipStream_t s) {
+  if (a.D <= 64) return launch_attention<TIN, 64>(a, blocks, s);
+  if (a.D <= 128) return launch_attention<TIN, 128>(a, blocks, s);
+  return launch_attention<TIN, 256>(a, blocks, s);
 }
 
 }  // namespace
@@ -460,15 +717,21 @@ extern "C" int kad_attention_general(
   if (D > 256) KAD_UNSUPPORTED("attention supports head dims <= 256, got %d", D);
   const int64_t rows = (int64_t)B * W * Tq * H;
   if (rows > 0x7fffffffLL) KAD_UNSUPPORTED("too many query rows for one launch");
-  AttnArgs a{q, prefix_k, prefix_v, suffix_k, suffix_v, gate, (const uint8_t*)prefix_mask, out,
-             sq_n, sq_t, sq_h, sp_b, sp_l, sp_h, ssk_n, ssk_t, ssk_h, ssv_n, ssv_t, ssv_h,
-             sg_n, sg_t, sg_h, so_n, so_t, so_h, W, Tq, Tk, H, HK, L, D, dtype, scale};
+  // The rows of a request's beams share tiles while their suffixes are short:
+  // a suffix token is then a step of its own, of which a row uses one key, so
+  // past a few tokens a step of 16 of one beam's tokens is less work.
+  const int by_token = Tk <= 8;
+  const int beams = by_token ? W : 1;
+  const int64_t grows = (int64_t)beams * Tq * (H / HK);
+  const int64_t tiles = kad_cdiv(grows, 16);
+  const int64_t blocks = (int64_t)B * (W / beams) * HK * tiles;
+  if (blocks > 0x7fffffffLL) KAD_UNSUPPORTED("too many query rows for one launch");
+  const AttnArgs a{q, prefix_k, prefix_v, suffix_k, suffix_v, gate, (const uint8_t*)prefix_mask,
+                   out, sq_n, sq_t, sq_h, sp_b, sp_l, sp_h, ssk_n, ssk_t, ssk_h, ssv_n, ssv_t,
+                   ssv_h, sg_n, sg_t, sg_h, so_n, so_t, so_h, W, Tq, Tk, H, HK, L, D, by_token,
+                   beams, (int)grows, (int)tiles, scale};
   hipStream_t s = (hipStream_t)stream;
-  if (D <= 64)
-    hipLaunchKernelGGL(attention_general_kernel<64>, dim3((unsigned)rows), dim3(64), 0, s, a);
-  else if (D <= 128)
-    hipLaunchKernelGGL(attention_general_kernel<128>, dim3((unsigned)rows), dim3(64), 0, s, a);
-  else
-    hipLaunchKernelGGL(attention_general_kernel<256>, dim3((unsigned)rows), dim3(64), 0, s, a);
-  return kad_launch_status("attention_general_kernel");
+  if (dtype == KAD_DTYPE_F32) return launch_attention_dim<float>(a, (unsigned)blocks, s);
+  if (dtype == KAD_DTYPE_BF16) return launch_attention_dim<bf16_t>(a, (unsigned)blocks, s);
+  return launch_attention_dim<_Float16>(a, (unsigned)blocks, s);
 }

@@ -113,6 +113,53 @@ def test_prefix_attention_general_matches_oracle(device, dtype, B, W, T, H, HK, 
         assert_close_rel(got, expected, rtol=1e-2, atol_frac=4e-3, name="attention general")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("W,T,Tk,H,HK,L,D", [
+    (5, 1, 1, 2, 2, 1, 64),      # 16-row tiles that end inside a request, one key
+    (17, 1, 3, 4, 4, 16, 64),    # more beams than a tile's rows; a whole step of keys
+    (3, 2, 2, 8, 2, 17, 256),
+    (6, 3, 8, 8, 2, 65, 128),    # the longest suffix taken token by token
+    (2, 9, 9, 8, 2, 33, 256),    # the shortest taken 16 tokens at a time
+    (2, 2, 40, 8, 2, 0, 60),     # no prefix, a head dim of no whole vectors
+    (1, 50, 50, 3, 1, 0, 256),   # a prompt whose rows straddle tokens
+])
+def test_prefix_attention_general_tile_edges(device, dtype, W, T, Tk, H, HK, L, D):
+    """Rows against their own: the kernel's 16-row, 16-key steps and both suffix
+    orders against the oracle, masked; and the last row's bits alone."""
+    q, pk, pv, sk, sv = _attn_inputs(2, W, Tk, H, HK, L, D, dtype, seed=W + Tk + L)
+    mask = torch.rand(2, L, generator=torch.Generator().manual_seed(L)) > 0.4 if L else None
+    expected = ops_ref.prefix_attention(*(t.double() for t in (q, pk, pv, sk, sv)), beam_width=W,
+                                        prefix_mask=mask)[:, Tk - T:]
+    dev = _on(device, q[:, Tk - T:].contiguous(), pk, pv, sk, sv)
+    got = prefix_attention_decode(*dev, W, _on(device, mask)[0], D ** -0.5)
+    if dtype == torch.float32:
+        torch.testing.assert_close(got.double().cpu(), expected, atol=2e-5, rtol=1e-4)
+    else:  # half an ulp of the output, and of the inputs' 2^-11 products
+        assert_close_rel(got, expected, rtol=2e-3, atol_frac=1e-3, name="attention tiles")
+    last = prefix_attention_decode(dev[0][:, -1:].contiguous(), *dev[1:], W,
+                                   _on(device, mask)[0], D ** -0.5)
+    assert torch.equal(last, got[:, -1:])
+
+
+@pytest.mark.parametrize("Tk", [2, 20])
+def test_prefix_attention_general_nonfinite_values_stay_with_their_rows(device, Tk):
+    """Infinite or NaN V entries reach only the rows that see their key: not
+    through a mask, not into another beam, not before their position."""
+    B, W, H, HK, L, D = 1, 4, 4, 2, 40, 64
+    q, pk, pv, sk, sv = _attn_inputs(B, W, Tk, H, HK, L, D, torch.float32, seed=Tk)
+    mask = torch.arange(L)[None] < 30
+    pv[:, 30:] = float("nan")
+    clean = sv.clone()
+    sv[1, -1] = float("inf")
+    expected = ops_ref.prefix_attention(q, pk, pv.nan_to_num(0.0), sk, clean, beam_width=W,
+                                        prefix_mask=mask)
+    got = ops.prefix_attention(*_on(device, q, pk, pv, sk, sv), beam_width=W,
+                               prefix_mask=mask.to(device)).cpu()
+    assert not torch.isfinite(got[1, -1]).any()
+    got[1, -1] = expected[1, -1]
+    torch.testing.assert_close(got, expected, atol=2e-5, rtol=1e-4)
+
+
 def test_prefix_attention_general_query_offset_and_gate(device):
     """Queries that are the last Tq of Tk suffix tokens equal the last rows of
     the full Tk-token attention; a gate multiplies by its rounded sigmoid."""
