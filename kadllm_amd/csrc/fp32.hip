@@ -18,6 +18,8 @@
 // They serve small fp32 models (the reference's CPU-plumbing configuration);
 // the bf16 kernels serve the headline model.
 
+#include <type_traits>
+
 #include "kad_common.h"
 
 namespace {
@@ -33,85 +35,284 @@ __device__ __forceinline__ float silu_exact(float x) { return x / (1.0f + expf(-
 __device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 // ---------------------------------------------------------------------------
-// GEMM: 64 x 64 output tile per workgroup of 4 waves, each wave a 32 x 32
-// block of four 16 x 16 MFMA tiles.  K moves in 16-deep slices through LDS
-// (rows padded to 17 floats: the 16 lanes of an MFMA operand read 16 rows of
-// one column, conflict free).  Operand layout of v_mfma_f32_16x16x4_f32:
-// lane l holds A[l % 16][l / 16] and B[l / 16][l % 16]; the accumulator's
-// element r of lane l is C[(l / 16) * 4 + r][l % 16].
-constexpr int kBM = 64, kBN = 64, kBK = 16, kLd = kBK + 1, kCld = kBN + 1;
+// GEMM on v_mfma_f32_16x16x4_f32 (lane l holds A[l % 16][l / 16] and
+// B[l / 16][l % 16]; accumulator element r of lane l is C[(l / 16) * 4 + r][l % 16]).
+// K is taken in pieces of 16: lane group q = l / 16 supplies elements 4 q + e
+// in step e, so that a lane's share of a row is one 16-byte word.
+//
+// Large products, bound by the matrix rate: 64 x 64 tiles (small enough that
+// 1,000 rows against 1,024 columns give every CU one), a wave's 16 rows x 64
+// columns, K in 32-deep slices through a ring of kSlots LDS slots filled by
+// direct loads.  A slice row is 128 bytes; its 16-byte chunk c is stored at
+// chunk c ^ ((row >> 1) & 7), so that the 16 rows of a fragment read hit 16
+// distinct bank groups.  One wave per SIMD has nothing to hide its other
+// instructions behind but its own MFMAs, so LDS reads and loads are spread
+// between them and slot indexes are constants.  1,000 x 7,168 x 1,024 with
+// SwiGLU 275 -> 126 us (116 TFLOP/s), 1,000 x 1,024 x 3,584 399 -> 65 us (113);
+// at 4,096 rows 128 TFLOP/s of the 150 that MFMAs alone reach.
+constexpr int kSlots = 4, kSlice = 64 * 32;  // floats of one operand's slice
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// one output element (or gate / up pair) through the epilogue
+__device__ __forceinline__ void gemm_f32_store(int epilogue, float* C, int64_t ldc, const float* R,
+                                               int64_t ldr, int64_t row, int col, float v) {
+  if (epilogue == KAD_EPI_RESIDUAL) v += R[row * ldr + col];
+  C[row * ldc + col] = v;
+}
+
+__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ Wt, int64_t ldw,
-    float* C, int64_t ldc, const float* R, int64_t ldr, int M, int N, int K, int epilogue) {
-  __shared__ float As[kBM * kLd], Ws[kBN * kLd];
-  __shared__ float Cs[kBM * kCld];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int64_t m0 = (int64_t)blockIdx.y * kBM;
-  const int n0 = blockIdx.x * kBN;
-  f32x4_t acc[2][2];
+    float* C, int64_t ldc, const float* R, int64_t ldr, int M, int N, int K, int epilogue,
+    int mtiles) {
+  __shared__ __attribute__((aligned(1024))) float ring[kSlots][2 * kSlice];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lid = xcd_logical_id(blockIdx.x, gridDim.x);
+  const int m0 = (lid % mtiles) * 64, n0 = (lid / mtiles) * 64;
+  // a direct load writes 64 x 16 bytes in lane order: 8 rows of a slice, lane
+  // l row l / 8, and fetches the chunk that belongs at its place.  The wave
+  // loads row groups wave and wave + 4 of each operand; rows past the end
+  // repeat the last one (their results are not stored).  Buffer loads take a
+  // lane's row as a fixed offset and the slice as a uniform one, which costs
+  // no address arithmetic between the MFMAs (offsets below 2 GB: checked by
+  // the dispatch).
+  const int dr = lane >> 3;
+  const __amdgpu_buffer_rsrc_t ab = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(A + (int64_t)m0 * lda), 0, 0x7fffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wb = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(Wt + (int64_t)n0 * ldw), 0, 0x7fffffff, 0x00020000);
+  uint32_t ao[2], wo[2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  for (int k0 = 0; k0 < K; k0 += kBK) {
-    // 64 x 16 of A and of W: 1024 elements each, 4 per thread, zero outside
-    for (int e = tid; e < kBM * kBK; e += 256) {
-      const int r = e / kBK, c = e % kBK;
-      const int64_t gm = m0 + r;
-      const int gk = k0 + c, gn = n0 + r;
-      As[r * kLd + c] = (gm < M && gk < K) ? A[gm * lda + gk] : 0.f;
-      Ws[r * kLd + c] = (gn < N && gk < K) ? Wt[(int64_t)gn * ldw + gk] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < kBK; kk += 4) {
-      const int k = kk + lane / 16;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const float a = As[(wm * 32 + i * 16 + lane % 16) * kLd + k];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const float b = Ws[(wn * 32 + j * 16 + lane % 16) * kLd + k];
-          acc[i][j] = mfma16x16x4f32(a, b, acc[i][j]);
-        }
-      }
-    }
-    __syncthreads();
+  for (int i = 0; i < 2; ++i) {
+    const int r = (wave + 4 * i) * 8 + dr;
+    const int ch = ((lane & 7) ^ ((r >> 1) & 7)) * 4;
+    ao[i] = (uint32_t)(((int64_t)(min(m0 + r, M - 1) - m0) * lda + ch) * 4);
+    wo[i] = (uint32_t)(((int64_t)(min(n0 + r, N - 1) - n0) * ldw + ch) * 4);
   }
-  // stage the tile, then write it out row by row with the epilogue
+  const int KT = K / 32;
+  // slice t into slot `at`; past the last slice, that one again (never read)
+  auto issue = [&](int t, int at) {
+    float* slot = ring[at] + wave * 8 * 32;
+    const uint32_t k = (uint32_t)min(t, KT - 1) * 128;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ab, (lds_void_t*)(slot + i * 4 * 8 * 32), 16, ao[i],
+                                               k, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wb, (lds_void_t*)(slot + kSlice + i * 4 * 8 * 32),
+                                               16, wo[i], k, 0, 0);
+    }
+  };
+  f32x4_t acc[4];
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+  for (int g = 0; g < 4; ++g) acc[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int fr = lane & 15, fq = lane >> 4, sw = fr >> 1;  // rows differ by multiples of 16
+  struct Frags {
+    f32x4_t a[2], w[2][4];  // [16-deep piece]
+  };
+  auto read = [&](Frags& f, int at) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        Cs[(wm * 32 + i * 16 + (lane / 16) * 4 + r) * kCld + wn * 32 + j * 16 + lane % 16] =
-            acc[i][j][r];
-  __syncthreads();
+    for (int piece = 0; piece < 2; ++piece) {
+      const float* p = ring[at] + fr * 32 + ((piece * 4 + fq) ^ sw) * 4;
+      f.a[piece] = *(const f32x4_t*)(p + wave * 16 * 32);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) f.w[piece][g] = *(const f32x4_t*)(p + kSlice + g * 16 * 32);
+    }
+  };
+  auto mfmas = [&](const Frags& f, int piece) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        acc[g] = mfma16x16x4f32(f.a[piece][e], f.w[piece][g][e], acc[g]);
+  };
+  // A wave holds slice t in registers when it reaches the barrier between the
+  // slice's two halves: after it the slot takes slice t + kSlots, and slice
+  // t + 1 (landed by then) is read while the second half multiplies.  The
+  // barrier does not wait for the loads still in flight (4 a slice); the empty
+  // asm statements keep LDS accesses on their side of it.
+#pragma unroll
+  for (int t = 0; t < kSlots; ++t) issue(t, t);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(4 * (kSlots - 1)) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  Frags f[2];
+  read(f[0], 0);
+  // false after the last slice
+  auto step = [&](int t, auto slot) -> bool {
+    constexpr int at = decltype(slot)::value;
+    Frags &cur = f[at & 1], &next = f[(at + 1) & 1];
+    mfmas(cur, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + 1 == KT) {
+      mfmas(cur, 1);
+      return false;
+    }
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(4 * (kSlots - 2)) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(next, (at + 1) % kSlots);
+    issue(t + kSlots, at);
+    mfmas(cur, 1);
+    // a read (a load) behind each of the first MFMAs
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if (i < 10) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (i >= 10 && i < 14) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    return true;
+  };
+  static_assert(kSlots == 4, "one step below for each slot");
+  for (int t = 0;; t += kSlots) {
+    if (!step(t, std::integral_constant<int, 0>{})) break;
+    if (!step(t + 1, std::integral_constant<int, 1>{})) break;
+    if (!step(t + 2, std::integral_constant<int, 2>{})) break;
+    if (!step(t + 3, std::integral_constant<int, 3>{})) break;
+  }
+  // no load may land in LDS that is another workgroup's by then
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+  const int64_t row0 = m0 + wave * 16 + fq * 4;
   if (epilogue == KAD_EPI_SWIGLU) {
     // the tile's 64 columns are one [gate 32 | up 32] block of W rows
-    const int oc0 = n0 / 2;
-    for (int e = tid; e < kBM * 32; e += 256) {
-      const int r = e / 32, c = e % 32;
-      const int64_t gm = m0 + r;
-      if (gm < M && n0 + c < N)
-        C[gm * ldc + oc0 + c] = silu_exact(Cs[r * kCld + c]) * Cs[r * kCld + 32 + c];
-    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (row0 + r < M)
+          C[(row0 + r) * ldc + n0 / 2 + g * 16 + fr] = silu_exact(acc[g][r]) * acc[g + 2][r];
     return;
   }
-  for (int e = tid; e < kBM * kBN; e += 256) {
-    const int r = e / kBN, c = e % kBN;
-    const int64_t gm = m0 + r;
-    const int gn = n0 + c;
-    if (gm < M && gn < N) {
-      float v = Cs[r * kCld + c];
-      if (epilogue == KAD_EPI_RESIDUAL) v += R[gm * ldr + gn];
-      C[gm * ldc + gn] = v;
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (row0 + r < M && n0 + g * 16 + fr < N)
+        gemm_f32_store(epilogue, C, ldc, R, ldr, row0 + r, n0 + g * 16 + fr, acc[g][r]);
+}
+
+// Products whose 64 x 64 tiles would leave CUs idle, and rows the direct loads
+// do not take: 16 MT rows x 16 columns (SwiGLU: 16 gate and their 16 up
+// columns) per workgroup, whose 8 waves take the 32-deep K slices in turn,
+// operands straight from memory, the next slice loading during the current
+// one; the partial sums merge through LDS.  With few rows the weight's bytes
+// bound it: 8 rows against 7,168 x 1,024 68 -> 9 us, 1,024 x 3,584 227 -> 13 us.
+template <int MT, bool SWIGLU, bool VEC>
+__global__ __launch_bounds__(512) void gemm_f32_split_kernel(
+    const float* __restrict__ A, int64_t lda, const float* __restrict__ Wt, int64_t ldw,
+    float* C, int64_t ldc, const float* R, int64_t ldr, int M, int N, int K, int epilogue,
+    int mtiles) {
+  constexpr int NG = SWIGLU ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) f32x4_t part[8][MT * NG][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lid = xcd_logical_id(blockIdx.x, gridDim.x);
+  const int m0 = (lid % mtiles) * 16 * MT, nt = lid / mtiles;
+  // SwiGLU: tile nt holds gate rows (nt / 2) * 64 + (nt % 2) * 16 .. of W and
+  // the up rows 32 further
+  const int n0 = SWIGLU ? (nt >> 1) * 64 + (nt & 1) * 16 : nt * 16;
+  const int fr = lane & 15, fq = lane >> 4;
+  const float *ap[MT], *wp[NG];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) ap[i] = A + (int64_t)min(m0 + i * 16 + fr, M - 1) * lda;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) wp[g] = Wt + (int64_t)min(n0 + g * 32 + fr, N - 1) * ldw;
+  auto load4 = [&](const float* p, int k) -> f32x4_t {
+    if constexpr (VEC) {  // K a multiple of 4
+      return k < K ? *(const f32x4_t*)(p + k) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    } else {
+      f32x4_t r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = k + e < K ? p[k + e] : 0.f;
+      return r;
+    }
+  };
+  f32x4_t acc[MT][NG];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int g = 0; g < NG; ++g) acc[i][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t a[2][MT], w[2][NG];
+  auto load = [&](int u, f32x4_t (&ar)[2][MT], f32x4_t (&wr)[2][NG]) {
+#pragma unroll
+    for (int piece = 0; piece < 2; ++piece) {
+      const int k = u * 32 + piece * 16 + fq * 4;
+#pragma unroll
+      for (int g = 0; g < NG; ++g) wr[piece][g] = load4(wp[g], k);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) ar[piece][i] = load4(ap[i], k);
+    }
+  };
+  const int units = (K + 31) / 32;
+  if (wave < units) load(wave, a, w);
+  for (int u = wave; u < units; u += 8) {
+    f32x4_t an[2][MT], wn[2][NG];
+    load(u + 8 < units ? u + 8 : u, an, wn);
+#pragma unroll
+    for (int piece = 0; piece < 2; ++piece)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int g = 0; g < NG; ++g)
+            acc[i][g] = mfma16x16x4f32(a[piece][i][e], w[piece][g][e], acc[i][g]);
+#pragma unroll
+    for (int piece = 0; piece < 2; ++piece) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) a[piece][i] = an[piece][i];
+#pragma unroll
+      for (int g = 0; g < NG; ++g) w[piece][g] = wn[piece][g];
     }
   }
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int g = 0; g < NG; ++g) part[wave][i * NG + g][lane] = acc[i][g];
+  __syncthreads();
+  auto total = [&](int f, int at) {  // element at of fragment f, waves in order
+    float v = 0.f;
+#pragma unroll
+    for (int x = 0; x < 8; ++x) v += ((const float*)part[x][f])[at];
+    return v;
+  };
+  for (int o = tid; o < MT * 256; o += 512) {
+    // output (row, column) of the tile, columns fastest
+    const int rr = o >> 4, cc = o & 15, i = rr >> 4, r = rr & 15;
+    const int at = ((r >> 2) * 16 + cc) * 4 + (r & 3);
+    const int64_t row = m0 + rr;
+    if (row >= M) continue;
+    if constexpr (SWIGLU) {
+      C[row * ldc + (nt >> 1) * 32 + (nt & 1) * 16 + cc] =
+          silu_exact(total(i * 2, at)) * total(i * 2 + 1, at);
+    } else if (n0 + cc < N) {
+      gemm_f32_store(epilogue, C, ldc, R, ldr, row, n0 + cc, total(i, at));
+    }
+  }
+}
+
+template <int MT, bool SWIGLU>
+void launch_split(bool vec, const float* A, int64_t lda, const float* W, int64_t ldw, float* C,
+                  int64_t ldc, const float* R, int64_t ldr, int M, int N, int K, int epilogue,
+                  hipStream_t s) {
+  const int mtiles = (int)kad_cdiv(M, 16 * MT);
+  const dim3 grid((unsigned)(mtiles * kad_cdiv(N, SWIGLU ? 32 : 16)));
+  if (vec)
+    hipLaunchKernelGGL((gemm_f32_split_kernel<MT, SWIGLU, true>), grid, dim3(512), 0, s, A, lda, W,
+                       ldw, C, ldc, R, ldr, M, N, K, epilogue, mtiles);
+  else
+    hipLaunchKernelGGL((gemm_f32_split_kernel<MT, SWIGLU, false>), grid, dim3(512), 0, s, A, lda, W,
+                       ldw, C, ldc, R, ldr, M, N, K, epilogue, mtiles);
+}
+
+template <int MT>
+void launch_split_epi(bool vec, const float* A, int64_t lda, const float* W, int64_t ldw, float* C,
+                      int64_t ldc, const float* R, int64_t ldr, int M, int N, int K, int epilogue,
+                      hipStream_t s) {
+  if (epilogue == KAD_EPI_SWIGLU)
+    launch_split<MT, true>(vec, A, lda, W, ldw, C, ldc, R, ldr, M, N, K, epilogue, s);
+  else
+    launch_split<MT, false>(vec, A, lda, W, ldw, C, ldc, R, ldr, M, N, K, epilogue, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -230,11 +431,29 @@ extern "C" int kad_gemm_f32(const float* A, int64_t lda, const float* W, int64_t
   KAD_REQUIRE(lda >= K && ldw >= K, "row strides too small");
   const int n_out = epilogue == KAD_EPI_SWIGLU ? N / 2 : N;
   KAD_REQUIRE(ldc >= n_out && (epilogue != KAD_EPI_RESIDUAL || ldr >= N), "row strides too small");
-  dim3 grid((unsigned)kad_cdiv(N, kBN), (unsigned)kad_cdiv(M, kBM));
-  KAD_REQUIRE(grid.y < 65536, "too many rows for one launch");
-  hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(256), 0, (hipStream_t)stream, A, lda, W, ldw, C,
-                     ldc, R, ldr, M, N, K, epilogue);
-  return kad_launch_status("gemm_f32_kernel");
+  const int64_t tiles = kad_cdiv(M, 64) * kad_cdiv(N, 64);
+  KAD_REQUIRE(kad_cdiv(M, 64) < 65536, "too many rows for one launch");
+  if (kad_cdiv(M, 16) * kad_cdiv(N, 16) > 0x7fffffff) KAD_UNSUPPORTED("gemm grid too large");
+  const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ((uintptr_t)A % 16) == 0 &&
+                   ((uintptr_t)W % 16) == 0;
+  hipStream_t s = (hipStream_t)stream;
+  // The tile kernel from 72 tiles: at K = 3,584 it takes 60 us however few of
+  // its tiles there are (one per CU), the split one 36 us at 64 tiles' worth
+  // of rows and columns and 70 us at 80.  At most 32 rows leave half a tile
+  // empty: 32 rows against 7,168 x 1,024 are 13 us split, 20 us in tiles.
+  if (vec && K % 32 == 0 && M > 32 && tiles >= 72 && (lda > ldw ? lda : ldw) * 64 + K < 0x1fffffff) {
+    hipLaunchKernelGGL(gemm_f32_tile_kernel, dim3((unsigned)tiles), dim3(256), 0, s, A, lda, W,
+                       ldw, C, ldc, R, ldr, M, N, K, epilogue, (int)kad_cdiv(M, 64));
+    return kad_launch_status("gemm_f32_tile_kernel");
+  }
+  const int64_t cols = kad_cdiv(N, epilogue == KAD_EPI_SWIGLU ? 32 : 16);
+  if (kad_cdiv(M, 64) * cols >= 256)
+    launch_split_epi<4>(vec, A, lda, W, ldw, C, ldc, R, ldr, M, N, K, epilogue, s);
+  else if (M > 16 && kad_cdiv(M, 32) * cols >= 64)
+    launch_split_epi<2>(vec, A, lda, W, ldw, C, ldc, R, ldr, M, N, K, epilogue, s);
+  else
+    launch_split_epi<1>(vec, A, lda, W, ldw, C, ldc, R, ldr, M, N, K, epilogue, s);
+  return kad_launch_status("gemm_f32_split_kernel");
 }
 
 extern "C" int kad_rmsnorm_f32(const float* x, int64_t ldx, const float* w, float w_offset,

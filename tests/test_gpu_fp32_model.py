@@ -52,6 +52,34 @@ def test_gemm_f32_matches_torch(device, M, N, K):
         torch.testing.assert_close(got, expected.reshape(M, N // 2), atol=1e-4, rtol=1e-5)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (33, 64 * 72, 32), (100, 64 * 36 + 4, 64), (64, 64 * 80, 96), (257, 1088, 128),
+    (1000, 1024, 160), (129, 2304, 288),                     # 64 x 64 tiles, 1 .. 9 slices
+    (256, 1024, 64), (300, 200, 36), (17, 96, 260), (16, 128, 31), (5, 33, 1), (700, 640, 33),
+])
+def test_gemm_f32_kernels_at_their_edges(device, M, N, K):
+    """Tile and split kernels: partial tiles, every remainder of the slice ring,
+    K short of a slice and rows that are not 16-byte aligned.  Sums of at most
+    288 products of unit by 0.05: 1e-4."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, K + 3, generator=g)[:, :K] if K % 2 else torch.randn(M, K, generator=g)
+    w = torch.randn(N, K, generator=g) * 0.05
+    r = torch.randn(M, N, generator=g)
+    ad = torch.empty(M, a.stride(0), device=device)[:, :K].copy_(a)
+    wd, rd = w.to(device), r.to(device)
+    ref = a.double() @ w.double().T
+    torch.testing.assert_close(gemm(ad, wd).cpu().double(), ref, atol=1e-4, rtol=1e-5)
+    out = torch.full((M, N + 5), 7.0, device=device)
+    gemm(ad, wd, out=out[:, :N], epilogue=EPI_RESIDUAL, residual=rd)
+    torch.testing.assert_close(out[:, :N].cpu().double(), ref + r.double(), atol=1e-4, rtol=1e-5)
+    assert bool((out[:, N:] == 7.0).all()), "wrote past the output width"
+    if N % 64 == 0:
+        blocks = ref.view(M, N // 64, 2, 32)
+        expected = (F.silu(blocks[:, :, 0]) * blocks[:, :, 1]).reshape(M, N // 2)
+        torch.testing.assert_close(gemm(ad, wd, epilogue=EPI_SWIGLU).cpu().double(), expected,
+                                   atol=1e-4, rtol=1e-5)
+
+
 def test_rmsnorm_f32_matches_oracle(device):
     g = torch.Generator().manual_seed(2)
     x = torch.randn(33, 256, generator=g)
