@@ -193,7 +193,9 @@ int kad_gemm_bf16_conv(const void* A, int64_t lda, const void* W, int64_t ldw, v
  * MFMA phases and load phases across workgroup barriers, M and N multiples
  * of 256, 16-byte store epilogue as 16; 24 = 256x256 persistent with 4
  * waves of 128x128, M and N multiples of 256, epilogues from the
- * accumulators, aligned outputs as 16).  Every
+ * accumulators, aligned outputs as 16; 32 .. 37 = tiles of 16x16, 16x32, 32x32,
+ * 32x64, 64x64 and 128x64 whose K streams through a ring of LDS slots, K a
+ * multiple of 128 (of 64 for 64x64 and 128x64), 32 without SwiGLU).  Every
  * configuration accumulates K in the same order, so all give bit-identical
  * results (the automatic choice may also split the columns of one call
  * between two of them); other numbers are rejected (KAD_ERR_UNSUPPORTED). */

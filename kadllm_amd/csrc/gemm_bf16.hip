@@ -23,32 +23,15 @@
 
 #include <cstdlib>
 
-#include "kad_common.h"
+#include "gemm_common.h"
 
 namespace {
+
+using namespace kad_gemm;
 
 constexpr int kBK = 64;
 constexpr int kPad = 8;
 constexpr int kLdk = kBK + kPad;  // LDS row stride (elements)
-
-// SiLU of the SwiGLU epilogues: x / (1 + e^-x) with the hardware reciprocal
-// (1 ulp) in place of the IEEE divide, which is most of the epilogue's VALU
-// work; every tile configuration uses it, so they still agree bit for bit
-__device__ __forceinline__ float silu_rcp(float x) {
-  return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x));
-}
-
-// SwiGLU of two adjacent outputs, bf16(bf16(silu(bf16(g))) * bf16(u)) for
-// (g0, u0) in the low half and (g1, u1) in the high half: each bf16
-// rounding of the pair is one packed conversion (the same bits as rounding
-// each value on its own, with half the conversions and their widenings)
-__device__ __forceinline__ uint32_t swiglu2(float g0, float g1, float u0, float u1) {
-  const uint32_t gp = pack_bf16x2(g0, g1), up = pack_bf16x2(u0, u1);
-  const float ua = __uint_as_float(up << 16), ub = __uint_as_float(up & 0xffff0000u);
-  const uint32_t sp =
-      pack_bf16x2(silu_rcp(__uint_as_float(gp << 16)), silu_rcp(__uint_as_float(gp & 0xffff0000u)));
-  return pack_bf16x2(__uint_as_float(sp << 16) * ua, __uint_as_float(sp & 0xffff0000u) * ub);
-}
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_kernel(
@@ -1832,7 +1815,27 @@ int launch_n32(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, 
 enum { CFG_AUTO = 0, CFG_32x256 = 1, CFG_128x128 = 2, CFG_256x256_8W = 5, CFG_64x32 = 11,
        CFG_32x64 = 12, CFG_N32 = 13,
        CFG_256x256_X16 = 16, CFG_256x256_X16P = 18, CFG_128x128_X16 = 19,
-       CFG_256x256_S3 = 20, CFG_256x256_PPP = 22, CFG_256x256_W4E = 24 };
+       CFG_256x256_S3 = 20, CFG_256x256_PPP = 22, CFG_256x256_W4E = 24,
+       CFG_RING = 32 /* + RingTile */ };
+
+// Tile of the ring kernel for a product, or -1: the smallest whose tiles number
+// at most one per CU -- a second round costs more than a larger tile's bytes
+// (N = 1,024, K = 3,584: 200 rows 17.0 us as 832 tiles of 16x16, 9.3 as 224 of
+// 32x32; 1,000 rows 33.0 as 1,024 of 32x32, 19.1 as 256 of 64x64) -- then 128x64
+// up to two per CU (400 x 8,192 x 1,024: 15.9 us against 17.9 in 128x128 tiles;
+// 600 rows 24.8 against 19.3).  At most 16 rows are bound by the weight's bytes,
+// whatever its columns (16 x 248,320 x 1,024: 98 us in 64x64 tiles, 106 in 32x256).
+int ring_tile(int M, int N, int K, int epi) {
+  static constexpr int kTiles[][3] = {{16, 16, RING_16x16}, {16, 32, RING_16x32},
+                                      {32, 32, RING_32x32}, {32, 64, RING_32x64},
+                                      {64, 64, RING_64x64}, {128, 64, RING_128x64}};
+  const int64_t cus = device_cu_count();
+  for (const auto& t : kTiles)
+    if (ring_ok((RingTile)t[2], K, epi) && kad_cdiv(M, t[0]) * kad_cdiv(N, t[1]) <= cus)
+      return t[2];
+  if (N > 32 && kad_cdiv(M, 128) * kad_cdiv(N, 64) <= 2 * cus) return RING_128x64;
+  return M <= 16 ? RING_64x64 : -1;
+}
 
 template <int EPI>
 int pick(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
@@ -1849,17 +1852,22 @@ int pick(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, void* 
     // persistent form is 2% faster, interleaved medians); then the
     // 128x128 form, two workgroups per CU, when its tiles fill two rounds
     // (N = 1,024 at M = 8,192: 5-7% faster than 8-wave 256x128 tiles, and
-    // 14% slower than 256x256 where those fill the chip); 64x32 for outputs
-    // of at most 32 columns (the GDN gate projection); the register-staged
-    // 128x128 kernel otherwise (all measured on the decode/prefill shapes)
+    // 14% slower than 256x256 where those fill the chip; a tenth faster than
+    // the register-staged 128x128 kernel where they do not); that one for
+    // outputs that do not suit 16-byte stores (all measured on the
+    // decode/prefill shapes)
     const int64_t tiles256 = kad_cdiv(M, 256) * kad_cdiv(N, 256);
-    const int64_t tiles128 = kad_cdiv(M, 128) * kad_cdiv(N, 128);
     const bool vec = vector_epilogue_ok(C, ldc, R, ldr, N, EPI);
-    if (M <= 64)
-      cfg = N <= 2048 && EPI != KAD_EPI_SWIGLU ? CFG_32x64 : CFG_32x256;
+    const int ring = ring_tile(M, N, K, EPI);
+    if (ring >= 0)
+      cfg = CFG_RING + ring;
+    else if (M <= 128 && vec)
+      // many columns and few rows (the vocabulary head): 256-row tiles would be
+      // half empty (64 rows 111 against 170 us, 128 rows 124 against 137)
+      cfg = CFG_128x128_X16;
     else if (N <= 32)
-      // whole-K waves of 32 rows (the GDN gate projection at M = 8,192 and
-      // 32,768), else 64x32 tiles
+      // whole-K waves of 32 rows (the GDN gate projection at M = 32,768),
+      // else 64x32 tiles
       cfg = n32_ok(A, lda, W, ldw, N, K, EPI) ? CFG_N32 : CFG_64x32;
     else if (tiles256 >= 256 && !vec)
       cfg = CFG_256x256_8W;
@@ -1882,7 +1890,7 @@ int pick(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, void* 
     else if (tiles256 >= 256)
       cfg = EPI == KAD_EPI_SWIGLU && tiles256 < 8 * device_cu_count() ? CFG_256x256_X16
                                                                         : CFG_256x256_X16P;
-    else if (vec && tiles128 >= 512)
+    else if (vec)
       cfg = CFG_128x128_X16;
     else
       cfg = CFG_128x128;
@@ -1917,9 +1925,6 @@ int pick(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, void* 
   switch (cfg) {
     case CFG_32x256: return launch<32, 256, 1, 4, EPI>(A, lda, W, ldw, C, ldc, R, ldr, M, N, K, s);
     case CFG_32x64:
-      // a few rows against a narrow weight (the pruned last prefill layer's
-      // output and down projections, M = 32, N = 1,024): four times the
-      // workgroups of 32x256 tiles (13.2 against 25.8 us at K = 2,048)
       if (EPI == KAD_EPI_SWIGLU) KAD_UNSUPPORTED("tile configuration 12 has no SwiGLU epilogue");
       return launch<32, 64, 1, 2, EPI == KAD_EPI_SWIGLU ? KAD_EPI_STORE : EPI>(
           A, lda, W, ldw, C, ldc, R, ldr, M, N, K, s);
@@ -1957,6 +1962,14 @@ int pick(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, void* 
         return launch_x16<EPI, TileX16<128, 128, 2, 2>>(A, lda, W, ldw, C, ldc, R, ldr, M, N, K,
                                                         s);
       return launch_x16p<EPI, 256>(A, lda, W, ldw, C, ldc, R, ldr, M, N, K, s);
+    case CFG_RING + RING_16x16:
+    case CFG_RING + RING_16x32:
+    case CFG_RING + RING_32x32:
+    case CFG_RING + RING_32x64:
+    case CFG_RING + RING_64x64:
+    case CFG_RING + RING_128x64:
+      return launch_ring((RingTile)(cfg - CFG_RING), EPI, A, lda, W, ldw, C, ldc, R, ldr, M, N, K,
+                         s);
     default: KAD_UNSUPPORTED("unknown gemm tile configuration %d", cfg);
   }
 }

@@ -364,6 +364,53 @@ def test_gemm_pipelined_tile_rejects_unaligned_output(device):
                   0, 256, 256, 64, layers.EPI_STORE, 16, _lib.stream_of(a))
 
 
+@pytest.mark.parametrize("epi", [layers.EPI_STORE, layers.EPI_RESIDUAL, layers.EPI_SWIGLU])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 64, 128), (15, 192, 256), (17, 1088, 384), (33, 320, 512), (65, 448, 640),
+    (129, 64, 1152), (64, 128, 64), (130, 192, 320), (100, 1000, 896), (70, 30, 1152),
+])
+def test_gemm_ring_tiles_agree(device, M, N, K, epi):
+    """Configurations 32 .. 37 (K through a ring of LDS slots) and the automatic
+    choice equal configuration 2 bit for bit: partial tiles, every remainder of
+    the ring, outputs of no whole 4-column words, an in-place residual."""
+    from kadllm_amd import _lib
+    if epi == layers.EPI_SWIGLU and N % 64:
+        pytest.skip("SwiGLU takes whole [gate 32 | up 32] blocks")
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g).bfloat16().to(device)
+    w = (torch.randn(N, K, generator=g) * 0.05).bfloat16().to(device)
+    n_out = N // 2 if epi == layers.EPI_SWIGLU else N
+    x = torch.randn(M, n_out, generator=g).bfloat16().to(device)
+    outs = {}
+    for cfg in (2, 0, 32, 33, 34, 35, 36, 37):
+        if (cfg == 32 and epi == layers.EPI_SWIGLU) or (K % 128 and 32 <= cfg < 36):
+            continue
+        for ldc in (n_out + 8 - n_out % 8, n_out + 3):  # 4-column words, and not
+            c = torch.zeros(M, ldc, dtype=torch.bfloat16, device=device)
+            cv = c[:, :n_out]
+            res = epi == layers.EPI_RESIDUAL
+            if res:
+                cv.copy_(x)
+            _lib.call("kad_gemm_bf16_tiled", _lib.ptr(a), K, _lib.ptr(w), K, _lib.ptr(cv), ldc,
+                      _lib.ptr(cv) if res else None, ldc if res else 0, M, N, K, epi, cfg,
+                      _lib.stream_of(a))
+            assert (c[:, n_out:] == 0).all(), f"config {cfg} wrote past the output width"
+            outs.setdefault(2, cv.clone())
+            assert torch.equal(cv, outs[2]), f"config {cfg} differs from config 2"
+
+
+@pytest.mark.parametrize("cfg,K,epi", [(32, 64, layers.EPI_STORE), (35, 192, layers.EPI_STORE),
+                                       (32, 128, layers.EPI_SWIGLU)])
+def test_gemm_ring_tiles_reject(device, cfg, K, epi):
+    from kadllm_amd import _lib
+    a = torch.zeros(64, K, dtype=torch.bfloat16, device=device)
+    w = torch.zeros(64, K, dtype=torch.bfloat16, device=device)
+    c = torch.zeros(64, 64, dtype=torch.bfloat16, device=device)
+    with pytest.raises(_lib.KadLibraryError, match="ring tile configurations need"):
+        _lib.call("kad_gemm_bf16_tiled", _lib.ptr(a), K, _lib.ptr(w), K, _lib.ptr(c), 64, None,
+                  0, 64, 64, K, epi, cfg, _lib.stream_of(a))
+
+
 @pytest.mark.parametrize("cfg", [11, 12, 13])
 def test_gemm_skinny_tiles_reject_swiglu(device, cfg):
     """The 64x32 and 32x64 register-staged tiles carry no SwiGLU epilogue (a
