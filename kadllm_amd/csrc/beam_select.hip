@@ -15,11 +15,12 @@
 // order is the logit order, so the request's top W is among these rows'
 // top min(W, V) entries.  Keys are ((x - max) - log(sum exp)) + parent in fp32.
 //
-// Stage 2, kad_beam_merge_select (one workgroup per request): an 8-bit radix
-// select over the request's Wp*K candidate keys finds the W-th key, a second
-// radix select over flat indices resolves ties (lower flat index first), and
-// the W winners are bitonic-sorted by (key desc, index asc) in LDS, for W up
-// to 16384.  kad_beam_merge_select_wide serves wider levels (the reference's
+// Stage 2, kad_beam_merge_select (one workgroup per request): a sampled
+// threshold keeps a few times W of the request's Wp*K candidates, which are
+// sorted by (key desc, index asc); wide or heavily tied levels take an 8-bit
+// radix select over the keys for the W-th key, a second over flat indices for
+// its ties (lower flat index first), and a bitonic sort of the W winners in
+// LDS, for W up to 16384.  kad_beam_merge_select_wide serves wider levels (the reference's
 // topk has no width cap): the same radix rounds, histogrammed by many
 // workgroups per request, and the winners sorted in caller workspace.
 //
@@ -553,7 +554,7 @@ __device__ __forceinline__ bool before(float ka, int ia, float kb, int ib) {
 // Every radix round reads the request's candidate keys again (L2-resident);
 // each thread loads kMergeBatch of them before using any, so that many loads
 // are in flight instead of one.
-constexpr int kMergeBatch = 8;
+constexpr int kMergeBatch = 16;
 
 // Run by one full wave: the bin d at which the running count of hist,
 // taken from bin 255 down (DESC) or from bin 0 up, first reaches need, and
@@ -704,6 +705,87 @@ __device__ __forceinline__ void hist_add_grouped(int* hist, bool active, int bin
   if ((pending >> lane) & 1ull) atomicAdd(&hist[bin], 1);
 }
 
+// Candidates as sortable words: key descending, then flat index ascending, is
+// word descending.  A zero of either sign is one key.
+__device__ __forceinline__ uint64_t merge_word(float key, int idx) {
+  return ((uint64_t)order32(key + 0.f) << 32) | (uint32_t)~idx;
+}
+
+// words the merge sorts without the radix rounds
+constexpr int kPruneCap = 4096;
+
+// Bitonic sort, largest first, of kMergeThreads * E words, thread t holding
+// words t * E + e: partners within a wave by shuffles, farther ones through
+// lds (as many words).
+template <int E>
+__device__ void sort_words(uint64_t (&v)[E], uint64_t* lds) {
+  const int tid = threadIdx.x;
+#pragma unroll 1
+  for (int size = 2; size <= kMergeThreads * E; size <<= 1) {
+#pragma unroll 1
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      auto pick = [&](int e, uint64_t other) {
+        const int i = tid * E + e;
+        const bool larger = ((i & stride) == 0) == ((i & size) == 0);
+        return (v[e] > other) == larger ? v[e] : other;
+      };
+      if (stride < E) {
+        uint64_t w[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          uint64_t other = 0;
+#pragma unroll
+          for (int x = 0; x < E; ++x)
+            if (x == (e ^ stride)) other = v[x];
+          w[e] = pick(e, other);
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = w[e];
+      } else if (stride < 64 * E) {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+          v[e] = pick(e, __shfl_xor((unsigned long long)v[e], stride / E, 64));
+      } else {
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < E; ++e) lds[tid * E + e] = v[e];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = pick(e, lds[(tid * E + e) ^ stride]);
+      }
+    }
+  }
+}
+
+// Sorted winners of one request from its `count` collected words.
+template <int E>
+__device__ void emit_sorted(uint64_t* words, int count, int W, int V, float* scores,
+                            int64_t* parents, int64_t* tokens, uint8_t* valid) {
+  const int tid = threadIdx.x;
+  uint64_t v[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = tid * E + e < count ? words[tid * E + e] : 0;
+  sort_words<E>(v, words);
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int i = tid * E + e;
+    if (i >= W) break;
+    const uint32_t u = (uint32_t)(v[e] >> 32);
+    const float key = __uint_as_float((u & 0x80000000u) ? u ^ 0x80000000u : ~u);
+    const int id = (int)~(uint32_t)v[e];
+    scores[i] = key;
+    parents[i] = id / V;
+    tokens[i] = id % V;
+    valid[i] = (key == key) && (key != INFINITY) && (key != -INFINITY);
+  }
+}
+
+// One workgroup per request.  Levels of up to kPruneCap candidates are sorted
+// whole; of more, a sample's order statistic gives a threshold that about
+// 2 W + 256 candidates reach, one pass collects those, and they are sorted --
+// what is collected holds the W best, ties by index included, whenever it
+// numbers at least W.  Otherwise (many equal keys, or W past about 1,400) the
+// radix rounds below.  8 requests x 65,536 candidates, W 256: @M0@.
 __global__ __launch_bounds__(kMergeThreads) void merge_select_kernel(
     const float* __restrict__ cand_key, const int* __restrict__ cand_idx, int ncand, int W,
     int V, float* __restrict__ scores, int64_t* __restrict__ parents,
@@ -731,6 +813,59 @@ __global__ __launch_bounds__(kMergeThreads) void merge_select_kernel(
     }
     for (int i = i0; i < ncand; i += kMergeThreads) f(order32(keys[i]), i);
   };
+
+  if (ncand <= kPruneCap || 2 * W + 256 <= kPruneCap * 3 / 4) {
+    __shared__ int sh_reach[32];
+    uint64_t* words = (uint64_t*)merge_lds;
+    if (tid < 32) sh_reach[tid] = 0;
+    if (tid == 0) sh_count = 0;
+    __syncthreads();
+    uint32_t thr = 0;  // order key, low 12 bits zero
+    if (ncand > kPruneCap) {
+      constexpr int kS = kPruneCap / kMergeThreads;
+      const int stride = (ncand + kPruneCap - 1) / kPruneCap;
+      const int rank = (2 * W + 256 + stride - 1) / stride;
+      uint32_t u[kS];
+#pragma unroll
+      for (int q = 0; q < kS; ++q) {
+        const int i = (tid * kS + q) * stride;
+        u[q] = i < ncand ? order32(keys[i]) : 0u;
+      }
+      for (int bit = 31; bit >= 12; --bit) {
+        const uint32_t t = thr | (1u << bit);
+        int c = 0;
+#pragma unroll
+        for (int q = 0; q < kS; ++q) c += __popcll(__ballot(u[q] >= t));
+        if ((tid & 63) == 0) atomicAdd(&sh_reach[bit], c);
+        __syncthreads();
+        if (sh_reach[bit] >= rank) thr = t;
+      }
+    }
+    for_each([&](uint32_t k, int i) {
+      const bool take = k >= thr;
+      const uint64_t takers = __ballot(take);
+      if (takers == 0) return;
+      const int lane = tid & 63, leader = __ffsll((unsigned long long)takers) - 1;
+      int base = 0;
+      if (lane == leader) base = atomicAdd(&sh_count, (int)__popcll(takers));
+      base = __shfl(base, leader, 64);
+      const int slot = base + (int)__popcll(takers & ((1ull << lane) - 1));
+      if (take && slot < kPruneCap) words[slot] = merge_word(keys[i], idxs[i]);
+    });
+    __syncthreads();
+    const int count = sh_count;
+    if (count >= W && count <= kPruneCap) {
+      const int64_t o = (int64_t)b * W;
+      if (count <= kMergeThreads)
+        emit_sorted<1>(words, count, W, V, scores + o, parents + o, tokens + o, valid + o);
+      else if (count <= 2 * kMergeThreads)
+        emit_sorted<2>(words, count, W, V, scores + o, parents + o, tokens + o, valid + o);
+      else
+        emit_sorted<4>(words, count, W, V, scores + o, parents + o, tokens + o, valid + o);
+      return;
+    }
+    __syncthreads();
+  }
 
   // radix select of the W-th largest key (order32 space), 4 x 8 bits
   uint32_t prefix = 0, pmask = 0;
@@ -1128,7 +1263,7 @@ int launch_merge(const float* cand_key, const int* cand_idx, int B, int ncand, i
                  float* scores, int64_t* parents, int64_t* tokens, void* valid, hipStream_t s) {
   int cap = 1;
   while (cap < W) cap <<= 1;
-  const size_t lds = (size_t)cap * 8;
+  const size_t lds = (size_t)std::max(cap, kPruneCap) * 8;
   if (lds > 64 * 1024) {
     // beyond the default 64 KB of dynamic LDS per workgroup (the CU has 160 KB)
     const hipError_t e = hipFuncSetAttribute((const void*)merge_select_kernel,

@@ -84,6 +84,40 @@ def test_select_level_unsampled_outlier(device):
     _check_selection(logits, scores, W)
 
 
+@pytest.mark.parametrize("ncand,W", [(1, 1), (1000, 1000), (4096, 7), (4097, 300), (5000, 1408),
+                                     (70000, 1408), (70000, 1409), (65536, 256), (8192, 8192)])
+@pytest.mark.parametrize("values", ["distinct", "ties", "masked", "one"])
+def test_merge_equals_stable_sort(device, ncand, W, values):
+    """The request-level stage against a sort by (key descending, flat index
+    ascending): around the sizes it sorts whole, samples and radix-selects, with
+    keys that tie at the cut, keys of masked slots, and one key for all."""
+    from kadllm_amd import _lib
+    from kadllm_amd.grbeam import merge
+    g = torch.Generator().manual_seed(ncand + W)
+    B, V = 2, 4 * ncand  # flat indices below V, of rows of Vr columns
+    Vr = 2 * ncand
+    key = torch.randn(B, ncand, generator=g) * 3 - 20
+    if values == "ties":
+        key = key.round()
+    elif values == "masked":
+        key[torch.rand(B, ncand, generator=g) < 0.9] = -float("inf")
+    elif values == "one":
+        key.fill_(-7.5)
+    idx = torch.stack([torch.randperm(V, generator=g)[:ncand] for _ in range(B)]).int()
+    order = [sorted(range(ncand), key=lambda i: (-k[i], x[i]))[:W]
+             for k, x in zip(key.tolist(), idx.tolist())]
+    order = torch.tensor(order)
+    dk, di = key.to(device), idx.to(device)
+    scores = torch.empty(B, W, device=device)
+    parents, tokens = (torch.empty(B, W, dtype=torch.int64, device=device) for _ in range(2))
+    valid = torch.empty(B, W, dtype=torch.bool, device=device)
+    merge(dk, di, B, ncand, W, Vr, scores, parents, tokens, valid, _lib.stream_of(dk))
+    flat = idx.gather(1, order).long()
+    assert torch.equal(scores.cpu(), key.gather(1, order))
+    assert torch.equal(parents.cpu(), flat // (Vr)) and torch.equal(tokens.cpu(), flat % (Vr))
+    assert torch.equal(valid.cpu(), key.gather(1, order) > -float("inf"))
+
+
 def test_history_update(device):
     B, Wp, step, W = 2, 3, 2, 5
     hist = torch.arange(B * Wp * step).reshape(B, Wp, step)
