@@ -6,14 +6,13 @@
 //   parents = idx // V; tokens = idx % V; history = cat(history[parents], tokens)
 // without materialising any [W, V] fp32 temporary.
 //
-// Stage 1, kad_beam_row_select (one workgroup per beam row): a first pass
-// takes the row max and a 4096-bin histogram of the top 12 bits of the bf16
-// order key of every allowed logit; a second pass sums exp(x - max) for the
-// row's log-sum-exp and resolves the low 4 bits inside the bin that holds the
-// row's K-th largest logit, giving its exact value; a third pass emits exactly
-// the row's K best entries (ties taken in column order).  Within a row the score
-// order is the logit order, so the request's top W is among these rows'
-// top min(W, V) entries.  Keys are ((x - max) - log(sum exp)) + parent in fp32.
+// Stage 1, kad_beam_row_select (one workgroup per beam row): a sampled
+// threshold, one pass for the row max, the sum of exp and the entries past the
+// threshold, and a radix select of exactly the row's K best among those (ties
+// taken in column order); rows that do not thin out so take exact histogram
+// passes over the whole row.  Within a row the score order is the logit order,
+// so the request's top W is among these rows' top min(W, V) entries.  Keys are
+// ((x - max) - log(sum exp)) + parent in fp32.
 //
 // Stage 2, kad_beam_merge_select (one workgroup per request): a sampled
 // threshold keeps a few times W of the request's Wp*K candidates, which are
@@ -29,6 +28,7 @@
 #include "kad_common.h"
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 // Scratch of kad_beam_select_noalloc (32 MiB per GPU; see scratch_address).
@@ -36,7 +36,6 @@ static __device__ __align__(256) uint8_t scratch[32ll << 20];
 
 namespace {
 
-constexpr int kRowThreads = 256;
 constexpr int kBins = 4096;
 
 __device__ __forceinline__ uint32_t order16(uint16_t bits) {
@@ -47,7 +46,8 @@ __device__ __forceinline__ uint32_t order32(float f) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-// block-wide exclusive scan of one int per thread (blockDim = kRowThreads)
+// block-wide exclusive scan of one int per thread (blockDim = NT)
+template <int NT>
 __device__ int block_exclusive_scan(int v, int* scratch, int* total) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int x = v;
@@ -59,7 +59,7 @@ __device__ int block_exclusive_scan(int v, int* scratch, int* total) {
   if (lane == 63) scratch[wave] = x;
   __syncthreads();
   int base = 0, tot = 0;
-  for (int w = 0; w < kRowThreads / 64; ++w) {
+  for (int w = 0; w < NT / 64; ++w) {
     if (w < wave) base += scratch[w];
     tot += scratch[w];
   }
@@ -68,26 +68,27 @@ __device__ int block_exclusive_scan(int v, int* scratch, int* total) {
   return base + x - v;
 }
 
+template <int NT>
 __device__ void row_select_exact(int64_t row,
     const bf16_t* __restrict__ logits, int64_t ld, const uint8_t* __restrict__ mask,
     int64_t ld_mask, const float* __restrict__ parent, int Wp, int V, int K,
     float* __restrict__ cand_key, int* __restrict__ cand_idx, int* hist) {
-  __shared__ int scan_tmp[kRowThreads / 64];
-  __shared__ float red_m[kRowThreads / 64], red_s[kRowThreads / 64];
+  __shared__ int scan_tmp[NT / 64];
+  __shared__ float red_m[NT / 64], red_s[NT / 64];
   __shared__ int sh_bin, sh_above, sh_low;
   __shared__ int sh_emit;
   const int tid = threadIdx.x;
   const bf16_t* x = logits + row * ld;
   const uint8_t* mk = mask ? mask + row * ld_mask : nullptr;
 
-  for (int i = tid; i < kBins; i += kRowThreads) hist[i] = 0;
+  for (int i = tid; i < kBins; i += NT) hist[i] = 0;
   if (tid == 0) sh_emit = 0;
   __syncthreads();
 
   // pass 1: max over all logits (log_softmax normalises before masking);
   // histogram of the order keys of the allowed logits
   float m = -INFINITY;
-  for (int c = tid; c < V; c += kRowThreads) {
+  for (int c = tid; c < V; c += NT) {
     const uint16_t bits = x[c];
     m = fmaxf(m, bf2f(bits));
     const bool ok = mk ? mk[c] != 0 : true;
@@ -97,7 +98,7 @@ __device__ void row_select_exact(int64_t row,
   if ((tid & 63) == 0) red_m[tid >> 6] = m;
   __syncthreads();
   float M = -INFINITY;
-  for (int w = 0; w < kRowThreads / 64; ++w) M = fmaxf(M, red_m[w]);
+  for (int w = 0; w < NT / 64; ++w) M = fmaxf(M, red_m[w]);
 
   // find the bin holding the K-th largest allowed key (masked entries count
   // in bin 0 so that rows with fewer than K allowed logits still yield K)
@@ -112,12 +113,12 @@ __device__ void row_select_exact(int64_t row,
   }
   __syncthreads();
   const int bin = sh_bin;
-  for (int i = tid; i < 16; i += kRowThreads) hist[i] = 0;
+  for (int i = tid; i < 16; i += NT) hist[i] = 0;
   __syncthreads();
 
   // pass 2: exact sum exp(x - M); low-4-bit histogram inside `bin`
   float se = 0.f;
-  for (int c = tid; c < V; c += kRowThreads) {
+  for (int c = tid; c < V; c += NT) {
     const uint16_t bits = x[c];
     se += expf(bf2f(bits) - M);
     const bool ok = mk ? mk[c] != 0 : true;
@@ -138,7 +139,7 @@ __device__ void row_select_exact(int64_t row,
   }
   __syncthreads();
   float SE = 0.f;
-  for (int w = 0; w < kRowThreads / 64; ++w) SE += red_s[w];
+  for (int w = 0; w < NT / 64; ++w) SE += red_s[w];
   const float lse = logf(SE);
   const uint32_t thr = ((uint32_t)bin << 4) | (uint32_t)sh_low;
   const int need_ties = K - sh_above;
@@ -148,9 +149,9 @@ __device__ void row_select_exact(int64_t row,
   int* ci = cand_idx + row * K;
 
   // pass 3: emit entries above the threshold, and the first `need_ties`
-  // threshold entries in column order (tiles of kRowThreads consecutive columns)
+  // threshold entries in column order (tiles of NT consecutive columns)
   int ties_taken = 0;
-  for (int c0 = 0; c0 < V; c0 += kRowThreads) {
+  for (int c0 = 0; c0 < V; c0 += NT) {
     const int c = c0 + tid;
     uint32_t u = 0;
     float v = -INFINITY;
@@ -164,7 +165,7 @@ __device__ void row_select_exact(int64_t row,
     const bool above = c < V && u > thr;
     const bool tie = c < V && u == thr;
     int tot = 0;
-    const int rank = block_exclusive_scan(tie ? 1 : 0, scan_tmp, &tot);
+    const int rank = block_exclusive_scan<NT>(tie ? 1 : 0, scan_tmp, &tot);
     const bool take_tie = tie && (ties_taken + rank < need_ties);
     if (above || take_tie) {
       const int slot = atomicAdd(&sh_emit, 1);
@@ -178,368 +179,6 @@ __device__ void row_select_exact(int64_t row,
   }
 }
 
-
-// LDS candidate capacity: 2048 (16 KB) while about 2K + 256 <= 1024
-// candidates are expected, which leaves room for two workgroups more per CU
-// than 4096 (32 KB); the samples (bf16 keys) and the exact path's 4096-bin
-// histogram alias the same buffer
-constexpr int kCandCapSmall = 2048, kCandCapLarge = 4096;
-constexpr int kLine = 64;                      // logits per 128-byte line
-constexpr int kTargetLines = 128;              // sampled lines per row (~8k samples)
-
-// r-th largest of the keys histogrammed in hist[256] (bin 0 excluded), run by
-// one full wave: lane l owns bins 4l..4l+3.  Returns the bin and, through
-// *above, how many keys lie in higher bins; bin -1 if fewer than r keys.
-__device__ int wave_rank_bin(const int* hist, int r, int* above) {
-  const int lane = threadIdx.x & 63;
-  int b[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) b[i] = (lane == 0 && i == 0) ? 0 : hist[lane * 4 + i];
-  const int t = b[0] + b[1] + b[2] + b[3];
-  int suf = t;  // keys in lanes >= lane
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_down(suf, o, 64);
-    if (lane + o < 64) suf += y;
-  }
-  const uint64_t reach = __ballot(suf >= r);
-  const int L = __popcll(reach) - 1;  // suffix sums fall with the lane: reach is a prefix
-  int bin = -1, acc = 0;
-  if (L >= 0 && lane == L) {
-    acc = suf - t;
-    for (int i = 3; i >= 0; --i) {
-      if (acc + b[i] >= r) {
-        bin = lane * 4 + i;
-        break;
-      }
-      acc += b[i];
-    }
-  }
-  if (L < 0) return -1;
-  *above = __shfl(acc, L, 64);
-  return __shfl(bin, L, 64);
-}
-
-// Fast path, one workgroup per beam row:
-//  1. sample every line_stride-th 128-byte line of the row and take the
-//     rank-th largest sampled key (exact, two 8-bit radix rounds); about
-//     rank * line_stride >= 2K + 256 entries are expected at or above it;
-//  2. one vectorised pass over the row computes the max and the sum of exp
-//     (online rescaling) and gathers every allowed entry at or above the
-//     threshold into LDS;
-//  3. a radix select over the candidates' keys (ties at the K-th key ranked by
-//     column) emits the row's top K, unordered: the merge stage orders them.
-// If fewer than K or more than CAP entries qualify, the exact histogram path
-// runs instead, so the result never depends on the sample.
-template <int CAP, bool MASKED>
-__global__ __launch_bounds__(kRowThreads) void row_select_kernel(
-    const bf16_t* __restrict__ logits, int64_t ld, const uint8_t* __restrict__ mask,
-    int64_t ld_mask, const float* __restrict__ parent, int Wp, int V, int K,
-    float* __restrict__ cand_key, int* __restrict__ cand_idx, int line_stride, int rank) {
-  constexpr int kSampleCap = CAP * 4;   // bf16 sample keys aliasing the candidates
-  static_assert(CAP * 8 >= 4096 * 4, "the exact path's histogram must fit the buffer");
-  __shared__ __attribute__((aligned(16))) uint64_t cand[CAP];
-  __shared__ int hist[256];
-  __shared__ float red_m[kRowThreads / 64], red_s[kRowThreads / 64], red_smax[kRowThreads / 64];
-  __shared__ int sh_count, sh_hi, sh_above, sh_thr;
-  uint16_t* samples = (uint16_t*)cand;
-  const int tid = threadIdx.x;
-  const int64_t row = blockIdx.x;
-  const bf16_t* x = logits + row * ld;
-  // a separate instantiation for unmasked rows drops the mask tests from the
-  // per-logit loop, which is VALU-bound
-  const uint8_t* mk = MASKED ? mask + row * ld_mask : nullptr;
-  const bool vec = (ld % 8) == 0 && (((uintptr_t)logits) % 16) == 0 &&
-                   (!mask || ((ld_mask % 8) == 0 && (((uintptr_t)mask) % 8) == 0));
-  auto key_of = [&](uint16_t bits, int c) -> uint32_t {
-    return (mk && mk[c] == 0) ? 0u : order16(bits);
-  };
-
-  // ---- 1. sample and threshold
-  const int nlines = (V + kLine - 1) / kLine;
-  const int ns = min(kSampleCap, ((nlines + line_stride - 1) / line_stride) * kLine);
-  hist[tid] = 0;
-  if (tid == 0) sh_count = 0;
-  __syncthreads();
-  float smax = -INFINITY;  // max sampled logit (masked or not): the sum's start
-  for (int s = tid; s < ns; s += kRowThreads) {
-    const int c = (s / kLine) * line_stride * kLine + (s % kLine);
-    uint32_t k = 0u;
-    if (c < V) {
-      const uint16_t bits = x[c];
-      k = key_of(bits, c);
-      smax = fmaxf(smax, bf2f(bits));
-    }
-    samples[s] = (uint16_t)k;
-    atomicAdd(&hist[k >> 8], 1);
-  }
-  smax = wave_max(smax);
-  if ((tid & 63) == 0) red_smax[tid >> 6] = smax;
-  __syncthreads();
-  if (tid < 64) {
-    int above = 0;
-    const int hi = wave_rank_bin(hist, rank, &above);
-    if (tid == 0) {
-      sh_hi = hi;
-      sh_above = above;
-    }
-  }
-  __syncthreads();
-  const int hi = sh_hi;
-  if (hi > 0) {
-    hist[tid] = 0;
-    __syncthreads();
-    for (int s = tid; s < ns; s += kRowThreads) {
-      const uint32_t k = samples[s];
-      if ((int)(k >> 8) == hi) atomicAdd(&hist[k & 255], 1);
-    }
-    __syncthreads();
-    if (tid < 64) {
-      // bin 0 of this round is a real key (hi > 0): count it
-      const int lane = tid;
-      int b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) b[i] = hist[lane * 4 + i];
-      const int t = b[0] + b[1] + b[2] + b[3];
-      int suf = t;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_down(suf, o, 64);
-        if (lane + o < 64) suf += y;
-      }
-      const int need = rank - sh_above;
-      const uint64_t reach = __ballot(suf >= need);
-      const int L = __popcll(reach) - 1;  // need <= keys in bin hi, so L >= 0
-      if (lane == L) {
-        int acc = suf - t, lo = 0;
-        for (int i = 3; i >= 0; --i) {
-          if (acc + b[i] >= need) {
-            lo = lane * 4 + i;
-            break;
-          }
-          acc += b[i];
-        }
-        sh_thr = (hi << 8) | lo;
-      }
-    }
-  } else if (tid == 0) {
-    sh_thr = 0;
-  }
-  __syncthreads();
-  const uint32_t thr = (uint32_t)sh_thr;
-
-  // ---- 2. max, sum exp, and candidates >= thr in one pass.  The sum is taken
-  // against a fixed reference, the sample max (each term one fma and the
-  // hardware exp2: exp(v - m) = 2^(v log2 e - m log2 e)); a row whose true max
-  // exceeds it by more than 60 sums again against the true max.  Candidates
-  // are screened with a float compare against the threshold's value and
-  // confirmed on the order key.
-  constexpr float kLog2e = 1.4426950408889634f;
-  float mref = -INFINITY;
-  for (int w = 0; w < kRowThreads / 64; ++w) mref = fmaxf(mref, red_smax[w]);
-  if (mref == -INFINITY) mref = 0.f;
-  float m = -INFINITY, se = 0.f;
-  float nb = -mref * kLog2e;
-  const uint32_t tb = thr & 0x8000u ? (thr & 0x7fffu) : (~thr & 0xffffu);
-  const float tf = thr > 0 ? bf2f((uint16_t)tb) : INFINITY;
-  auto visit = [&](uint16_t bits, int c, bool ok) {
-    const float v = bf2f(bits);
-    m = fmaxf(m, v);
-    se += __builtin_amdgcn_exp2f(fmaf(v, kLog2e, nb));
-    if (v >= tf && ok) {
-      const uint32_t u = order16(bits);
-      if (u >= thr) {
-        const int slot = atomicAdd(&sh_count, 1);
-        if (slot < CAP) cand[slot] = ((uint64_t)u << 32) | (uint64_t)(0xffffffffu - (uint32_t)c);
-      }
-    }
-  };
-  const int V8 = vec ? V / 8 : 0;
-  constexpr int kUnroll = 4;
-  int c8 = tid;
-  for (; c8 + (kUnroll - 1) * kRowThreads < V8; c8 += kUnroll * kRowThreads) {
-    u32x4 r[kUnroll];
-    u32x2 mr[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      r[u] = *(const u32x4*)(x + (c8 + u * kRowThreads) * 8);
-      if (mk) mr[u] = *(const u32x2*)(mk + (c8 + u * kRowThreads) * 8);
-    }
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int c = (c8 + u * kRowThreads) * 8;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool ok0 = mk ? ((mr[u][e / 2] >> (16 * (e % 2))) & 0xffu) != 0 : true;
-        const bool ok1 = mk ? ((mr[u][e / 2] >> (16 * (e % 2) + 8)) & 0xffu) != 0 : true;
-        visit((uint16_t)(r[u][e] & 0xffffu), c + 2 * e, ok0);
-        visit((uint16_t)(r[u][e] >> 16), c + 2 * e + 1, ok1);
-      }
-    }
-  }
-  for (; c8 < V8; c8 += kRowThreads) {
-    const u32x4 r = *(const u32x4*)(x + c8 * 8);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      visit((uint16_t)(r[e] & 0xffffu), c8 * 8 + 2 * e, mk ? mk[c8 * 8 + 2 * e] != 0 : true);
-      visit((uint16_t)(r[e] >> 16), c8 * 8 + 2 * e + 1, mk ? mk[c8 * 8 + 2 * e + 1] != 0 : true);
-    }
-  }
-  for (int c = V8 * 8 + tid; c < V; c += kRowThreads) visit(x[c], c, mk ? mk[c] != 0 : true);
-  {
-    const float mm = wave_max(m), ss = wave_sum(se);
-    if ((tid & 63) == 0) {
-      red_m[tid >> 6] = mm;
-      red_s[tid >> 6] = ss;
-    }
-  }
-  __syncthreads();
-  float M = -INFINITY;
-  for (int w = 0; w < kRowThreads / 64; ++w) M = fmaxf(M, red_m[w]);
-  float SE = 0.f;
-  for (int w = 0; w < kRowThreads / 64; ++w) SE += red_s[w];
-  if (M > mref + 60.f) {
-    // the sample missed the top by far: sum again against the true max
-    __syncthreads();
-    mref = M;
-    nb = -mref * kLog2e;
-    float s2 = 0.f;
-    for (int c = tid; c < V; c += kRowThreads) s2 += __builtin_amdgcn_exp2f(fmaf(bf2f(x[c]), kLog2e, nb));
-    s2 = wave_sum(s2);
-    if ((tid & 63) == 0) red_s[tid >> 6] = s2;
-    __syncthreads();
-    SE = 0.f;
-    for (int w = 0; w < kRowThreads / 64; ++w) SE += red_s[w];
-  }
-  // log sum exp(v - M) = log(sum exp(v - mref)) + (mref - M)
-  const float lse = logf(SE) + (mref - M);
-  const int count = sh_count;
-  if (thr == 0 || count < K || count > CAP) {
-    // exact fallback: reuses the candidate buffer as the 4096-bin histogram
-    __syncthreads();
-    row_select_exact(row, logits, ld, mask, ld_mask, parent, Wp, V, K, cand_key, cand_idx,
-                     (int*)cand);
-    return;
-  }
-  // ---- 3. exact top K of the candidates (the merge stage orders them; the
-  // row's output order is free).  Candidate = (order key u << 32) | ~column,
-  // unique per column: a radix select over u (two 8-bit rounds) finds the
-  // K-th largest key u*; the ties at u* are ranked by column.
-  const float p = parent[row];
-  const int r_local = (int)(row % Wp);
-  int* bins = hist;  // 256 ints
-  auto select_bin = [&](int need_in, int* above_out) -> int {
-    // one wave: the bin holding the need_in-th largest entry of bins[]
-    if (tid < 64) {
-      int above = 0;
-      int b = -1;
-      {
-        const int lane = tid;
-        int v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = bins[lane * 4 + i];
-        const int t = v[0] + v[1] + v[2] + v[3];
-        int suf = t;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const int y = __shfl_down(suf, o, 64);
-          if (lane + o < 64) suf += y;
-        }
-        const uint64_t reach = __ballot(suf >= need_in);
-        const int L = __popcll(reach) - 1;
-        int acc = 0;
-        if (lane == L) {
-          acc = suf - t;
-          for (int i = 3; i >= 0; --i) {
-            if (acc + v[i] >= need_in) {
-              b = lane * 4 + i;
-              break;
-            }
-            acc += v[i];
-          }
-        }
-        above = __shfl(acc, L, 64);
-        b = __shfl(b, L, 64);
-      }
-      if (tid == 0) {
-        sh_hi = b;
-        sh_above = above;
-      }
-    }
-    __syncthreads();
-    *above_out = sh_above;
-    return sh_hi;
-  };
-  // round 1: high byte of u
-  bins[tid] = 0;
-  __syncthreads();
-  for (int i = tid; i < count; i += kRowThreads) atomicAdd(&bins[(uint32_t)(cand[i] >> 40) & 255], 1);
-  __syncthreads();
-  int above1;
-  const int b1 = select_bin(K, &above1);
-  __syncthreads();
-  // round 2: low byte of u inside bin b1
-  bins[tid] = 0;
-  __syncthreads();
-  for (int i = tid; i < count; i += kRowThreads) {
-    const uint32_t u = (uint32_t)(cand[i] >> 32);
-    if ((int)(u >> 8) == b1) atomicAdd(&bins[u & 255], 1);
-  }
-  __syncthreads();
-  int above2;
-  const int b2 = select_bin(K - above1, &above2);
-  const uint32_t ustar = ((uint32_t)b1 << 8) | (uint32_t)b2;
-  const int need = K - above1 - above2;  // ties at u* to take, lowest columns first
-  auto emit = [&](uint64_t e) {
-    const int slot = atomicAdd(&sh_count, 1);
-    const int c = (int)(0xffffffffu - (uint32_t)e);
-    const float v = bf2f(x[c]);
-    if (slot < K) {  // exactly K qualify; the bound only guards memory
-      cand_key[row * K + slot] = ((v - M) - lse) + p;
-      cand_idx[row * K + slot] = r_local * V + c;
-    }
-  };
-  // keys above u* are taken; the ties at u* (their ~column words) are gathered
-  uint32_t* ties = (uint32_t*)bins;
-  if (tid == 0) {
-    sh_count = 0;
-    sh_thr = 0;  // number of ties
-  }
-  __syncthreads();
-  for (int i = tid; i < count; i += kRowThreads) {
-    const uint64_t e = cand[i];
-    const uint32_t u = (uint32_t)(e >> 32);
-    if (u > ustar) {
-      emit(e);
-    } else if (u == ustar) {
-      const int t = atomicAdd(&sh_thr, 1);
-      if (t < 256) ties[t] = (uint32_t)e;
-    }
-  }
-  __syncthreads();
-  const int nties = sh_thr;
-  if (nties <= 256) {
-    // rank of each tie = ties with a lower column (a larger ~column word)
-    for (int t = tid; t < nties; t += kRowThreads) {
-      const uint32_t me = ties[t];
-      int rank_t = 0;
-      for (int j = 0; j < nties; ++j) rank_t += ties[j] > me ? 1 : 0;
-      if (rank_t < need) emit(((uint64_t)ustar << 32) | me);
-    }
-  } else {
-    // many equal keys: rank every tie against the whole candidate list
-    for (int i = tid; i < count; i += kRowThreads) {
-      const uint64_t e = cand[i];
-      if ((uint32_t)(e >> 32) != ustar) continue;
-      int rank_t = 0;
-      for (int j = 0; j < count; ++j) {
-        const uint64_t f = cand[j];
-        rank_t += ((uint32_t)(f >> 32) == ustar && (uint32_t)f > (uint32_t)e) ? 1 : 0;
-      }
-      if (rank_t < need) emit(e);
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 constexpr int kMergeThreads = 1024;
@@ -590,43 +229,48 @@ __device__ __forceinline__ bool pick_bin(const int* hist, int need, int lane, in
   return lane == L;  // the lane that holds the result
 }
 
-// Rows of fp32 or fp16 logits (the reference upcasts any float dtype before
-// its log-softmax, src/kadllm/grbeam.py:91), one workgroup per row, exact:
-// the row max, the sum of exp(x - max), four 8-bit radix rounds over the
+// LDS candidate capacity: 2048 (16 KB) while about 2K + 256 <= 1024
+// candidates are expected, which leaves room for two workgroups more per CU
+// than 4096 (32 KB); the exact paths' histograms alias the buffer
+constexpr int kCandCapSmall = 2048, kCandCapLarge = 4096;
+constexpr int kLine = 64;                      // logits per sampled line
+constexpr int kTargetLines = 128;              // sampled lines per row (~8k samples)
+
+// A row of fp32 or fp16 logits (the reference upcasts any float dtype before
+// its log-softmax, src/kadllm/grbeam.py:91), exact without a threshold: the row max, the sum of exp(x - max), four 8-bit radix rounds over the
 // order keys of the row's scores key = ((x - max) - lse) + parent (-inf where
 // masked) for the K-th largest, then one pass that emits every key above it
 // and the first ties in column order.  Each pass recomputes the keys with the
 // same operations, so every pass sees the same values.
-__global__ __launch_bounds__(kRowThreads) void row_select_float_kernel(
-    const void* __restrict__ logits, int dtype, int64_t ld, const uint8_t* __restrict__ mask,
-    int64_t ld_mask, const float* __restrict__ parent, int Wp, int V, int K,
-    float* __restrict__ cand_key, int* __restrict__ cand_idx) {
-  __shared__ int hist[256];
-  __shared__ int scan_tmp[kRowThreads / 64];
-  __shared__ float red[kRowThreads / 64];
+template <int NT>
+__device__ void row_select_exact_float(
+    int64_t row, const void* __restrict__ logits, int dtype, int64_t ld,
+    const uint8_t* __restrict__ mask, int64_t ld_mask, const float* __restrict__ parent, int Wp,
+    int V, int K, float* __restrict__ cand_key, int* __restrict__ cand_idx, int* hist) {
+  __shared__ int scan_tmp[NT / 64];
+  __shared__ float red[NT / 64];
   __shared__ uint32_t sh_prefix;
   __shared__ int sh_need, sh_emit;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t row = blockIdx.x;
   const int64_t xrow = row * ld;
   const uint8_t* mk = mask ? mask + row * ld_mask : nullptr;
 
   float m = -INFINITY;
-  for (int c = tid; c < V; c += kRowThreads) m = fmaxf(m, load_as_float(logits, xrow + c, dtype));
+  for (int c = tid; c < V; c += NT) m = fmaxf(m, load_as_float(logits, xrow + c, dtype));
   m = wave_max(m);
   if (lane == 0) red[wave] = m;
   __syncthreads();
   float M = -INFINITY;
-  for (int w = 0; w < kRowThreads / 64; ++w) M = fmaxf(M, red[w]);
+  for (int w = 0; w < NT / 64; ++w) M = fmaxf(M, red[w]);
   __syncthreads();
   float se = 0.f;
-  for (int c = tid; c < V; c += kRowThreads) se += expf(load_as_float(logits, xrow + c, dtype) - M);
+  for (int c = tid; c < V; c += NT) se += expf(load_as_float(logits, xrow + c, dtype) - M);
   se = wave_sum(se);
   if (lane == 0) red[wave] = se;
   if (tid == 0) sh_emit = 0;
   __syncthreads();
   float SE = 0.f;
-  for (int w = 0; w < kRowThreads / 64; ++w) SE += red[w];
+  for (int w = 0; w < NT / 64; ++w) SE += red[w];
   const float lse = logf(SE);
   const float p = parent[row];
   auto key_at = [&](int c) -> float {
@@ -637,9 +281,9 @@ __global__ __launch_bounds__(kRowThreads) void row_select_float_kernel(
   uint32_t prefix = 0, pmask = 0;
   int need = K;
   for (int shift = 24; shift >= 0; shift -= 8) {
-    hist[tid] = 0;  // kRowThreads == 256 bins
+    if (tid < 256) hist[tid] = 0;
     __syncthreads();
-    for (int c = tid; c < V; c += kRowThreads) {
+    for (int c = tid; c < V; c += NT) {
       const uint32_t u = order32(key_at(c));
       if ((u & pmask) == prefix) atomicAdd(&hist[(u >> shift) & 255], 1);
     }
@@ -662,7 +306,7 @@ __global__ __launch_bounds__(kRowThreads) void row_select_float_kernel(
   float* ck = cand_key + row * K;
   int* ci = cand_idx + row * K;
   int ties_taken = 0;
-  for (int c0 = 0; c0 < V; c0 += kRowThreads) {
+  for (int c0 = 0; c0 < V; c0 += NT) {
     const int c = c0 + tid;
     float key = -INFINITY;
     uint32_t u = 0;
@@ -673,7 +317,7 @@ __global__ __launch_bounds__(kRowThreads) void row_select_float_kernel(
     const bool above = c < V && u > kth;
     const bool tie = c < V && u == kth;
     int tot = 0;
-    const int rank = block_exclusive_scan(tie ? 1 : 0, scan_tmp, &tot);
+    const int rank = block_exclusive_scan<NT>(tie ? 1 : 0, scan_tmp, &tot);
     if (above || (tie && ties_taken + rank < need)) {
       const int slot = atomicAdd(&sh_emit, 1);
       if (slot < K) {  // exactly K entries qualify; the bound only guards memory
@@ -685,6 +329,340 @@ __global__ __launch_bounds__(kRowThreads) void row_select_float_kernel(
   }
 }
 
+
+// inverse of order32
+__device__ __forceinline__ float unorder32(uint32_t u) {
+  return __uint_as_float((u & 0x80000000u) ? u ^ 0x80000000u : ~u);
+}
+
+// Row selection, one workgroup of NT threads per beam row:
+//  1. the max of each 16-byte word of a sample (every line_stride-th 64-logit
+//     line) and, by a binary search over the order key's bits, the rank-th
+//     largest of these maxima: about 2K + 256 entries of the row are at or
+//     above it.  (Taking maxima first leaves a few keys per thread, counted by
+//     ballots; a histogram of the samples serialises on the few LDS bins that
+//     the top byte of similar logits falls in.)
+//  2. one vectorised pass over the row computes the max and the sum of exp
+//     and gathers every allowed entry at or above the threshold into LDS;
+//  3. a radix select over the candidates' keys (ties at the K-th key ranked by
+//     column) emits the row's top K, unordered: the merge stage orders them.
+// Rows of at most CAP columns are all candidates.  If fewer than K or more
+// than CAP entries qualify, the exact path runs instead, so the result never
+// depends on the sample.  bf16 rows are ranked by logit; of fp32 and fp16 ones,
+// whose logits may differ and their fp32 keys not, the keys are ranked, and the
+// K-th must exceed the threshold's own key, below which nothing was gathered.
+// NT: 1,024 threads where the rows number at most two per CU (one row on a CU
+// is bound by the loads its waves keep in flight: 8 rows of 248,320 bf16
+// logits 96 -> 35 us), else 256 (2,048 rows 272 -> 246 us, 4.1 TB/s; of fp32, by
+// six passes before, 7.3 ms -> 0.43).
+template <typename T, int CAP, bool MASKED, int NT>
+__global__ __launch_bounds__(NT) void row_select_kernel(
+    const T* __restrict__ logits, int64_t ld, const uint8_t* __restrict__ mask, int64_t ld_mask,
+    const float* __restrict__ parent, int Wp, int V, int K, float* __restrict__ cand_key,
+    int* __restrict__ cand_idx, int line_stride, int rank) {
+  constexpr bool kBf16 = Elem<T>::code == KAD_DTYPE_BF16;
+  constexpr int VE = 16 / sizeof(T);                     // logits per 16-byte word
+  constexpr int kRounds = kBf16 ? 2 : 4;                 // key bytes that differ
+  constexpr int kPer = kLine / VE;                       // words per line
+  constexpr int kGroups = 2 * kTargetLines * kPer / NT;  // fewer than 2 kTargetLines lines
+  typedef T word_t __attribute__((ext_vector_type(VE)));
+  typedef uint8_t mword_t __attribute__((ext_vector_type(VE)));
+  static_assert(CAP * 8 >= kBins * 4, "the exact path's histogram must fit the buffer");
+  __shared__ __attribute__((aligned(16))) uint64_t cand[CAP];
+  __shared__ int bins[256];
+  __shared__ float red_m[NT / 64], red_s[NT / 64], red_smax[NT / 64];
+  __shared__ int sh_reach[32];
+  __shared__ int sh_count, sh_hi, sh_above, sh_ties;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t row = blockIdx.x;
+  const T* x = logits + row * ld;
+  // a separate instantiation for unmasked rows drops the mask tests from the
+  // per-logit loop, which is VALU-bound
+  const uint8_t* mk = MASKED ? mask + row * ld_mask : nullptr;
+  // words start at column head, the row's first 16-byte boundary (rows of an
+  // odd vocabulary begin anywhere)
+  const int head = (int)((16 - (uintptr_t)x % 16) % 16 / sizeof(T));
+  const bool mvec = MASKED && ((uintptr_t)(mk + head) % VE) == 0;
+  auto mask_word = [&](int c) {
+    mword_t mw;
+    if (mvec) {
+      mw = *(const mword_t*)(mk + c);
+    } else {
+#pragma unroll
+      for (int e = 0; e < VE; ++e) mw[e] = mk[c + e];
+    }
+    return mw;
+  };
+  // the word at column c; where that lies outside the row, -inf and not allowed
+  auto load = [&](int c, float (&v)[VE], bool (&ok)[VE]) {
+    if (c >= 0 && c + VE <= V) {
+      const word_t w = *(const word_t*)(x + c);
+      mword_t mw;
+      if constexpr (MASKED) mw = mask_word(c);
+#pragma unroll
+      for (int e = 0; e < VE; ++e) {
+        v[e] = Elem<T>::to_f(w[e]);
+        ok[e] = MASKED ? mw[e] != 0 : true;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < VE; ++e) {
+        const bool in = c + e >= 0 && c + e < V;
+        v[e] = in ? Elem<T>::to_f(x[c + e]) : -INFINITY;
+        ok[e] = in && (!MASKED || mk[c + e] != 0);
+      }
+    }
+  };
+
+  // a bf16 logit's order key is the top half of its word
+  auto order_of = [](float v) { return order32(v) & (kBf16 ? 0xffff0000u : 0xffffffffu); };
+  auto value_of = [](uint32_t u) {
+    const float v = unorder32(u);
+    return kBf16 ? __uint_as_float(__float_as_uint(v) & 0xffff0000u) : v;
+  };
+
+  // ---- 1. sample and threshold (order key, low bits zero)
+  if (tid < 32) sh_reach[tid] = 0;
+  if (tid == 0) sh_count = 0;
+  float smax = -INFINITY;  // max sampled logit (masked or not): the sum's start
+  uint32_t thr = 0;
+  const bool whole = V <= CAP;
+  {
+    const int nlines = (V + kLine - 1) / kLine;
+    const int ng = ((nlines + line_stride - 1) / line_stride) * kPer;
+    uint32_t u[kGroups];
+#pragma unroll
+    for (int i = 0; i < kGroups; ++i) {
+      const int g = tid + i * NT;
+      u[i] = 0u;
+      if (g >= ng) continue;
+      float v[VE];
+      bool ok[VE];
+      load(head + (g / kPer) * line_stride * kLine + (g % kPer) * VE, v, ok);
+      float best = -INFINITY;
+      bool any = false;
+#pragma unroll
+      for (int e = 0; e < VE; ++e) {
+        smax = fmaxf(smax, v[e]);
+        if (ok[e]) {
+          best = fmaxf(best, v[e]);
+          any = true;
+        }
+      }
+      if (any) u[i] = order_of(best);
+    }
+    smax = wave_max(smax);
+    if (lane == 0) red_smax[tid >> 6] = smax;
+    __syncthreads();
+    if (!whole) {
+#pragma unroll 1
+      for (int bit = 31; bit >= (kBf16 ? 16 : 12); --bit) {
+        const uint32_t t = thr | (1u << bit);
+        int c = 0;
+#pragma unroll
+        for (int i = 0; i < kGroups; ++i) c += (int)__popcll(__ballot(u[i] >= t));
+        if (lane == 0) atomicAdd(&sh_reach[bit], c);
+        __syncthreads();
+        if (sh_reach[bit] >= rank) thr = t;
+      }
+    }
+  }
+  // order key 0 (too few allowed samples): the exact path below
+  const float tf = whole ? -INFINITY : (thr ? value_of(thr) : INFINITY);
+
+  // ---- 2. max, sum exp, and candidates >= thr in one pass.  The sum is taken
+  // against a fixed reference, the sample max (each term one fma and the
+  // hardware exp2: exp(v - m) = 2^(v log2 e - m log2 e)); a row whose true max
+  // exceeds it by more than 60 sums again against the true max.
+  constexpr float kLog2e = 1.4426950408889634f;
+  float mref = -INFINITY;
+  for (int w = 0; w < NT / 64; ++w) mref = fmaxf(mref, red_smax[w]);
+  if (mref == -INFINITY) mref = 0.f;
+  float m = -INFINITY, se = 0.f;
+  float nb = -mref * kLog2e;
+  // fp32 and fp16 terms from the exact difference, an instruction more
+  auto term = [&](float v) {
+    return __builtin_amdgcn_exp2f(kBf16 ? fmaf(v, kLog2e, nb) : (v - mref) * kLog2e);
+  };
+  auto visit = [&](int c, const float (&v)[VE], const bool (&ok)[VE]) {
+    float mx = v[0];
+#pragma unroll
+    for (int e = 1; e < VE; ++e) mx = fmaxf(mx, v[e]);
+    m = fmaxf(m, mx);
+#pragma unroll
+    for (int e = 0; e < VE; ++e) se += term(v[e]);
+    if (mx >= tf) {
+#pragma unroll
+      for (int e = 0; e < VE; ++e)
+        if (v[e] >= tf && ok[e]) {
+          const int slot = atomicAdd(&sh_count, 1);
+          if (slot < CAP)
+            cand[slot] = ((uint64_t)order_of(v[e]) << 32) | (uint32_t)~(uint32_t)(c + e);
+        }
+    }
+  };
+  auto visit_at = [&](int c) {
+    float v[VE];
+    bool ok[VE];
+    load(c, v, ok);
+    visit(c, v, ok);
+  };
+  constexpr int kUnroll = 4, kStep = NT * VE;
+  if (tid == 0 && head > 0) visit_at(head - VE);
+  int c0 = head + tid * VE;
+  for (; c0 + (kUnroll - 1) * kStep + VE <= V; c0 += kUnroll * kStep) {
+    word_t r[kUnroll];
+    mword_t mr[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      r[u] = *(const word_t*)(x + c0 + u * kStep);
+      if constexpr (MASKED) mr[u] = mask_word(c0 + u * kStep);
+    }
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      float v[VE];
+      bool ok[VE];
+#pragma unroll
+      for (int e = 0; e < VE; ++e) {
+        v[e] = Elem<T>::to_f(r[u][e]);
+        ok[e] = MASKED ? mr[u][e] != 0 : true;
+      }
+      visit(c0 + u * kStep, v, ok);
+    }
+  }
+  for (; c0 < V; c0 += kStep) visit_at(c0);
+  {
+    const float mm = wave_max(m), ss = wave_sum(se);
+    if (lane == 0) {
+      red_m[tid >> 6] = mm;
+      red_s[tid >> 6] = ss;
+    }
+  }
+  __syncthreads();
+  float M = -INFINITY;
+  for (int w = 0; w < NT / 64; ++w) M = fmaxf(M, red_m[w]);
+  float SE = 0.f;
+  for (int w = 0; w < NT / 64; ++w) SE += red_s[w];
+  if (M > mref + 60.f) {
+    // the sample missed the top by far: sum again against the true max
+    __syncthreads();
+    mref = M;
+    nb = -mref * kLog2e;
+    float s2 = 0.f;
+    for (int c = tid; c < V; c += NT) s2 += term(Elem<T>::to_f(x[c]));
+    s2 = wave_sum(s2);
+    if (lane == 0) red_s[tid >> 6] = s2;
+    __syncthreads();
+    SE = 0.f;
+    for (int w = 0; w < NT / 64; ++w) SE += red_s[w];
+  }
+  // bf16: log sum exp(v - M) = log(sum exp(v - mref)) + (mref - M); fp32 and fp16
+  // keys are taken from mref, a rounding less
+  if constexpr (!kBf16) M = mref;
+  const float lse = logf(SE) + (mref - M);
+  const int count = sh_count;
+  const float p = parent[row];
+  auto exact = [&] {
+    __syncthreads();
+    if constexpr (kBf16)
+      row_select_exact<NT>(row, logits, ld, mask, ld_mask, parent, Wp, V, K, cand_key, cand_idx,
+                           (int*)cand);
+    else
+      row_select_exact_float<NT>(row, logits, Elem<T>::code, ld, mask, ld_mask, parent, Wp, V, K,
+                                 cand_key, cand_idx, (int*)cand);
+  };
+  if ((!whole && thr == 0) || count < K || count > CAP) return exact();
+
+  // ---- 3. exact top K of the candidates (the merge stage orders them; the
+  // row's output order is free).  Candidate = (order key << 32) | ~column,
+  // unique per column: a radix select over the key finds the K-th largest,
+  // u*; the ties at u* are ranked by column.
+  auto key_of = [&](float v) { return ((v - M) - lse) + p; };
+  if constexpr (!kBf16) {
+    for (int i = tid; i < count; i += NT) {
+      const uint64_t e = cand[i];
+      cand[i] = ((uint64_t)order32(key_of(value_of((uint32_t)(e >> 32))) + 0.f) << 32) |
+                (uint32_t)e;
+    }
+  }
+  uint32_t ustar = 0, umask = 0;
+  int need = K;  // rank of the K-th within the current prefix class
+  for (int round = 0; round < kRounds; ++round) {
+    const int shift = 24 - 8 * round;
+    __syncthreads();
+    if (tid < 256) bins[tid] = 0;
+    __syncthreads();
+    for (int i = tid; i < count; i += NT) {
+      const uint32_t u = (uint32_t)(cand[i] >> 32);
+      if ((u & umask) == ustar) atomicAdd(&bins[(u >> shift) & 255], 1);
+    }
+    __syncthreads();
+    if (tid < 64) {
+      int d = 0, acc = 0;
+      if (pick_bin<true>(bins, need, tid, d, acc)) {
+        sh_hi = d;
+        sh_above = acc;
+      }
+    }
+    __syncthreads();
+    ustar |= (uint32_t)sh_hi << shift;
+    umask |= 255u << shift;
+    need -= sh_above;
+  }
+  if constexpr (!kBf16) {
+    if (!whole && ustar <= order32(key_of(tf) + 0.f)) return exact();
+  }
+  const int r_local = (int)(row % Wp);
+  auto emit = [&](uint64_t e) {
+    const int slot = atomicAdd(&sh_count, 1);
+    const float f = value_of((uint32_t)(e >> 32));
+    if (slot < K) {  // exactly K qualify; the bound only guards memory
+      cand_key[row * K + slot] = kBf16 ? key_of(f) : f;
+      cand_idx[row * K + slot] = r_local * V + (int)~(uint32_t)e;
+    }
+  };
+  // keys above u* are taken; the ties at u* (their ~column words) are gathered
+  uint32_t* ties = (uint32_t*)bins;
+  __syncthreads();
+  if (tid == 0) {
+    sh_count = 0;
+    sh_ties = 0;
+  }
+  __syncthreads();
+  for (int i = tid; i < count; i += NT) {
+    const uint64_t e = cand[i];
+    const uint32_t u = (uint32_t)(e >> 32);
+    if (u > ustar) {
+      emit(e);
+    } else if (u == ustar) {
+      const int t = atomicAdd(&sh_ties, 1);
+      if (t < 256) ties[t] = (uint32_t)e;
+    }
+  }
+  __syncthreads();
+  const int nties = sh_ties;
+  if (nties <= 256) {
+    // rank of each tie = ties with a lower column (a larger ~column word)
+    for (int t = tid; t < nties; t += NT) {
+      const uint32_t me = ties[t];
+      int rank_t = 0;
+      for (int j = 0; j < nties; ++j) rank_t += ties[j] > me ? 1 : 0;
+      if (rank_t < need) emit(((uint64_t)ustar << 32) | me);
+    }
+  } else {
+    // many equal keys: rank every tie against the whole candidate list
+    for (int i = tid; i < count; i += NT) {
+      const uint64_t e = cand[i];
+      if ((uint32_t)(e >> 32) != ustar) continue;
+      int rank_t = 0;
+      for (int j = 0; j < count; ++j) {
+        const uint64_t f = cand[j];
+        rank_t += ((uint32_t)(f >> 32) == ustar && (uint32_t)f > (uint32_t)e) ? 1 : 0;
+      }
+      if (rank_t < need) emit(e);
+    }
+  }
+}
 // hist[bin] += 1 for the active lanes.  The merge's keys are cumulative
 // log-probabilities of one request, so its first radix rounds put nearly
 // every key in one or two bins, where one atomic per lane serialises on a
@@ -1233,28 +1211,41 @@ __global__ __launch_bounds__(256) void gather_beam_rows_kernel(
 int launch_row_select(const void* logits, int logits_dtype, int64_t ld, const void* mask,
                       int64_t ld_mask, const float* parent_scores, int rows, int Wp, int V,
                       int K, float* cand_key, int* cand_idx, hipStream_t s) {
-  if (logits_dtype != KAD_DTYPE_BF16) {
-    hipLaunchKernelGGL(row_select_float_kernel, dim3(rows), dim3(kRowThreads), 0, s, logits,
-                       logits_dtype, ld, (const uint8_t*)mask, ld_mask, parent_scores, Wp, V, K,
-                       cand_key, cand_idx);
-    return kad_launch_status("row_select_float_kernel");
-  }
-  // sample ~kTargetLines lines; rank chosen so that rank * line_stride >= 2K + 256
+  // sample ~kTargetLines lines: about rank * line_stride = 2K + 256 entries of
+  // the row are at or above the rank-th largest sample.  Of the n word maxima
+  // about n (1 - e^(-rank / n)) are.
   const int nlines = (V + kLine - 1) / kLine;
   const int line_stride = nlines > kTargetLines ? nlines / kTargetLines : 1;
-  const int rank = (int)kad_cdiv(2 * (int64_t)K + 256, line_stride);
-#define KAD_ROW_SELECT(CAP, MASKED)                                                        \
-  hipLaunchKernelGGL((row_select_kernel<CAP, MASKED>), dim3(rows), dim3(kRowThreads), 0, s,  \
-                     (const bf16_t*)logits, ld, (const uint8_t*)mask, ld_mask, parent_scores,  \
-                     Wp, V, K, cand_key, cand_idx, line_stride, rank)
+  const double samples = (double)kad_cdiv(2 * (int64_t)K + 256, line_stride);
+  const double words = (double)kad_cdiv(nlines, line_stride) * kLine /
+                       (logits_dtype == KAD_DTYPE_F32 ? 4 : 8);
+  const int rank = (int)std::ceil(words * (1.0 - std::exp(-samples / words)));
   const bool small = 2 * (int64_t)K + 256 <= kCandCapSmall / 2;
-  if (mask) {
-    if (small) KAD_ROW_SELECT(kCandCapSmall, true);
-    else KAD_ROW_SELECT(kCandCapLarge, true);
-  } else {
-    if (small) KAD_ROW_SELECT(kCandCapSmall, false);
-    else KAD_ROW_SELECT(kCandCapLarge, false);
+  const bool few = rows <= 512;
+#define KAD_ROW_SELECT(T, CAP, MASKED, NT)                                                      \
+  hipLaunchKernelGGL((row_select_kernel<T, CAP, MASKED, NT>), dim3(rows), dim3(NT), 0, s,       \
+                     (const T*)logits, ld, (const uint8_t*)mask, ld_mask, parent_scores, Wp, V, \
+                     K, cand_key, cand_idx, line_stride, rank)
+#define KAD_ROW_SELECT_NT(T, CAP, MASKED)                \
+  if (few) KAD_ROW_SELECT(T, CAP, MASKED, 1024);         \
+  else KAD_ROW_SELECT(T, CAP, MASKED, 256)
+#define KAD_ROW_SELECT_T(T)                                         \
+  if (mask) {                                                       \
+    if (small) { KAD_ROW_SELECT_NT(T, kCandCapSmall, true); }       \
+    else { KAD_ROW_SELECT_NT(T, kCandCapLarge, true); }             \
+  } else {                                                          \
+    if (small) { KAD_ROW_SELECT_NT(T, kCandCapSmall, false); }      \
+    else { KAD_ROW_SELECT_NT(T, kCandCapLarge, false); }            \
   }
+  if (logits_dtype == KAD_DTYPE_BF16) {
+    KAD_ROW_SELECT_T(bf16_t)
+  } else if (logits_dtype == KAD_DTYPE_F32) {
+    KAD_ROW_SELECT_T(float)
+  } else {
+    KAD_ROW_SELECT_T(_Float16)
+  }
+#undef KAD_ROW_SELECT_T
+#undef KAD_ROW_SELECT_NT
 #undef KAD_ROW_SELECT
   return kad_launch_status("row_select_kernel");
 }

@@ -203,6 +203,44 @@ def test_triton_conv_backend_requires_width4_silu_nobias(device):
                           activation=None, backend="triton")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("B,Wp,V,width,masked", [
+    (2, 3, 4095, 40, False),     # rows that are candidates whole, at odd offsets
+    (1, 2, 4097, 1500, True),
+    (2, 3, 60001, 300, True),    # sampled, every row at another alignment
+    (1, 520, 9001, 9, False),    # more rows than two per CU: 256 threads a row
+    (1, 2, 300000, 256, False),
+])
+def test_select_rows_of_any_length(device, dtype, B, Wp, V, width, masked):
+    """The row stage over its ways in: rows below and above the candidate
+    buffer, misaligned rows, both workgroup sizes, masks.  Scores 1e-5 from the
+    64-bit log-softmax (fp32 sums of up to 300,000 terms)."""
+    g = torch.Generator().manual_seed(V + width)
+    logits = (torch.randn(B, Wp, V, generator=g) * 2).to(dtype)
+    scores = -torch.rand(B, Wp, generator=g) * 3
+    mask = torch.rand(B, Wp, V, generator=g) > 0.5 if masked else None
+    s, p, t, valid = select_level(logits.to(device), scores.to(device), width,
+                                  None if mask is None else mask.to(device))
+    keys = logits.double().log_softmax(-1) + scores.double()[..., None]
+    if masked:
+        keys = keys.masked_fill(~mask, -float("inf"))
+    assert bool(valid.all())
+    assert_selection_gap_aware(s, p, t, keys, width, 1e-5, name="rows")
+
+
+def test_select_float_rows_with_equal_keys_take_lower_columns(device):
+    """fp32 logits that differ by less than their keys' precision tie, and the
+    lower columns of all of them are taken, sampled or not."""
+    V, W = 50000, 20
+    logits = torch.full((1, 1, V), -3.0)         # one value: every key equal
+    s, p, t, _ = select_level(logits.to(device), torch.zeros(1, 1, device=device), W)
+    assert t[0].tolist() == list(range(W))
+    logits[0, 0, 40000:40010] = 1e-6             # logits apart, keys (near -7.8) equal
+    logits[0, 0, 40000:40010] += torch.arange(10) * 1e-9
+    s, p, t, _ = select_level(logits.to(device), torch.zeros(1, 1, device=device), 4)
+    assert t[0].tolist() == [40000, 40001, 40002, 40003]
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_select_float_logits_matches_oracle(device, dtype):
     g = torch.Generator().manual_seed(11)
