@@ -70,9 +70,9 @@ int kad_gdn_suffix_replay(const void* q, const void* k, const void* v, int64_t l
  * aligned); conv_state / history / conv_weight ([C, 4] bf16, 8-byte aligned)
  * as in kad_causal_conv_suffix; the rest as in kad_gdn_suffix_replay.  The
  * outputs are the two calls' bits.  Supported: K = V = 128, T in {1, 2},
- * W % 16 == 0, fp32 log decays and bf16 betas (even ld_gate); anything else
- * is KAD_ERR_UNSUPPORTED (the caller then makes the two calls).  No
- * counterpart in the reference as one call: it fuses the decode's
+ * W % 16 == 0 (the gated forms below: any W), fp32 log decays and bf16
+ * betas (even ld_gate); anything else is KAD_ERR_UNSUPPORTED (the caller then
+ * makes the two calls).  No counterpart in the reference as one call: it fuses the decode's
  * causal_conv1d and gated_delta calls (src/kadllm/adapters/qwen3_5.py:146-174),
  * so the suffix rows make one pass through memory instead of three. */
 int kad_gdn_suffix_replay_conv(const void* proj, int64_t ld_proj, const void* conv_state,

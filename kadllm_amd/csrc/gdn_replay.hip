@@ -417,7 +417,7 @@ struct ParentRows {
 
 // LAST (with GATED, last token only): the earlier tokens' q, whose outputs
 // nothing reads, enter no product (their k and v still update the state)
-template <int T, int NS, bool CONV, bool GATED = false, bool LAST = false, bool PAR = false>
+template <int T, int NS, bool CONV, bool GATED = false, bool LAST = false, bool PAR = false, bool PART = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T == 1 ? 3 : (T == 4 ? 1 : 2), 8)))
 void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                            const bf16_t* __restrict__ v, int64_t ld_qk, int64_t ld_v,
@@ -462,12 +462,17 @@ void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restric
 
   const int n_begin = bb * beams_per_block;
   const int n_end = min(W, n_begin + beams_per_block);
-  const int ngroups = (n_end - n_begin) / 16;
+  // PART: the last group may hold fewer than 16 beams; its other lanes repeat
+  // the last one and store nothing (a form of its own: the clamps cost whole
+  // groups 3%)
+  const int ngroups = (n_end - n_begin + 15) / 16;
+  const int last_beam = n_end - n_begin - 1;
+  auto beam_of = [&](int beam) { return PART ? min(beam, last_beam) : beam; };
 
   // DMA of group gi into stage s: wave w moves 1 KB pieces w*T .. w*T+T-1 of
   // each block; lane L of piece I fills row 4I + L/16, swizzled chunk L%16
   auto dma_group = [&](int gi, int s) {
-    const int64_t row0 = ((int64_t)b * W + n_begin + gi * 16) * T;
+    const int64_t row0 = ((int64_t)b * W + n_begin) * T;
     uint8_t* sb = stage_buf + s * STAGE;
     const int w = __builtin_amdgcn_readfirstlane(wave);
 #pragma unroll
@@ -479,7 +484,7 @@ void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restric
       if constexpr (PAR) {
         // (beam, token) of row r: an earlier token from the parent's cached
         // row, the new token from the compact buffer
-        const int beam = gi * 16 + r / T, t = r % T;
+        const int beam = beam_of(gi * 16 + r / T), t = r % T;
         const bf16_t* base =
             t < T - 1 ? pr.prev + ((int64_t)(b * pr.Wp + par_lds[beam]) * (T - 1) + t) * pr.ld_prev
                       : pr.cur + ((int64_t)b * W + n_begin + beam) * pr.ld_cur;
@@ -487,8 +492,10 @@ void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restric
         ks = base + (int64_t)(H + h) * KD + c * 8;
         vs = base + (int64_t)2 * H * KD + (int64_t)hv * VD + c * 8;
       } else {
-        const int64_t qrow = (row0 + r) * ld_qk + (int64_t)h * KD + c * 8;
-        const int64_t vrow = (row0 + r) * ld_v + (int64_t)hv * VD + c * 8;
+        const int64_t row =
+            row0 + (PART ? beam_of(gi * 16 + r / T) * T + r % T : gi * 16 * T + r);
+        const int64_t qrow = row * ld_qk + (int64_t)h * KD + c * 8;
+        const int64_t vrow = row * ld_v + (int64_t)hv * VD + c * 8;
         qs = q + qrow;
         ks = k + qrow;
         vs = v + vrow;
@@ -504,7 +511,9 @@ void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restric
     // decays, wave 1 the 4-byte words holding the bf16 betas (rows have an
     // even stride, so a beta's half of its word is hv % 2)
     if (w < 2 && lane < ROWS) {
-      const int64_t gix = (row0 + lane) * ld_gate + hv;
+      const int64_t gix =
+          (row0 + (PART ? beam_of(gi * 16 + lane / T) * T + lane % T : gi * 16 * T + lane)) *
+              ld_gate + hv;
       const void* src = w == 0 ? (const void*)((const float*)gdecay + gix)
                                : (const void*)((const uint32_t*)beta + (gix >> 1));
       __builtin_amdgcn_global_load_lds((replay_global_t*)src,
@@ -627,7 +636,7 @@ void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restric
     // waiting for them does not wait for it
     u32x2 zg[GATED ? T : 1][GATED ? MT : 1];
     if constexpr (GATED) {
-      const int64_t nz = (int64_t)b * W + n_begin + gi * 16 + col;
+      const int64_t nz = (int64_t)b * W + n_begin + beam_of(gi * 16 + col);
 #pragma unroll
       for (int t = 0; t < T; ++t)
         if (t >= go.t_first) {
@@ -690,6 +699,7 @@ void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restric
     const uint8_t* sv = sq + 2 * BLK;
     const int g0 = n_begin + gi * 16;
     const int64_t n = (int64_t)b * W + g0 + col;
+    const bool stored = !PART || gi * 16 + col <= last_beam;
 
     f32x4 acc_q[T][MT], acc_k[T][MT];
 #pragma unroll
@@ -818,7 +828,8 @@ void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restric
           y[i] = wn * silu_fast(zv);
         }
         const u32x2 yv = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
-        *(u32x2*)(out + orow * ld_out + (int64_t)hv * VD + v0 + mt * 16 + quad * 4) = yv;
+        if (stored)
+          *(u32x2*)(out + orow * ld_out + (int64_t)hv * VD + v0 + mt * 16 + quad * 4) = yv;
       }
     };
     float u[T][MT][4];
@@ -858,7 +869,7 @@ void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restric
         if constexpr (GATED) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) og[mt][i] = ov[i];
-        } else {
+        } else if (stored) {
           store4<bf16_t>(out + (n * T + t) * ld_out + (int64_t)hv * VD + e, ov);
         }
       }
@@ -871,43 +882,55 @@ void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restric
   for (int gi = 0; gi < ngroups; ++gi) group(gi);
 }
 
+// Beams per workgroup, whole groups of 16, at most `most`: a request's beams in
+// one workgroup pay the state prologue once per (request, head) -- two-token
+// suffixes of 32 requests x 256 beams ran 7% faster so than in two of 128 --
+// unless that leaves the CUs with fewer than two workgroups each (16 heads: 8
+// requests x 50 beams, two tokens 17.6 -> 9.9 us; 1 x 256, one token 21 -> 7.4).
+int beams_per_block(int64_t heads, int W, int most) {
+  int bpb = W < most ? (W + 15) / 16 * 16 : (W > most ? 128 : most);
+  while (bpb > 16 && heads * kad_cdiv(W, bpb) < 512) bpb = (bpb / 2 + 15) / 16 * 16;
+  return bpb;
+}
+
 template <int KD, int VD, typename TIN>
 int launch_replay(const void* q, const void* k, const void* v, int64_t ld_qk, int64_t ld_v,
                   const void* g, int gdt, const void* beta, int bdt, int64_t ld_gate,
                   const void* state, int sdt, void* out, int64_t ld_out, int B, int W,
                   int T, int H, int HV, float scale, hipStream_t stream) {
-  int bpb = W >= 256 ? 128 : ((W + 15) / 16) * 16;
-  if (bpb > 128) bpb = 128;
-  // the staged kernel takes a request's beams in one workgroup up to 256, so
-  // the state prologue is paid once per (request, head): two-token suffixes
-  // at 256 beams 7% faster than two workgroups of 128
-  if (KD == 128 && VD == 128 && sizeof(TIN) == 2 && T <= 4 && W % 16 == 0 && W <= 256) bpb = W;
+  const bool lds_form = KD == 128 && VD == 128 && sizeof(TIN) == 2 && T <= 4;
+  const int bpb = beams_per_block((int64_t)B * HV, W, lds_form ? 256 : 128);
   const int nbb = (int)kad_cdiv(W, bpb);
   const int64_t nblocks = (int64_t)B * HV * nbb;
   if (nblocks > 0x7fffffff) {
     kad_set_error("gdn replay grid too large");
     return KAD_ERR_UNSUPPORTED;
   }
-  // the LDS-staged kernel for the decode shapes (all groups full, 16-byte rows)
+  // the LDS-staged kernel for the decode shapes (16-byte rows)
   if constexpr (KD == 128 && VD == 128 && sizeof(TIN) == 2) {
-    const bool staged = T <= 4 && W % 16 == 0 && bpb % 16 == 0 && gdt == KAD_DTYPE_F32 &&
+    const bool staged = T <= 4 && gdt == KAD_DTYPE_F32 &&
                         bdt == KAD_DTYPE_BF16 && ld_gate % 2 == 0 &&
                         ((uintptr_t)beta % 4) == 0 && ((uintptr_t)g % 4) == 0 && ld_qk % 8 == 0 &&
                         ld_v % 8 == 0 && ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % 16 == 0;
     if (staged) {
-#define KAD_REPLAY_LDS(TT, NS)                                                                \
-  if (T == TT) {                                                                              \
-    hipLaunchKernelGGL((gdn_replay_lds_kernel<TT, NS, false>), dim3((unsigned)nblocks),       \
+#define KAD_REPLAY_LDS(TT, NS, PARTV)                                                         \
+  if (T == TT && (W % 16 != 0) == PARTV) {                                                    \
+    hipLaunchKernelGGL((gdn_replay_lds_kernel<TT, NS, false, false, false, false, PARTV>),    \
+                       dim3((unsigned)nblocks),                                               \
                        dim3(256), 0, stream, (const bf16_t*)q, (const bf16_t*)k,              \
                        (const bf16_t*)v, ld_qk, ld_v, g, gdt, beta, bdt, ld_gate, state, sdt, \
                        (bf16_t*)out, ld_out, W, H, HV, scale, bpb, nbb, ConvArgs{},           \
                        GateOutArgs{}, ParentRows{});                                          \
     return kad_launch_status("gdn_replay_lds_kernel");                                        \
   }
-      KAD_REPLAY_LDS(1, 3)
-      KAD_REPLAY_LDS(2, 3)
-      KAD_REPLAY_LDS(3, 2)
-      KAD_REPLAY_LDS(4, 2)
+      KAD_REPLAY_LDS(1, 3, false)
+      KAD_REPLAY_LDS(2, 3, false)
+      KAD_REPLAY_LDS(3, 2, false)
+      KAD_REPLAY_LDS(4, 2, false)
+      KAD_REPLAY_LDS(1, 3, true)
+      KAD_REPLAY_LDS(2, 3, true)
+      KAD_REPLAY_LDS(3, 2, true)
+      KAD_REPLAY_LDS(4, 2, true)
 #undef KAD_REPLAY_LDS
     }
   }
@@ -955,7 +978,7 @@ int launch_replay_conv(const bf16_t* proj, int64_t ld, const ConvArgs& cv, const
                        const void* beta, int64_t ld_gate, const void* state, int sdt, void* out,
                        int64_t ld_out, int B, int W, int T, int H, int HV, float scale,
                        const GateOutArgs* go, const ParentRows* par, hipStream_t stream) {
-  const int bpb = W <= 256 ? W : 128;
+  const int bpb = beams_per_block((int64_t)B * HV, W, 256);
   const int nbb = (int)kad_cdiv(W, bpb);
   const int64_t nblocks = (int64_t)B * HV * nbb;
   KAD_REQUIRE(nblocks <= 0x7fffffff, "gdn replay grid too large");
@@ -964,21 +987,25 @@ int launch_replay_conv(const bf16_t* proj, int64_t ld, const ConvArgs& cv, const
   const bf16_t* v = proj + (int64_t)2 * H * 128;
   const bool last = go != nullptr && go->t_first == T - 1 && T > 1;
   const bool pv = par != nullptr;
-#define KAD_REPLAY_CONV(TT, GV, LV, PV)                                                        \
-  if (T == TT && (go != nullptr) == GV && last == LV && pv == PV) {                            \
-    hipLaunchKernelGGL((gdn_replay_lds_kernel<TT, 3, true, GV, LV, PV>),                       \
+#define KAD_REPLAY_CONV(TT, GV, LV, PV, PARTV)                                                 \
+  if (T == TT && (go != nullptr) == GV && last == LV && pv == PV && (W % 16 != 0) == PARTV) {  \
+    hipLaunchKernelGGL((gdn_replay_lds_kernel<TT, 3, true, GV, LV, PV, PARTV>),                \
                        dim3((unsigned)nblocks), dim3(256), 0, stream, q, k, v, ld, ld, g,      \
                        KAD_DTYPE_F32, beta, KAD_DTYPE_BF16, ld_gate, state, sdt, (bf16_t*)out, \
                        ld_out, W, H, HV, scale, bpb, nbb, cv, go ? *go : GateOutArgs{},        \
                        par ? *par : ParentRows{});                                             \
     return kad_launch_status("gdn_replay_lds_kernel");                                         \
   }
-  KAD_REPLAY_CONV(1, false, false, false)
-  KAD_REPLAY_CONV(2, false, false, false)
-  KAD_REPLAY_CONV(1, true, false, false)
-  KAD_REPLAY_CONV(2, true, false, false)
-  KAD_REPLAY_CONV(2, true, true, false)
-  KAD_REPLAY_CONV(2, true, true, true)
+  KAD_REPLAY_CONV(1, false, false, false, false)
+  KAD_REPLAY_CONV(2, false, false, false, false)
+  KAD_REPLAY_CONV(1, true, false, false, false)
+  KAD_REPLAY_CONV(2, true, false, false, false)
+  KAD_REPLAY_CONV(2, true, true, false, false)
+  KAD_REPLAY_CONV(2, true, true, true, false)
+  KAD_REPLAY_CONV(1, true, false, false, true)
+  KAD_REPLAY_CONV(2, true, false, false, true)
+  KAD_REPLAY_CONV(2, true, true, false, true)
+  KAD_REPLAY_CONV(2, true, true, true, true)
 #undef KAD_REPLAY_CONV
   KAD_UNSUPPORTED("the fused conv replay takes 1 or 2 suffix tokens, got %d", T);
 }
@@ -1006,9 +1033,10 @@ int replay_conv_common(
   for (int dt : {gate_dtype, beta_dtype, state_dtype})
     KAD_REQUIRE(dt == KAD_DTYPE_BF16 || dt == KAD_DTYPE_F16 || dt == KAD_DTYPE_F32,
                 "unknown dtype code %d", dt);
-  if (!(K == 128 && V == 128 && (T == 1 || T == 2) && W % 16 == 0))
-    KAD_UNSUPPORTED("the fused conv replay takes K = V = 128, 1 or 2 suffix tokens and beam "
-                    "counts that are multiples of 16 (got K=%d V=%d T=%d W=%d)", K, V, T, W);
+  if (!(K == 128 && V == 128 && (T == 1 || T == 2) && (go || W % 16 == 0)))
+    KAD_UNSUPPORTED("the fused conv replay takes K = V = 128, 1 or 2 suffix tokens and, without "
+                    "the gated output, beam counts that are multiples of 16 (got K=%d V=%d T=%d "
+                    "W=%d)", K, V, T, W);
   if (!(gate_dtype == KAD_DTYPE_F32 && beta_dtype == KAD_DTYPE_BF16 && ld_gate % 2 == 0 &&
         ((uintptr_t)beta % 4) == 0 && ((uintptr_t)log_decay % 4) == 0))
     KAD_UNSUPPORTED("the fused conv replay takes fp32 log decays and bf16 betas with an even "

@@ -270,11 +270,11 @@ class Qwen35Runner:
             _lib.call("kad_gdn_recurrent", *args, W, _lib.ptr(o), self.vd, None, B * W, T, H_, HV,
                       dk, dv, float(dk ** -0.5), _lib.stream_of(conv))
 
-    def _mixer_fusable(self, lyr, W):
+    def _mixer_fusable(self, lyr):
         """Whether the fused decode mixer takes this layer's shapes (besides
         the suffix length and row alignment, checked where it is called)."""
         cfg = self.cfg
-        return (W % 16 == 0 and cfg.linear_key_head_dim == 128
+        return (cfg.linear_key_head_dim == 128
                 and cfg.linear_value_head_dim == 128 and self.gdn_cols % 8 == 0
                 and lyr.conv_w.is_contiguous() and lyr.conv_w.data_ptr() % 8 == 0
                 and lyr.norm_w.data_ptr() % 8 == 0
@@ -333,7 +333,7 @@ class Qwen35Runner:
         cs, S = cached
         g, beta = self._gdn_gates(lyr, proj)
         z = proj[:, C:C + self.vd]
-        if (T <= 2 and W % 16 == 0 and dk == 128 and dv == 128 and g.stride(0) % 2 == 0
+        if (T <= 2 and dk == 128 and dv == 128 and g.stride(0) % 2 == 0
                 and ld % 8 == 0 and proj.data_ptr() % 16 == 0 and lyr.conv_w.is_contiguous()
                 and lyr.conv_w.data_ptr() % 8 == 0 and lyr.norm_w.data_ptr() % 8 == 0):
             y = torch.empty(BW if last_only else BW * T, self.vd, dtype=torch.bfloat16,
@@ -604,7 +604,7 @@ class Qwen35Runner:
             n = layers.rmsnorm(x, lyr.input_norm, cfg.rms_norm_eps)
             if isinstance(lyr, _GdnLayer):
                 cols = self.gdn_cols
-                if T == 2 and not keep_cache and self._mixer_fusable(lyr, W):
+                if T == 2 and not keep_cache and self._mixer_fusable(lyr):
                     # the last level reads the earlier token's rows from the
                     # parents' cache in place: no row gather
                     y = self._gdn_mix_parents(lyr, n, cache.layers[li], parents, cached, B, W,

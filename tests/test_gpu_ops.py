@@ -396,3 +396,73 @@ def test_gdn_replay_conv_gated_parents_equals_gather(device, W, Wp, H, HV):
               _lib.ptr(y2), HV * K, B, W, T, H, HV, K, K, K ** -0.5, stream)
     torch.cuda.synchronize()
     assert torch.equal(y2, y1), "parent-row fused replay differs from gather + fused replay"
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 4])
+@pytest.mark.parametrize("B,W", [(1, 1), (2, 10), (3, 17), (8, 50), (1, 300), (40, 130)])
+def test_gdn_replay_partial_groups_equal_register_kernel(device, T, B, W):
+    """Beam counts that end inside a group of 16, over one and several
+    workgroups a request: the staged kernel's bits are the register one's (which
+    an fp32 beta selects), and it writes no row past the last beam's."""
+    H, HV, K = 2, 4, 128
+    q, k, v, g, beta, S = _to(device, *gdn_inputs(B, W, T, H, HV, K, K, seed=T * 100 + W))
+    out = torch.full((B * W * T + 16 * T, HV, K), 7.0, dtype=torch.bfloat16, device=device)
+    _lib.call("kad_gdn_suffix_replay", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), H * K, HV * K, 0,
+              _lib.ptr(g), 2, _lib.ptr(beta), 0, HV, _lib.ptr(S), 2, _lib.ptr(out), HV * K, B, W,
+              T, H, HV, K, K, K ** -0.5, _lib.stream_of(q))
+    plain = ops.gated_delta(q, k, v, g, beta.float(), S, beam_width=W)
+    assert torch.equal(out[:B * W * T].view(plain.shape), plain)
+    assert bool((out[B * W * T:] == 7.0).all())
+
+
+@pytest.mark.parametrize("T", [1, 2])
+@pytest.mark.parametrize("B,W,Wp,H,HV", [(1, 1, 1, 2, 2), (2, 10, 7, 2, 4), (3, 50, 50, 1, 2),
+                                         (1, 130, 33, 2, 2)])
+def test_gdn_replay_conv_gated_partial_groups(device, T, B, W, Wp, H, HV):
+    """The fused mixer (and its parent-row form) at beam counts that end inside
+    a group of 16 against conv, replay and gated norm as three calls."""
+    K, hist, eps = 128, 4, 1e-6
+    C = 2 * H * K + HV * K
+    ld = C + HV * K + 40                 # q | k | v | z | more columns
+    g = torch.Generator().manual_seed(W * 10 + T)
+    prev = (torch.randn(B * Wp, ld, generator=g) * 0.7).bfloat16().to(device)
+    cur = (torch.randn(B * W, ld, generator=g) * 0.7).bfloat16().to(device)
+    parents = torch.randint(0, Wp, (B, W), generator=g).to(device)
+    cs = (torch.randn(B, C, hist, generator=g) * 0.7).bfloat16().to(device)
+    cw = (torch.rand(C, 4, generator=g) - 0.5).bfloat16().to(device)
+    logd = (-torch.rand(B * W * T, HV, generator=g) * 0.3).to(device)
+    beta = torch.rand(B * W * T, HV, generator=g).bfloat16().to(device)
+    S = (torch.randn(B, HV, K, K, generator=g) * 0.05).to(device)
+    nw = (1.0 + 0.1 * torch.randn(K, generator=g)).bfloat16().to(device)
+    stream = _lib.stream_of(cur)
+    full = torch.empty(B * W, T, ld, dtype=torch.bfloat16, device=device)
+    if T == 2:
+        full[:, 0] = prev.view(B, Wp, ld).gather(
+            1, parents[..., None].expand(B, W, ld)).view(B * W, ld)
+    full[:, T - 1] = cur
+    conv = torch.empty(B * W * T, C, dtype=torch.bfloat16, device=device)
+    _lib.call("kad_causal_conv_suffix", _lib.ptr(full), T * ld, 1, ld, _lib.ptr(cs), *cs.stride(),
+              hist, _lib.ptr(cw), 4, None, _lib.ptr(conv), T * C, 1, C, B, W, C, T, 0, 1, stream)
+    q, k, v = (t.reshape(B * W, T, -1, K) for t in conv.split([H * K, H * K, HV * K], 1))
+    o = ops.gated_delta(q, k, v, logd.view(B * W, T, HV), beta.view(B * W, T, HV).float(), S,
+                        beam_width=W).view(B * W * T, HV * K)
+    rows = full.view(B * W * T, ld)
+    every = layers.rmsnorm_gated(o, rows[:, C:C + HV * K], nw, eps, HV)
+    for last in (0, 1):
+        want = every.view(B * W, T, -1)[:, -1] if last else every
+        got = torch.full((want.shape[0] + 16 * T, HV * K), 5.0, dtype=torch.bfloat16,
+                         device=device)
+        _lib.call("kad_gdn_suffix_replay_conv_gated", _lib.ptr(rows), ld, _lib.ptr(cs),
+                  *cs.stride(), hist, _lib.ptr(cw), _lib.ptr(logd), 2, _lib.ptr(beta), 0, HV,
+                  _lib.ptr(S), 2, _lib.ptr(rows[:, C:]), ld, _lib.ptr(nw), eps, last,
+                  _lib.ptr(got), HV * K, B, W, T, H, HV, K, K, K ** -0.5, stream)
+        assert torch.equal(got[:want.shape[0]], want), f"last={last}"
+        assert bool((got[want.shape[0]:] == 5.0).all())
+    if T == 2:
+        got = torch.full((B * W + 16, HV * K), 5.0, dtype=torch.bfloat16, device=device)
+        _lib.call("kad_gdn_suffix_replay_conv_gated_parents", _lib.ptr(prev), ld,
+                  _lib.ptr(parents), Wp, _lib.ptr(cur), ld, _lib.ptr(cs), *cs.stride(), hist,
+                  _lib.ptr(cw), _lib.ptr(logd), 2, _lib.ptr(beta), 0, HV, _lib.ptr(S), 2,
+                  _lib.ptr(cur[:, C:]), ld, _lib.ptr(nw), eps, _lib.ptr(got), HV * K, B, W, T, H,
+                  HV, K, K, K ** -0.5, stream)
+        assert torch.equal(got[:B * W], want) and bool((got[B * W:] == 5.0).all())
