@@ -10,11 +10,10 @@
 // (silu_fast: they are VALU-bound and the result is rounded to bf16); fp16 and
 // fp32 tensors keep the IEEE exp and divide.
 //
-// Three paths: a vectorised one when channels are contiguous in x and out
-// (8 channels per thread, 16-byte accesses; the [rows, T, C] layout produced by
-// the projection GEMM), a vectorised one for the reference's contiguous
-// [BW, C, T] layout (8 channels x T tokens per thread), and a scalar one for
-// any other strides, widths and dtypes.
+// Three paths: a vectorised one when channels are contiguous in x and out (the
+// [rows, T, C] layout produced by the projection GEMM), a vectorised one for the
+// reference's contiguous [BW, C, T] layout, both in 16-byte words of any of the
+// three types, and a scalar one for any other strides and widths.
 
 #include "kad_common.h"
 
@@ -81,178 +80,229 @@ __global__ __launch_bounds__(256) void conv_suffix_scalar(
   }
 }
 
-// 8 contiguous bf16 channels per thread, kConvBeams beams of one request per
-// thread (the request's weights and prefix taps are loaded once); width 4
-// (3 taps), any T.  Grid: x = request x beam group, y = channel groups of 256
-// threads.  The next (beam, token) row is loaded before the current one is
-// computed so that every thread keeps one 16-byte load in flight.
-constexpr int kConvBeams = 8;
+// A 16-byte word of channels and the layout-independent parts of the vector
+// kernels: VE channels per thread, whose weights ([C, 4]) are 64 bytes and
+// whose prefix taps are 64 bytes in the model's state layout ([B, C, 4]).
+template <typename T>
+struct ConvVec {
+  static constexpr int VE = 16 / sizeof(T);
+  __device__ static __forceinline__ void unpack(const u32x4& r, float (&f)[VE]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (Elem<T>::code == KAD_DTYPE_BF16) {
+        f[2 * e] = __uint_as_float(r[e] << 16);
+        f[2 * e + 1] = __uint_as_float(r[e] & 0xffff0000u);
+      } else if constexpr (Elem<T>::code == KAD_DTYPE_F16) {
+        f[2 * e] = (float)__builtin_bit_cast(_Float16, (uint16_t)(r[e] & 0xffffu));
+        f[2 * e + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(r[e] >> 16));
+      } else {
+        f[e] = __uint_as_float(r[e]);
+      }
+    }
+  }
+  // conv results to outputs: rounded, SiLU, rounded (bf16 pairs as one packed
+  // conversion each, the same bits)
+  __device__ static __forceinline__ u32x4 finish(const float (&acc)[VE], bool silu) {
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (Elem<T>::code == KAD_DTYPE_BF16) {
+        uint32_t p = pack_bf16x2(acc[2 * e], acc[2 * e + 1]);
+        if (silu)
+          p = pack_bf16x2(silu_fast(__uint_as_float(p << 16)),
+                          silu_fast(__uint_as_float(p & 0xffff0000u)));
+        o[e] = p;
+      } else if constexpr (Elem<T>::code == KAD_DTYPE_F16) {
+        uint32_t p = 0;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float y = (float)(_Float16)acc[2 * e + h];
+          if (silu) y = silu_for<T>(y);
+          p |= (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)y) << (16 * h);
+        }
+        o[e] = p;
+      } else {
+        o[e] = __float_as_uint(silu ? silu_for<T>(acc[e]) : acc[e]);
+      }
+    }
+    return o;
+  }
+  // VE channels x 4 from 64 contiguous bytes
+  __device__ static __forceinline__ void load4(const T* p, float (&f)[VE][4]) {
+    float g[VE];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      unpack(((const u32x4*)p)[j], g);
+#pragma unroll
+      for (int e = 0; e < VE; ++e) f[(j * VE + e) / 4][(j * VE + e) % 4] = g[e];
+    }
+  }
+  // the last 3 taps of channels c0 .. c0 + VE - 1
+  __device__ static __forceinline__ void taps(const T* sb, int c0, int64_t ss_c, int64_t ss_t,
+                                              int history, float (&tap)[VE][3]) {
+    if (ss_t == 1 && ss_c == 4 && history == 4 && ((uintptr_t)sb % 16) == 0) {
+      float f[VE][4];
+      load4(sb + (int64_t)c0 * 4, f);
+#pragma unroll
+      for (int ch = 0; ch < VE; ++ch)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) tap[ch][i] = f[ch][i + 1];
+    } else {
+#pragma unroll
+      for (int ch = 0; ch < VE; ++ch)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          tap[ch][i] = Elem<T>::to_f(sb[(c0 + ch) * ss_c + (history - 3 + i) * ss_t]);
+    }
+  }
+};
+
+// Channels contiguous (a projection's rows): VE channels per thread, up to
+// kConvBeams beams of one request per thread (the request's weights and prefix
+// taps are loaded once); width 4 (3 taps), any T.  Grid: x = request x beam
+// group, y = channel groups of 256 threads, z = runs of kConvRun tokens of
+// suffixes longer than 4 (an fp32 model's whole prompts, which one thread per channel would
+// walk).  The next (beam,
+// token) row is loaded before the current one is computed so that every thread
+// keeps one 16-byte load in flight.
+constexpr int kConvBeams = 8, kConvRun = 16;
 
 // TT > 0: the suffix length fixed at compile time (the search's one- to
 // four-token suffixes), so the (beam, token) of each step needs no division
-template <int TT>
-__global__ __launch_bounds__(256) void conv_suffix_vec_bf16(
-    const bf16_t* __restrict__ x, int64_t sx_n, int64_t sx_t, const bf16_t* __restrict__ state,
-    int64_t ss_b, int64_t ss_c, int64_t ss_t, int history, const bf16_t* __restrict__ w,
-    bf16_t* __restrict__ out, int64_t so_n, int64_t so_t, int W, int C, int T_rt, int nbg,
+template <typename T, int TT>
+__global__ __launch_bounds__(256) void conv_suffix_vec(
+    const T* __restrict__ x, int64_t sx_n, int64_t sx_t, const T* __restrict__ state,
+    int64_t ss_b, int64_t ss_c, int64_t ss_t, int history, const T* __restrict__ w,
+    T* __restrict__ out, int64_t so_n, int64_t so_t, int W, int C, int T_rt, int nbg, int beams,
     int silu) {
-  const int T_ = TT > 0 ? TT : T_rt;
-  const int c8 = blockIdx.y * 256 + threadIdx.x;
-  if (c8 >= C / 8) return;
-  const int c0 = c8 * 8;
+  constexpr int VE = ConvVec<T>::VE;
+  const int t0 = TT > 0 ? 0 : blockIdx.z * kConvRun;
+  const int T_ = TT > 0 ? TT : min(kConvRun, T_rt - t0);
+  const int cv = blockIdx.y * 256 + threadIdx.x;
+  if (cv >= C / VE) return;
+  const int c0 = cv * VE;
   const int b = blockIdx.x / nbg;
-  const int j0 = (blockIdx.x % nbg) * kConvBeams;
-  const int nj = min(W - j0, kConvBeams);
-  float wt[8][4];
-  {
-    const u32x4* wp = (const u32x4*)(w + (int64_t)c0 * 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      u32x4 r = wp[j];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int flat = j * 8 + e * 2;  // channel c0 + flat/4, tap flat%4
-        wt[flat / 4][flat % 4] = __uint_as_float(r[e] << 16);
-        wt[(flat + 1) / 4][(flat + 1) % 4] = __uint_as_float(r[e] & 0xffff0000u);
-      }
-    }
-  }
-  // prefix taps: the last 3 of the request's state, per channel
-  float tap[8][3];
-  const bf16_t* sb = state + (int64_t)b * ss_b;
-  if (ss_t == 1 && ss_c == 4 && history == 4 && (((uintptr_t)sb) % 16) == 0) {
-    const u32x4* sp = (const u32x4*)(sb + (int64_t)c0 * 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      u32x4 r = sp[j];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int flat = j * 8 + e * 2;  // channel flat/4, slot flat%4 (slots 1..3 are taps)
-        if (flat % 4 != 0) tap[flat / 4][flat % 4 - 1] = __uint_as_float(r[e] << 16);
-        tap[(flat + 1) / 4][(flat + 1) % 4 - 1] = __uint_as_float(r[e] & 0xffff0000u);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int ch = 0; ch < 8; ++ch)
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-        tap[ch][i] = bf2f(sb[(int64_t)(c0 + ch) * ss_c + (int64_t)(history - 3 + i) * ss_t]);
-  }
-
+  const int j0 = (blockIdx.x % nbg) * beams;
+  const int nj = min(W - j0, beams);
   const int64_t n0 = (int64_t)b * W + j0;
   const int steps = nj * T_;
   auto row = [&](int k) {
     const int j = k / T_, t = k - (k / T_) * T_;
-    return x + (n0 + j) * sx_n + (int64_t)t * sx_t + c0;
+    return x + (n0 + j) * sx_n + (int64_t)(t0 + t) * sx_t + c0;
   };
   u32x4 next = *(const u32x4*)row(0);
-  float win[8][4];
+  float wt[VE][4], tap[VE][3];
+  ConvVec<T>::load4(w + (int64_t)c0 * 4, wt);
+  if (TT > 0 || t0 == 0) ConvVec<T>::taps(state + b * ss_b, c0, ss_c, ss_t, history, tap);
+
+  float win[VE][4];
   for (int k = 0, t = 0; k < steps; ++k) {
     const u32x4 r = next;
     if (k + 1 < steps) next = *(const u32x4*)row(k + 1);
     if (t == 0) {
+      if (TT > 0 || t0 == 0) {
 #pragma unroll
-      for (int ch = 0; ch < 8; ++ch) {
-        win[ch][1] = tap[ch][0];
-        win[ch][2] = tap[ch][1];
-        win[ch][3] = tap[ch][2];
+        for (int ch = 0; ch < VE; ++ch)
+#pragma unroll
+          for (int i = 0; i < 3; ++i) win[ch][i + 1] = tap[ch][i];
+      } else {  // the three tokens before the run
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          float f[VE];
+          ConvVec<T>::unpack(*(const u32x4*)(row(k) + (int64_t)(i - 3) * sx_t), f);
+#pragma unroll
+          for (int ch = 0; ch < VE; ++ch) win[ch][i + 1] = f[ch];
+        }
       }
     }
-    u32x4 o;
+    float xv[VE], acc[VE];
+    ConvVec<T>::unpack(r, xv);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float xv[2] = {__uint_as_float(r[e] << 16), __uint_as_float(r[e] & 0xffff0000u)};
-      float acc[2];
+    for (int ch = 0; ch < VE; ++ch) {
+      win[ch][0] = win[ch][1];
+      win[ch][1] = win[ch][2];
+      win[ch][2] = win[ch][3];
+      win[ch][3] = xv[ch];
+      float s = 0.f;
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int ch = e * 2 + hh;
-        win[ch][0] = win[ch][1];
-        win[ch][1] = win[ch][2];
-        win[ch][2] = win[ch][3];
-        win[ch][3] = xv[hh];
-        float s = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s += wt[ch][i] * win[ch][i];
-        acc[hh] = s;
-      }
-      // the pair's roundings as one packed conversion each (the same bits)
-      uint32_t packed = pack_bf16x2(acc[0], acc[1]);
-      if (silu)
-        packed = pack_bf16x2(silu_fast(__uint_as_float(packed << 16)),
-                             silu_fast(__uint_as_float(packed & 0xffff0000u)));
-      o[e] = packed;
+      for (int i = 0; i < 4; ++i) s += wt[ch][i] * win[ch][i];
+      acc[ch] = s;
     }
     const int j = k / T_;
-    *(u32x4*)(out + (n0 + j) * so_n + (int64_t)t * so_t + c0) = o;
+    *(u32x4*)(out + (n0 + j) * so_n + (int64_t)(t0 + t) * so_t + c0) =
+        ConvVec<T>::finish(acc, silu);
     if (++t == T_) t = 0;
   }
 }
 
-
 // The reference's contiguous [BW, C, T] layout (each beam's block of C * T
-// elements is one contiguous run, tokens fastest): 8 channels x TT tokens per
-// thread are TT consecutive 16-byte words, so a beam streams through with
-// vector loads and stores exactly as the token-major kernel does.  Same grid
-// and arithmetic as conv_suffix_vec_bf16 (kConvBeams beams of one request per
-// thread, the next beam's words loaded before the current one is computed).
-template <int TT>
-__global__ __launch_bounds__(256) void conv_suffix_ct_bf16(
-    const bf16_t* __restrict__ x, int64_t sx_n, const bf16_t* __restrict__ state, int64_t ss_b,
-    int64_t ss_c, int64_t ss_t, int history, const bf16_t* __restrict__ w,
-    bf16_t* __restrict__ out, int64_t so_n, int W, int C, int nbg, int silu) {
-  const int c8 = blockIdx.y * 256 + threadIdx.x;
-  if (c8 >= C / 8) return;
-  const int c0 = c8 * 8;
+// elements is one contiguous run, tokens fastest): VE channels x TT tokens per
+// thread are TT consecutive 16-byte words.  A wave moves its 64 TT words as
+// they lie in memory and hands each lane its own TT through LDS (a lane loading
+// its own words touches every line TT times: 32 x 256 beams x 6,144 channels of
+// three bf16 tokens 159 us, 126 this way, 4.8 TB/s as the token-major kernel).  Lane l's words are l TT + k; bits 4 and up of a
+// word's index are folded into its low ones so that the 16 lanes of an access
+// hit 16 bank groups (TT = 2, 4; at 3 they do as they are).  Same grid and
+// arithmetic as conv_suffix_vec; the next beam's words load meanwhile.
+template <typename T, int TT>
+__global__ __launch_bounds__(256) void conv_suffix_ct(
+    const T* __restrict__ x, int64_t sx_n, const T* __restrict__ state, int64_t ss_b,
+    int64_t ss_c, int64_t ss_t, int history, const T* __restrict__ w, T* __restrict__ out,
+    int64_t so_n, int W, int C, int nbg, int beams, int silu) {
+  constexpr int VE = ConvVec<T>::VE;
+  __shared__ __attribute__((aligned(16))) u32x4 words[4][64 * TT];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int cw = blockIdx.y * 256 + wave * 64;  // the wave's first channel group
+  const int lanes = min(64, C / VE - cw);       // its channel groups
+  if (lanes <= 0) return;
+  u32x4* own = words[wave];
+  auto slot = [](int i) { return TT == 2 ? i ^ ((i >> 4) & 1) : (TT == 4 ? i ^ ((i >> 4) & 3) : i); };
+  const int c0 = (cw + min(lane, lanes - 1)) * VE;
   const int b = blockIdx.x / nbg;
-  const int j0 = (blockIdx.x % nbg) * kConvBeams;
-  const int nj = min(W - j0, kConvBeams);
-  float wt[8][4];
-  {
-    const u32x4* wp = (const u32x4*)(w + (int64_t)c0 * 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      u32x4 r = wp[j];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int flat = j * 8 + e * 2;
-        wt[flat / 4][flat % 4] = __uint_as_float(r[e] << 16);
-        wt[(flat + 1) / 4][(flat + 1) % 4] = __uint_as_float(r[e] & 0xffff0000u);
-      }
-    }
-  }
-  float tap[8][3];
-  const bf16_t* sb = state + (int64_t)b * ss_b;
-#pragma unroll
-  for (int ch = 0; ch < 8; ++ch)
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-      tap[ch][i] = bf2f(sb[(int64_t)(c0 + ch) * ss_c + (int64_t)(history - 3 + i) * ss_t]);
-
+  const int j0 = (blockIdx.x % nbg) * beams;
+  const int nj = min(W - j0, beams);
   const int64_t n0 = (int64_t)b * W + j0;
-  const int64_t off = (int64_t)c0 * TT;  // this thread's 8 * TT elements in a beam's block
+  const int64_t off = (int64_t)cw * VE * TT;    // the wave's words in a beam's block
+  const int nw = lanes * TT;
   u32x4 next[TT];
+  auto fetch = [&](int j) {
 #pragma unroll
-  for (int k = 0; k < TT; ++k) next[k] = ((const u32x4*)(x + n0 * sx_n + off))[k];
+    for (int k = 0; k < TT; ++k)
+      next[k] = ((const u32x4*)(x + (n0 + j) * sx_n + off))[min(k * 64 + lane, nw - 1)];
+  };
+  // The hardware keeps a wave's LDS accesses in order, so lanes exchange words
+  // without a barrier; the compiler, to which each lane's addresses look
+  // disjoint, must be told to.
+  auto wave_order = [] { asm volatile("" ::: "memory"); };
+  fetch(0);
+  float wt[VE][4], tap[VE][3];
+  ConvVec<T>::load4(w + (int64_t)c0 * 4, wt);
+  ConvVec<T>::taps(state + b * ss_b, c0, ss_c, ss_t, history, tap);
+
   for (int j = 0; j < nj; ++j) {
     u32x4 cur[TT];
+    if constexpr (TT > 1) {
 #pragma unroll
-    for (int k = 0; k < TT; ++k) cur[k] = next[k];
-    if (j + 1 < nj) {
+      for (int k = 0; k < TT; ++k) own[slot(k * 64 + lane)] = next[k];
+      wave_order();
+      if (j + 1 < nj) fetch(j + 1);
 #pragma unroll
-      for (int k = 0; k < TT; ++k) next[k] = ((const u32x4*)(x + (n0 + j + 1) * sx_n + off))[k];
+      for (int k = 0; k < TT; ++k) cur[k] = own[slot(lane * TT + k)];
+      wave_order();
+    } else {
+      cur[0] = next[0];
+      if (j + 1 < nj) fetch(j + 1);
     }
-    u32x4 o[TT];
+    float f[TT][VE], y[TT][VE];
 #pragma unroll
-    for (int k = 0; k < TT; ++k) o[k] = u32x4{0u, 0u, 0u, 0u};
+    for (int k = 0; k < TT; ++k) ConvVec<T>::unpack(cur[k], f[k]);
 #pragma unroll
-    for (int ch = 0; ch < 8; ++ch) {
+    for (int ch = 0; ch < VE; ++ch) {
       float w0 = tap[ch][0], w1 = tap[ch][1], w2 = tap[ch][2];
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
-        const int e = ch * TT + t;  // element index within the thread's run
-        const uint32_t word = cur[e / 8][(e % 8) / 2];
-        const float xv = __uint_as_float((e & 1) ? (word & 0xffff0000u) : (word << 16));
+        const int e = ch * TT + t;  // element index within the lane's words
+        const float xv = f[e / VE][e % VE];
         float acc = 0.f;
         acc += wt[ch][0] * w0;
         acc += wt[ch][1] * w1;
@@ -261,13 +311,23 @@ __global__ __launch_bounds__(256) void conv_suffix_ct_bf16(
         w0 = w1;
         w1 = w2;
         w2 = xv;
-        float y = round_bf(acc);
-        if (silu) y = silu_fast(y);
-        o[e / 8][(e % 8) / 2] |= (uint32_t)f2bf(y) << (16 * (e & 1));
+        y[e / VE][e % VE] = acc;
       }
     }
+    u32x4* o = (u32x4*)(out + (n0 + j) * so_n + off);
 #pragma unroll
-    for (int k = 0; k < TT; ++k) ((u32x4*)(out + (n0 + j) * so_n + off))[k] = o[k];
+    for (int k = 0; k < TT; ++k) cur[k] = ConvVec<T>::finish(y[k], silu);
+    if constexpr (TT > 1) {
+#pragma unroll
+      for (int k = 0; k < TT; ++k) own[slot(lane * TT + k)] = cur[k];
+      wave_order();
+#pragma unroll
+      for (int k = 0; k < TT; ++k) cur[k] = own[slot(k * 64 + lane)];
+      wave_order();
+    }
+#pragma unroll
+    for (int k = 0; k < TT; ++k)
+      if (k * 64 + lane < nw) o[k * 64 + lane] = cur[k];
   }
 }
 
@@ -395,6 +455,66 @@ int launch_scalar(const void* x, int64_t sx_n, int64_t sx_c, int64_t sx_t, const
   return kad_launch_status("conv_suffix_scalar");
 }
 
+// 16-byte words of channels: the vector kernels where the layout has them, the
+// scalar one for other strides, widths and a bias
+template <typename T>
+int launch_typed(const void* x, int64_t sx_n, int64_t sx_c, int64_t sx_t, const void* state,
+                 int64_t ss_b, int64_t ss_c, int64_t ss_t, int history, const void* w, int width,
+                 const void* bias, void* out, int64_t so_n, int64_t so_c, int64_t so_t, int B,
+                 int W, int C, int T_, int silu, hipStream_t s) {
+  constexpr int VE = ConvVec<T>::VE;
+  const bool words = width == 4 && bias == nullptr && C % VE == 0 && sx_n % VE == 0 &&
+                     so_n % VE == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
+                     ((uintptr_t)w % 16) == 0;
+  // token-major rows (of one token both layouts are that)
+  const bool vec = words && sx_c == 1 && so_c == 1 &&
+                   (T_ == 1 || (sx_t % VE == 0 && so_t % VE == 0));
+  // [BW, C, T] with each beam's C * T block contiguous (the reference's layout)
+  const bool ct = words && T_ <= 4 && sx_t == 1 && sx_c == T_ && so_t == 1 && so_c == T_;
+  const int groups = (int)kad_cdiv(C / VE, 256);
+  // fewer beams per thread where that leaves fewer than four workgroups per CU
+  int beams = kConvBeams;
+  while (beams > 1 && (int64_t)B * kad_cdiv(W, beams) * groups < 1024) beams /= 2;
+  const int nbg = (int)kad_cdiv(W, beams);
+  if (vec) {
+    KAD_REQUIRE((int64_t)B * nbg < 2147483647, "too many beams for the grid");
+    const int64_t runs = T_ > 4 ? kad_cdiv(T_, kConvRun) : 1;
+    KAD_REQUIRE(runs < 65536, "too many tokens for the grid");
+    const dim3 grid((unsigned)(B * nbg), (unsigned)groups, (unsigned)runs);
+#define KAD_CONV_VEC(TTV)                                                                       \
+  hipLaunchKernelGGL((conv_suffix_vec<T, TTV>), grid, dim3(256), 0, s, (const T*)x, sx_n, sx_t, \
+                     (const T*)state, ss_b, ss_c, ss_t, history, (const T*)w, (T*)out, so_n,    \
+                     so_t, W, C, T_, nbg, beams, silu)
+    switch (T_) {
+      case 1: KAD_CONV_VEC(1); break;
+      case 2: KAD_CONV_VEC(2); break;
+      case 3: KAD_CONV_VEC(3); break;
+      case 4: KAD_CONV_VEC(4); break;
+      default: KAD_CONV_VEC(0); break;
+    }
+#undef KAD_CONV_VEC
+    return kad_launch_status("conv_suffix_vec");
+  }
+  if (ct) {
+    KAD_REQUIRE((int64_t)B * nbg < 2147483647, "too many beams for the grid");
+    const dim3 grid((unsigned)(B * nbg), (unsigned)groups);
+#define KAD_CONV_CT(TTV)                                                                        \
+  hipLaunchKernelGGL((conv_suffix_ct<T, TTV>), grid, dim3(256), 0, s, (const T*)x, sx_n,        \
+                     (const T*)state, ss_b, ss_c, ss_t, history, (const T*)w, (T*)out, so_n, W, \
+                     C, nbg, beams, silu)
+    switch (T_) {
+      case 1: KAD_CONV_CT(1); break;
+      case 2: KAD_CONV_CT(2); break;
+      case 3: KAD_CONV_CT(3); break;
+      default: KAD_CONV_CT(4); break;
+    }
+#undef KAD_CONV_CT
+    return kad_launch_status("conv_suffix_ct");
+  }
+  return launch_scalar<T>(x, sx_n, sx_c, sx_t, state, ss_b, ss_c, ss_t, history, w, width, bias,
+                          out, so_n, so_c, so_t, B, W, C, T_, silu, s);
+}
+
 }  // namespace
 
 extern "C" int kad_causal_conv_suffix(const void* x, int64_t sx_n, int64_t sx_c, int64_t sx_t,
@@ -409,63 +529,14 @@ extern "C" int kad_causal_conv_suffix(const void* x, int64_t sx_n, int64_t sx_c,
   KAD_REQUIRE(history >= width - 1, "state history %d shorter than width-1", history);
   KAD_REQUIRE((int64_t)B * W * C < ((int64_t)1 << 40), "problem too large");
   hipStream_t s = (hipStream_t)stream;
-  const bool vec = dtype == KAD_DTYPE_BF16 && width == 4 && bias == nullptr && sx_c == 1 &&
-                   so_c == 1 && C % 8 == 0 && sx_n % 8 == 0 && sx_t % 8 == 0 && so_n % 8 == 0 &&
-                   so_t % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
-                   ((uintptr_t)weight % 16) == 0;
-  if (vec) {
-    const int nbg = (int)kad_cdiv(W, kConvBeams);
-    KAD_REQUIRE((int64_t)B * nbg < 2147483647, "too many beams for the grid");
-    const dim3 grid((unsigned)(B * nbg), (unsigned)kad_cdiv(C / 8, 256));
-#define KAD_CONV_VEC(TTV)                                                                    \
-  hipLaunchKernelGGL((conv_suffix_vec_bf16<TTV>), grid, dim3(256), 0, s, (const bf16_t*)x,   \
-                     sx_n, sx_t, (const bf16_t*)state, ss_b, ss_c, ss_t, history,             \
-                     (const bf16_t*)weight, (bf16_t*)out, so_n, so_t, W, C, T, nbg,           \
-                     activation_silu)
-    switch (T) {
-      case 1: KAD_CONV_VEC(1); break;
-      case 2: KAD_CONV_VEC(2); break;
-      case 3: KAD_CONV_VEC(3); break;
-      case 4: KAD_CONV_VEC(4); break;
-      default: KAD_CONV_VEC(0); break;
-    }
-#undef KAD_CONV_VEC
-    return kad_launch_status("conv_suffix_vec_bf16");
-  }
-  // [BW, C, T] with each beam's C * T block contiguous (the reference's layout)
-  const bool ct = dtype == KAD_DTYPE_BF16 && width == 4 && bias == nullptr && T <= 4 &&
-                  sx_t == 1 && sx_c == T && so_t == 1 && so_c == T && C % 8 == 0 &&
-                  sx_n % 8 == 0 && so_n % 8 == 0 && ((uintptr_t)x % 16) == 0 &&
-                  ((uintptr_t)out % 16) == 0 && ((uintptr_t)weight % 16) == 0;
-  if (ct) {
-    const int nbg = (int)kad_cdiv(W, kConvBeams);
-    KAD_REQUIRE((int64_t)B * nbg < 2147483647, "too many beams for the grid");
-    const dim3 grid((unsigned)(B * nbg), (unsigned)kad_cdiv(C / 8, 256));
-#define KAD_CONV_CT(TTV)                                                                     \
-  hipLaunchKernelGGL((conv_suffix_ct_bf16<TTV>), grid, dim3(256), 0, s, (const bf16_t*)x,    \
-                     sx_n, (const bf16_t*)state, ss_b, ss_c, ss_t, history,                   \
-                     (const bf16_t*)weight, (bf16_t*)out, so_n, W, C, nbg, activation_silu)
-    switch (T) {
-      case 1: KAD_CONV_CT(1); break;
-      case 2: KAD_CONV_CT(2); break;
-      case 3: KAD_CONV_CT(3); break;
-      default: KAD_CONV_CT(4); break;
-    }
-#undef KAD_CONV_CT
-    return kad_launch_status("conv_suffix_ct_bf16");
-  }
-  if (dtype == KAD_DTYPE_BF16)
-    return launch_scalar<bf16_t>(x, sx_n, sx_c, sx_t, state, ss_b, ss_c, ss_t, history, weight,
-                                 width, bias, out, so_n, so_c, so_t, B, W, C, T,
-                                 activation_silu, s);
-  if (dtype == KAD_DTYPE_F32)
-    return launch_scalar<float>(x, sx_n, sx_c, sx_t, state, ss_b, ss_c, ss_t, history, weight,
-                                width, bias, out, so_n, so_c, so_t, B, W, C, T, activation_silu,
-                                s);
-  if (dtype == KAD_DTYPE_F16)
-    return launch_scalar<_Float16>(x, sx_n, sx_c, sx_t, state, ss_b, ss_c, ss_t, history, weight,
-                                   width, bias, out, so_n, so_c, so_t, B, W, C, T,
-                                   activation_silu, s);
+#define KAD_CONV(T)                                                                            \
+  return launch_typed<T>(x, sx_n, sx_c, sx_t, state, ss_b, ss_c, ss_t, history, weight, width, \
+                         bias, out, so_n, so_c, so_t, B, W, C, T_, activation_silu, s)
+  const int T_ = T;
+  if (dtype == KAD_DTYPE_BF16) KAD_CONV(bf16_t);
+  if (dtype == KAD_DTYPE_F32) KAD_CONV(float);
+  if (dtype == KAD_DTYPE_F16) KAD_CONV(_Float16);
+#undef KAD_CONV
   KAD_UNSUPPORTED("causal conv supports bf16, fp16 and fp32, got dtype %d", dtype);
 }
 

@@ -237,6 +237,30 @@ def test_conv_reference_layout_equals_token_major(device, T, history):
     assert ((a - e).abs() <= (e.abs() * 2 ** -7).clamp_min(1e-30)).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,W,C,T,history", [
+    (2, 1, 8, 1, 4), (3, 13, 776, 2, 3), (1, 9, 2056, 3, 4), (2, 17, 520, 4, 6),
+    (2, 3, 512, 5, 4), (1, 2, 264, 16, 3), (2, 1, 768, 33, 4), (1, 1, 6144, 50, 3),
+])
+def test_conv_word_kernels_equal_the_scalar_one(device, dtype, B, W, C, T, history):
+    """Both 16-byte-word kernels, in both layouts and of every type, against the
+    scalar kernel's bits (which an x with strides of its own selects): channel
+    counts off the waves and workgroups, beam groups, suffixes around the
+    16-token runs, and both layouts of the taps."""
+    x, st, w = conv_inputs(B, W, C, T, seed=C + T, history=history)
+    x, st, w = (t.to(dtype).to(device) for t in (x, st, w))
+    odd = torch.empty(B * W, C, T + 1, dtype=dtype, device=device)[:, :, :T]
+    want = ops.causal_conv1d(odd.copy_(x), st, w, beam_width=W)
+    rows = x.transpose(1, 2).contiguous().transpose(1, 2)
+    taps = st.transpose(1, 2).contiguous().transpose(1, 2)
+    assert torch.equal(ops.causal_conv1d(x, st, w, beam_width=W), want)
+    assert torch.equal(ops.causal_conv1d(x, taps, w, beam_width=W), want)
+    assert torch.equal(ops.causal_conv1d(rows, st, w, beam_width=W), want)
+    linear = ops.causal_conv1d(odd, st, w, beam_width=W, activation=None)
+    assert torch.equal(ops.causal_conv1d(rows, st, w, beam_width=W, activation=None), linear)
+    assert torch.equal(ops.causal_conv1d(x, st, w, beam_width=W, activation=None), linear)
+
+
 def test_conv_golden_fixture(device):
     f = load_npz("ops_bf16.npz")
     x, st, w = (bf16_from_bits(f[n]) for n in ("conv_x", "conv_state", "conv_w"))
