@@ -503,6 +503,79 @@ int kad_cache_prefetch(const void* p0, int64_t bytes0, const void* p1, int64_t b
                        kad_stream_t stream);
 
 /* --------------------------------------------------------------------------
+ * A Qwen3.5 bf16 model's layers as one call per pass: the entry points above
+ * in the order the reference adapter's prefill and decode take their steps
+ * (src/kadllm/adapters/qwen3_5.py:106-235), enqueued on one stream.  All
+ * pointers but the structs and the per-layer arrays are device memory; every
+ * buffer is the caller's and nothing is kept after the call returns.
+ *
+ * kad_qwen_model  packed weights: w_gu [2 ffn, hidden] in [gate 32 | up 32] row
+ *   blocks, w_down [hidden, ffn], w_in [conv_dim + vd, hidden] (q | k | v | z),
+ *   w_ab [ab_rows, hidden] (a | b), w_qkv [(2 q_heads + 2 kv_heads) head_dim,
+ *   hidden]; conv_dim = 2 kd + vd; rows of gdn_cols hold [q|k|v | z | a|b | pad].
+ * kad_qwen_prefill  layers 0 .. layers - 1 over x [B*L, hidden] (updated in
+ *   place).  state0/1[i]: a linear layer's conv state [B, conv_dim, 4] and fp32
+ *   state [B, v_heads, k_dim, v_dim], an attention layer's K and V
+ *   [B, kv_heads, L, head_dim] (written).  Scratch: n [B*L, hidden],
+ *   h [B*L, ffn], proj [B*L, max(gdn_cols, qkv columns)], mixed
+ *   [B*L, max(vd, q_heads head_dim)], q [B*L, q_heads head_dim], g fp32 and
+ *   beta bf16 [B*L, v_heads], conv: the workspace of kad_gemm_bf16_conv
+ *   (fuse_conv) or [B*L, conv_dim], chunk_ws as kad_gdn_chunk_gated.
+ * kad_qwen_decode_step  all layers over each beam's new token, x [B*W, hidden],
+ *   suffixes of T = 1 or 2 tokens, the first in the parents' rows (parents
+ *   [B, W], prev0/1[i] as the previous level's next0/1[i]: a linear layer's
+ *   rows [B*Wp*(T-1), gdn_cols], an attention layer's K and V
+ *   [B*Wp, T-1, kv_heads, head_dim]); next0/1 written with keep.  prefix[i]: a
+ *   linear layer's conv state (p0, strides s0..s2, history slots) and state
+ *   (p1, dtype); an attention layer's K, V (p0, p1, strides of [B, L, heads],
+ *   history = L).  Scratch as above over B*W rows, rows_ws [B*W, gdn_cols],
+ *   qkv [B*W, qkv columns], k_ws and v_ws [B*W, T, kv_heads, head_dim], ab
+ *   [B*W*T, ab_rows], g and beta [B*W*T, v_heads]. */
+typedef struct {
+  int linear; /* 1: gated delta layer, 0: attention */
+  const void *input_norm, *post_norm, *w_gu, *w_down;
+  const void *w_in, *w_ab, *conv_w, *A_log, *dt_bias, *norm_w, *w_out;
+  const void *w_qkv, *q_norm, *k_norm, *w_o;
+} kad_qwen_layer;
+
+typedef struct {
+  const kad_qwen_layer* layers;
+  const float* inv_freq;
+  int n_layers, hidden, ffn, conv_dim, kd, vd, gdn_cols, ab_rows;
+  int k_heads, v_heads, k_dim, v_dim, q_heads, kv_heads, head_dim, rot;
+  float eps, gdn_scale, attn_scale;
+} kad_qwen_model;
+
+typedef struct {
+  int layers, B, L, fuse_conv;
+  void **state0, **state1;
+  void *x, *n, *h, *proj, *mixed, *q, *beta, *conv, *chunk_ws;
+  float* g;
+  int64_t conv_bytes, chunk_bytes;
+} kad_qwen_prefill_args;
+
+typedef struct {
+  const void *p0, *p1;
+  int64_t s0, s1, s2;
+  int history, dtype;
+} kad_qwen_prefix;
+
+typedef struct {
+  int B, W, Wp, T, keep, prefetch;
+  int64_t pos;
+  const int64_t* parents;
+  const kad_qwen_prefix* prefix;
+  void **prev0, **prev1, **next0, **next1;
+  void *x, *n, *h, *mixed, *q, *qkv, *rows_ws, *k_ws, *v_ws, *ab, *beta;
+  float* g;
+} kad_qwen_step_args;
+
+int kad_qwen_prefill(const kad_qwen_model* m, const kad_qwen_prefill_args* a,
+                     kad_stream_t stream);
+int kad_qwen_decode_step(const kad_qwen_model* m, const kad_qwen_step_args* a,
+                         kad_stream_t stream);
+
+/* --------------------------------------------------------------------------
  * MFMA lane-layout self-test (no reference counterpart): C[16x16] = A[16x32]
  * B[32x16] (bf16 in, fp32 out, all row-major) computed by one wave with the
  * operand layout the kernels above assume for v_mfma_f32_16x16x32_bf16, and

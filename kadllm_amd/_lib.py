@@ -69,6 +69,8 @@ SIGNATURES = {
     "kad_embedding_f32": "ppplils",
     "kad_hbm_probe": "pplis",
     "kad_cache_prefetch": "plpls",
+    "kad_qwen_prefill": "pps",
+    "kad_qwen_decode_step": "pps",
     "kad_selftest_mfma_f32": "ppps",
     "kad_selftest_mfma16": "ppps",
     "kad_selftest_mfma32": "ppps",
@@ -131,6 +133,12 @@ def set_call_hook(hook):
     timing)."""
     global _call_hook
     _call_hook = hook
+
+
+def hooked():
+    """Whether a hook sees every call (callers that batch calls then make them
+    one by one)."""
+    return _call_hook is not None
 
 
 def _invoke(lib, name, args):

@@ -161,10 +161,9 @@ struct ConvVec {
 // kConvBeams beams of one request per thread (the request's weights and prefix
 // taps are loaded once); width 4 (3 taps), any T.  Grid: x = request x beam
 // group, y = channel groups of 256 threads, z = runs of kConvRun tokens of
-// suffixes longer than 4 (an fp32 model's whole prompts, which one thread per channel would
-// walk).  The next (beam,
-// token) row is loaded before the current one is computed so that every thread
-// keeps one 16-byte load in flight.
+// suffixes longer than 4 (an fp32 model's whole prompts, which one thread per
+// channel would walk).  The next (beam, token) row is loaded before the current
+// one is computed so that every thread keeps one 16-byte load in flight.
 constexpr int kConvBeams = 8, kConvRun = 16;
 
 // TT > 0: the suffix length fixed at compile time (the search's one- to

@@ -26,6 +26,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib, layers
+from .native_layers import NativeLayers
 from .attention import attention_prefill, prefix_attention_decode
 from .ops import REPLAY_MAX_T
 
@@ -179,6 +180,7 @@ class Qwen35Runner:
                 self.layers.append(_AttnLayer(w_qkv=w_qkv, q_norm=get(a + "q_norm.weight"),
                                               k_norm=get(a + "k_norm.weight"),
                                               w_o=get(a + "o_proj.weight"), **common))
+        self._native = None
         # optional observer: trace(phase, layer, x) after each layer with a copy
         # of the residual stream rows (the last position only past a pruned
         # last layer); phase is "prefill", "decode" or "step"
@@ -187,6 +189,19 @@ class Qwen35Runner:
         self.rot = rot
         self.inv_freq = (1.0 / (cfg.rope_theta ** (torch.arange(0, rot, 2, dtype=torch.float) / rot))
                          ).to(self.device)
+
+    def __getstate__(self):
+        # the native form holds addresses: a copy builds its own
+        return {**self.__dict__, "_native": None}
+
+    def _native_layers(self):
+        """The layers' one-call form, or None while something watches the
+        single steps (a trace, a call hook)."""
+        if self.trace is not None or _lib.hooked():
+            return None
+        if self._native is None:
+            self._native = NativeLayers(self)
+        return self._native
 
     # ------------------------------------------------------------------
     def _mlp(self, lyr, x, rows, prefetch=False):
@@ -208,6 +223,13 @@ class Qwen35Runner:
         layers.gemm(n, lyr.w_in, out=out[:, :c])
         return out
 
+    def conv_fuses(self, rows, L, lyr):
+        """Whether kad_gemm_bf16_conv takes a prefill's projection."""
+        C = self.conv_dim
+        return (L % 128 == 0 and rows % 256 == 0 and (C + self.vd) % 256 == 0 and C % 256 == 0
+                and self.cfg.hidden_size % 64 == 0 and lyr.conv_w.is_contiguous()
+                and lyr.conv_w.data_ptr() % 16 == 0)
+
     def _gdn_proj_conv(self, lyr, n, B, L, conv_state):
         """The prefill's projection rows and the causal conv (+ SiLU) of their
         q | k | v channels: (proj [rows, gdn_cols], conv) with conv the rows
@@ -222,9 +244,7 @@ class Qwen35Runner:
         dev = n.device
         stream = _lib.stream_of(n)
         w_in = lyr.w_in
-        if (L % 128 == 0 and rows % 256 == 0 and c % 256 == 0 and C % 256 == 0
-                and n.shape[1] % 64 == 0 and lyr.conv_w.is_contiguous()
-                and lyr.conv_w.data_ptr() % 16 == 0):
+        if self.conv_fuses(rows, L, lyr):
             proj = torch.empty(rows, self.gdn_cols, dtype=torch.bfloat16, device=dev)
             layers.gemm(n, lyr.w_ab, out=proj[:, c:c + lyr.w_ab.shape[0]])
             nb = ctypes.c_int64(0)
@@ -407,7 +427,14 @@ class Qwen35Runner:
         # position of each prompt is used (its logits); the prefix needs that
         # layer's state or K/V for every position, but not its outputs.
         x_last = x.view(B, L, -1)[:, -1]
+        native = self._native_layers()
+        first = 0
+        if native is not None and native.uniform:
+            first = len(self.layers) - 1
+            snap = native.prefill(self, x, B, L, first)
         for li, lyr in enumerate(self.layers):
+            if li < first:
+                continue
             terminal = li == len(self.layers) - 1
             n = layers.rmsnorm(x, lyr.input_norm, cfg.rms_norm_eps)
             if isinstance(lyr, _GdnLayer):
@@ -598,7 +625,12 @@ class Qwen35Runner:
         # once at HBM rate whether or not it was prefetched.
         prefetch = 2048 <= BW <= 16384
         new_layers = []
-        for li, (lyr, cached) in enumerate(zip(self.layers, prefix_layers)):
+        native = self._native_layers()
+        batched = native is not None and native.step_fits(T, prefix_layers)
+        if batched:
+            new_layers = native.decode_step(self, x, B, W, T, Wp, parents, prefix_layers,
+                                            prefix_length, cache, keep_cache, prefetch)
+        for li, (lyr, cached) in enumerate(zip(() if batched else self.layers, prefix_layers)):
             if prefetch and not isinstance(lyr, _GdnLayer):
                 layers.cache_prefetch(lyr.w_qkv)
             n = layers.rmsnorm(x, lyr.input_norm, cfg.rms_norm_eps)

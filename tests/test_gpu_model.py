@@ -630,3 +630,58 @@ def test_reference_bf16_run_replayed_through_hip(device):
         assert got.keys() == want.keys(), "search returns other beams than the reference's"
         for seq, sc in want.items():
             assert abs(got[seq] - sc) <= 3 * 2 * err + 1e-4, (seq, got[seq], sc)
+
+
+@pytest.mark.parametrize("last", ["full_attention", "linear_attention"])
+@pytest.mark.parametrize("B,L,W", [(1, 7, 10), (2, 128, 16), (3, 65, 5)])
+def test_layers_in_one_call_equal_the_steps(device, last, B, L, W):
+    """kad_qwen_prefill and kad_qwen_decode_step (one call per pass) against the
+    runner's own steps, which a call hook brings back: logits, prefix and cache
+    bit for bit, with the fused projection conv (L = 128) and without, kept and
+    last levels, and a deep copy of the adapter."""
+    import copy
+    from dataclasses import replace
+
+    from kadllm_amd import _lib
+    cfg = replace(tiny_hybrid_config(), linear_key_head_dim=128, linear_value_head_dim=128,
+                  layer_types=("linear_attention", "full_attention", "linear_attention", last))
+    sd = random_state_dict(cfg, seed=4, dtype=torch.bfloat16, device=device)
+    adapter = Qwen35GRBeamAdapter(*native_model(cfg, sd))
+    g = torch.Generator().manual_seed(B * L)
+
+    def ints(high, *shape):
+        return torch.randint(0, high, shape, generator=g).to(device)
+
+    ids, first = ints(cfg.vocab_size, B, L), ints(cfg.vocab_size, B, W, 1)
+    parents, token = ints(W, B, W), ints(cfg.vocab_size, B, W, 1)
+    second = torch.cat((first.gather(1, parents[..., None]), token), 2)
+
+    def passes(ad):
+        pre = ad.prefill(ids)
+        l1, c1 = ad.decode_incremental(first, None, pre.state, None)
+        l2, c2 = ad.decode_incremental(second, parents, pre.state, c1)
+        l3, _ = ad.decode_incremental(second, parents, pre.state, c1, keep_cache=False)
+        out = [pre.logits, l1, l2, l3, *(t for lyr in pre.state.layers for t in lyr)]
+        for c in (c1, c2):
+            for e in c.layers:
+                # the projection rows' pad columns are never written
+                out += list(e) if isinstance(e, tuple) else [e[:, :ad._runner.conv_dim
+                                                               + ad._runner.vd]]
+        return out
+
+    names = []
+
+    def hook(name, args, launch):
+        names.append(name)
+        launch()
+
+    _lib.set_call_hook(hook)
+    try:
+        steps = passes(adapter)
+    finally:
+        _lib.set_call_hook(None)
+    assert "kad_qwen_prefill" not in names and "kad_gemm_bf16" in names
+    for ad in (adapter, copy.deepcopy(adapter)):
+        for a, b in zip(passes(ad), steps):
+            assert torch.equal(a, b)
+    assert adapter._runner._native is not None
