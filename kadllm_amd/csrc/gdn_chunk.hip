@@ -133,7 +133,13 @@ __device__ __forceinline__ void hf_l2_apply(u32x4& r, float rs) {
 }
 
 // ---------------------------------------------------------------------------
-template <int K, bool HF>
+// N16: T' and In as A fragments of 16x16x32 MFMAs (gdn_chunk_scan16) instead of
+// 32x32x16 ones: fragment f of the 6 is the 16 rows it16(f) against the 32 tokens
+// of step s16(f), lane L holding X[it*16 + L%16][s*32 + (t/4)*16 + (L/16)*4 + t%4].
+__host__ __device__ __forceinline__ constexpr int it16(int f) { return f < 2 ? f : 2 + (f - 2) / 2; }
+__host__ __device__ __forceinline__ constexpr int s16(int f) { return f < 2 ? 0 : (f - 2) % 2; }
+
+template <int K, bool HF, bool N16>
 __global__ __launch_bounds__(kPrepThreads) void gdn_chunk_prep(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, int64_t ld_qk,
     const void* __restrict__ g, int gdt, const void* __restrict__ beta, int bdt, int64_t ld_gate,
@@ -258,13 +264,57 @@ __global__ __launch_bounds__(kPrepThreads) void gdn_chunk_prep(
       const bf16x8 b = as_bf16x8(*(const u32x4*)(kb + (tj * 32 + fr) * LD + s * 16 + fk));
       const bf16x8 bq = as_bf16x8(*(const u32x4*)(qb + (ti * 32 + fr) * LD + s * 16 + fk));
       gram = mfma32x32x16(a, b, gram);
-      inT = mfma32x32x16(b, bq, inT);
+      if constexpr (!N16) inT = mfma32x32x16(b, bq, inT);
+    }
+  }
+  // N16: In^T in 16 x 16 tiles, two (tokens s*32 and s*32 + 16) to a fragment,
+  // whose accumulators are the fragment's order; wave w forms fragments w, w + 4
+  f32x4 in16[2][2];
+  if constexpr (N16) {
+    const int c16 = lane & 15, k16 = (lane >> 4) * 8;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int f = min(wave + 4 * u, ChunkRec::frags - 1);
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 0; st < K / 32; ++st) {
+          const bf16x8 a = as_bf16x8(*(const u32x4*)(
+              kb + (s16(f) * 32 + half * 16 + c16) * LD + st * 32 + k16));
+          const bf16x8 b =
+              as_bf16x8(*(const u32x4*)(qb + (it16(f) * 16 + c16) * LD + st * 32 + k16));
+          acc = mfma16x16x32(a, b, acc);
+        }
+        in16[u][half] = acc;
+      }
     }
   }
   __syncthreads();  // rows no longer needed: the region becomes A / T'
   // In_ij = (q^_i . k^_j) qmul_i kmul_j e^{G_i - G_j} for j <= i, as hi/lo
   // A fragments (it = ti, s = tj * 2 + half) straight from the accumulators
-  if (wave < 3) {
+  if constexpr (N16) {
+    bf16_t* inf = (bf16_t*)(rec + ChunkRec::in);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int f = wave + 4 * u;
+      if (f >= ChunkRec::frags) break;
+      const int irow = it16(f) * 16 + (lane & 15);
+      const float qmi = qmul[irow], gi = g2s[irow];
+      float x[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const int j = s16(f) * 32 + (t / 4) * 16 + (lane >> 4) * 4 + t % 4;
+        x[t] = j <= irow ? (in16[u][t / 4][t % 4] * qmi * kmul[j]) *
+                               __builtin_amdgcn_exp2f(gi - g2s[j])
+                         : 0.f;
+      }
+      bf16x8 ih, il;
+      split8(x, ih, il);
+      *(bf16x8*)(inf + ((f * 2 + 0) * 64 + lane) * 8) = ih;
+      *(bf16x8*)(inf + ((f * 2 + 1) * 64 + lane) * 8) = il;
+    }
+  } else if (wave < 3) {
     const int irow = ti * 32 + (lane & 31);
     const float qmi = qmul[irow], gi = g2s[irow];
 #pragma unroll
@@ -375,10 +425,11 @@ __global__ __launch_bounds__(kPrepThreads) void gdn_chunk_prep(
       if (fl_ >= ChunkRec::frags * 64) break;
       const int f = fl_ >> 6, L = fl_ & 63;
       const int it = f < 2 ? 0 : 1, s = f < 2 ? f : f - 2;
-      const int i = it * 32 + (L & 31), jb = s * 16 + (L >> 5) * 4;
+      const int i = N16 ? it16(f) * 16 + (L & 15) : it * 32 + (L & 31);
+      const int jb = N16 ? s16(f) * 32 + (L >> 4) * 4 : s * 16 + (L >> 5) * 4;
       float x[8];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) x[t] = Tm[i][jb + (t / 4) * 8 + t % 4];
+      for (int t = 0; t < 8; ++t) x[t] = Tm[i][jb + (t / 4) * (N16 ? 16 : 8) + t % 4];
       bf16x8 fh, fl;
       split8(x, fh, fl);
       *(bf16x8*)(tf + ((f * 2 + 0) * 64 + L) * 8) = fh;
@@ -773,6 +824,239 @@ __global__ __launch_bounds__(V * 2, V == 128 ? 2 : 1) void gdn_chunk_scan(
   }
 }
 
+// The scan with 16 value columns per wave, 64 per workgroup, on 16x16x32 MFMAs:
+// half the MFMAs, splits and LDS reads a wave's chunk takes in gdn_chunk_scan.
+// A chunk is one dependent step, so where the (sequence, head) pairs leave the
+// chip idle the step's length is the whole time, and halving it over twice the
+// workgroups is worth reading q, k, T' and In twice: 4 x 16 heads of 1,000
+// tokens 111 -> 77 us (with the prep, 128.6 -> 95.3; loading a chunk ahead in
+// registers made either kernel 5% slower).
+//
+// S[kt][e] is row kt*16 + 4 (lane/16) + e, column lane%16 of the wave's 16.
+// Every product's K runs in the order of the accumulators: slot t of lane group
+// j = lane/16 is entry (t/4)*16 + 4 j + t%4 of a 32-deep step, so that two 16-row
+// accumulator tiles are a B fragment as they stand.
+constexpr int kCols16 = 64;
+
+template <int K, int V, bool HF>
+__global__ __launch_bounds__(256, 2) void gdn_chunk_scan16(
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, int64_t ld_qk,
+    const bf16_t* __restrict__ v, int64_t ld_v, const uint8_t* __restrict__ ws,
+    const void* __restrict__ state0, int sdt, int beams_per_state, bf16_t* __restrict__ out,
+    int64_t ld_out, float* __restrict__ final_state, int T, int H, int HV, int nchunks) {
+  constexpr int KT = K / 16, KS = K / 32, LDK = K + 8, LDV = kCols16 + 8, CPR = K / 8;
+  constexpr int NTH = 256, NVB = V / kCols16;
+  __shared__ __attribute__((aligned(16))) bf16_t kb[kC * LDK];
+  __shared__ __attribute__((aligned(16))) bf16_t qb[kC * LDK];
+  __shared__ __attribute__((aligned(16))) bf16_t vb[kC * LDV];
+  __shared__ __attribute__((aligned(16))) bf16_t tf[ChunkRec::tf_elems];
+  __shared__ __attribute__((aligned(16))) float sc[kScal][kC];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int c = lane & 15, j4 = (lane >> 4) * 4;
+  const int nh = blockIdx.x / NVB, v0 = (blockIdx.x % NVB) * kCols16;
+  const int n = nh / HV, hv = nh % HV;
+  const int h = hv / (HV / H);
+  const int vcol = wave * 16 + c;  // column within the workgroup's 64
+
+  f32x4 S[KT];
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      S[kt][e] = state0 ? load_as_float(state0,
+                                        ((int64_t)(n / beams_per_state) * HV + hv) * K * V +
+                                            (int64_t)(kt * 16 + j4 + e) * V + v0 + vcol,
+                                        sdt)
+                        : 0.f;
+
+  constexpr int kRowU = kC * CPR / NTH, kVU = kC * kCols16 / 8 / NTH;
+  constexpr int kTU = ChunkRec::tf_elems / 8 / NTH, kSU = (kScal * kC + NTH - 1) / NTH;
+  static_assert(kRowU * NTH == kC * CPR && kTU * NTH * 8 == ChunkRec::tf_elems,
+                "chunk tiles must split evenly");
+  for (int ch = 0; ch < nchunks; ++ch) {
+    const int t0 = ch * kC, nt = min(kC, T - t0);
+    const int64_t row0 = (int64_t)n * T + t0;
+    const uint8_t* rec = ws + ((size_t)nh * nchunks + ch) * ChunkRec::bytes;
+    const float* scg = (const float*)(rec + ChunkRec::scal);
+    // ---- the chunk's data, every load before the first LDS store
+    u32x4 rk[kRowU], rq[kRowU], rv[kVU], rt[kTU];
+    float rs[kSU], krs[kRowU], qrs[kRowU];
+#pragma unroll
+    for (int u = 0; u < kRowU; ++u) {
+      const int i = (tid + u * NTH) / CPR, chn = tid % CPR;
+      const bool live = i < nt;
+      const int64_t off = (row0 + (live ? i : 0)) * ld_qk + (int64_t)h * K + chn * 8;
+      rk[u] = live ? *(const u32x4*)(k + off) : u32x4{0u, 0u, 0u, 0u};
+      rq[u] = live ? *(const u32x4*)(q + off) : u32x4{0u, 0u, 0u, 0u};
+      if constexpr (HF) {
+        krs[u] = scg[S_KRS * kC + i];
+        qrs[u] = scg[S_QRS * kC + i];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kVU; ++u) {
+      const int i = (tid + u * NTH) / 8, v8 = (tid % 8) * 8;
+      rv[u] = i < nt ? *(const u32x4*)(v + (row0 + i) * ld_v + (int64_t)hv * V + v0 + v8)
+                     : u32x4{0u, 0u, 0u, 0u};
+    }
+    const bf16_t* tfg = (const bf16_t*)(rec + ChunkRec::tf);
+#pragma unroll
+    for (int u = 0; u < kTU; ++u) rt[u] = *(const u32x4*)(tfg + (tid + u * NTH) * 8);
+#pragma unroll
+    for (int u = 0; u < kSU; ++u) {
+      const int e = tid + u * NTH;
+      rs[u] = e < kScal * kC ? scg[e] : 0.f;
+    }
+    __syncthreads();  // previous chunk done with LDS
+#pragma unroll
+    for (int u = 0; u < kRowU; ++u) {
+      const int i = (tid + u * NTH) / CPR, chn = tid % CPR;
+      if constexpr (HF) {
+        hf_l2_apply(rk[u], krs[u]);
+        hf_l2_apply(rq[u], qrs[u]);
+      }
+      *(u32x4*)(kb + i * LDK + chn * 8) = rk[u];
+      *(u32x4*)(qb + i * LDK + chn * 8) = rq[u];
+    }
+#pragma unroll
+    for (int u = 0; u < kVU; ++u)
+      *(u32x4*)(vb + ((tid + u * NTH) / 8) * LDV + (tid % 8) * 8) = rv[u];
+#pragma unroll
+    for (int u = 0; u < kTU; ++u) *(u32x4*)(tf + (tid + u * NTH) * 8) = rt[u];
+#pragma unroll
+    for (int u = 0; u < kSU; ++u) {
+      const int e = tid + u * NTH;
+      if (e < kScal * kC) sc[e / kC][e % kC] = rs[u];
+    }
+    __syncthreads();
+
+    // A fragment of rows `row` .. of a [token][feature] tile, step s
+    auto row_frag = [&](const bf16_t* tile, int row, int s) {
+      const bf16_t* p = tile + (row + c) * LDK + s * 32 + j4;
+      const u32x2 lo = *(const u32x2*)p, up = *(const u32x2*)(p + 16);
+      return as_bf16x8(u32x4{lo[0], lo[1], up[0], up[1]});
+    };
+    // B fragments (hi, lo) of two 16-row accumulator tiles
+    auto tile_frags = [&](const f32x4& a, const f32x4& b, bf16x8& hi, bf16x8& lo) {
+      const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+      split8(x, hi, lo);
+    };
+    // ---- k S and q S
+    f32x4 KS4[4], QS4[4];
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt) KS4[tt] = QS4[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      bf16x8 sh, sl;
+      tile_frags(S[2 * s], S[2 * s + 1], sh, sl);
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) {
+        const bf16x8 ak = row_frag(kb, tt * 16, s), aq = row_frag(qb, tt * 16, s);
+        KS4[tt] = mfma16x16x32(ak, sh, KS4[tt]);
+        KS4[tt] = mfma16x16x32(ak, sl, KS4[tt]);
+        QS4[tt] = mfma16x16x32(aq, sh, QS4[tt]);
+        QS4[tt] = mfma16x16x32(aq, sl, QS4[tt]);
+      }
+    }
+    // ---- Z_j = beta_j v_j - ZK_j (k S)_j
+    f32x4 Z[4];
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt) {
+      const f32x4 zk = *(const f32x4*)&sc[S_ZK][tt * 16 + j4];
+      const f32x4 bt = *(const f32x4*)&sc[S_BT][tt * 16 + j4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        Z[tt][e] = fmaf(-zk[e], KS4[tt][e], bt[e] * bf2f(vb[(tt * 16 + j4 + e) * LDV + vcol]));
+    }
+    // ---- v_new = Z + T' Z, then o = e^G q S + In v_new (fragment f: rows it16,
+    // tokens of step s16)
+    bf16x8 zh[2], zl[2], vh[2], vl[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) tile_frags(Z[2 * s], Z[2 * s + 1], zh[s], zl[s]);
+    auto product = [&](const bf16_t* frags, int f, const bf16x8& bh, const bf16x8& bl, f32x4 acc) {
+      const bf16x8 ah = *(const bf16x8*)(frags + ((f * 2 + 0) * 64 + lane) * 8);
+      const bf16x8 al = *(const bf16x8*)(frags + ((f * 2 + 1) * 64 + lane) * 8);
+      acc = mfma16x16x32(ah, bh, acc);
+      acc = mfma16x16x32(ah, bl, acc);
+      return mfma16x16x32(al, bh, acc);
+    };
+    f32x4 VN[4];
+#pragma unroll
+    for (int it = 0; it < 4; ++it) VN[it] = Z[it];
+#pragma unroll
+    for (int f = 0; f < ChunkRec::frags; ++f)
+      VN[it16(f)] = product(tf, f, zh[s16(f)], zl[s16(f)], VN[it16(f)]);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) tile_frags(VN[2 * s], VN[2 * s + 1], vh[s], vl[s]);
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      const f32x4 eq = *(const f32x4*)&sc[S_EQ][it * 16 + j4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) QS4[it][e] *= eq[e];
+    }
+#pragma unroll
+    for (int f = 0; f < ChunkRec::frags; ++f)
+      QS4[it16(f)] = product(tf + ChunkRec::frag_elems, f, vh[s16(f)], vl[s16(f)], QS4[it16(f)]);
+    __syncthreads();  // every wave has read the v tile, which takes the output
+#pragma unroll
+    for (int it = 0; it < 4; ++it)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) vb[(it * 16 + j4 + e) * LDV + vcol] = f2bf(QS4[it][e]);
+    // ---- S <- e^{G_last} S + sum_i (kmul_i e^{G_last - G_i}) k_i v_new_i^T
+    bf16x8 wh[2], wl[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      f32x4 w[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const f32x4 wu = *(const f32x4*)&sc[S_WU][(2 * s + u) * 16 + j4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[u][e] = VN[2 * s + u][e] * wu[e];
+      }
+      tile_frags(w[0], w[1], wh[s], wl[s]);
+    }
+    const float egl = sc[S_EG][kC - 1];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[kt][e] *= egl;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        // k^T: lane 4 e + m of a 16-lane group addresses token e of its four,
+        // features 4 m .. +3 of the tile's 16 (see kt_frag)
+        tr_v4s_t part[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const bf16_t* p = kb + (s * 32 + r * 16 + j4 + (c >> 2)) * LDK + kt * 16 + (c & 3) * 4;
+          part[r] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) tr_v4s_t*)p);
+        }
+        const u32x2 lo = __builtin_bit_cast(u32x2, part[0]);
+        const u32x2 up = __builtin_bit_cast(u32x2, part[1]);
+        const bf16x8 a = as_bf16x8(u32x4{lo[0], lo[1], up[0], up[1]});
+        S[kt] = mfma16x16x32(a, wh[s], S[kt]);
+        S[kt] = mfma16x16x32(a, wl[s], S[kt]);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kVU; ++u) {
+      const int i = (tid + u * NTH) / 8, v8 = (tid % 8) * 8;
+      if (i < nt)
+        *(u32x4*)(out + (row0 + i) * ld_out + (int64_t)hv * V + v0 + v8) =
+            *(const u32x4*)(vb + i * LDV + v8);
+    }
+  }
+  if (final_state) {
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        final_state[((int64_t)n * HV + hv) * K * V + (int64_t)(kt * 16 + j4 + e) * V + v0 + vcol] =
+            S[kt][e];
+  }
+}
+
 template <int K, int V>
 int launch_chunk(const void* q, const void* k, const void* v, int64_t ld_qk, int64_t ld_v,
                  const void* g, int gdt, const void* beta, int bdt, int64_t ld_gate,
@@ -785,7 +1069,7 @@ int launch_chunk(const void* q, const void* k, const void* v, int64_t ld_qk, int
   // transformers' bf16 l2norm rounding (hf_norm) or the operator's fp32
   // scales: an instantiation each, so the VALU-bound loops carry no test
 #define KAD_CHUNK(HFV, GV)                                                                     \
-  hipLaunchKernelGGL((gdn_chunk_prep<K, HFV>), dim3((unsigned)nrec), dim3(kPrepThreads), 0, s, \
+  hipLaunchKernelGGL((gdn_chunk_prep<K, HFV, false>), dim3((unsigned)nrec), dim3(kPrepThreads), 0, s, \
                      (const bf16_t*)q, (const bf16_t*)k, ld_qk, g, gdt, beta, bdt, ld_gate,    \
                      (uint8_t*)ws, T, H, HV, nchunks, scale);                                  \
   if (const int rc = kad_launch_status("gdn_chunk_prep")) return rc;                           \
@@ -794,6 +1078,33 @@ int launch_chunk(const void* q, const void* k, const void* v, int64_t ld_qk, int
                      (const bf16_t*)v, ld_v, (const uint8_t*)ws, state0, sdt, bps,             \
                      (bf16_t*)out, ld_out, fin, T, H, HV, nchunks, ga);                        \
   return kad_launch_status("gdn_chunk_scan")
+#define KAD_CHUNK16(HFV)                                                                       \
+  hipLaunchKernelGGL((gdn_chunk_prep<K, HFV, true>), dim3((unsigned)nrec), dim3(kPrepThreads), \
+                     0, s, (const bf16_t*)q, (const bf16_t*)k, ld_qk, g, gdt, beta, bdt,       \
+                     ld_gate, (uint8_t*)ws, T, H, HV, nchunks, scale);                         \
+  if (const int rc = kad_launch_status("gdn_chunk_prep")) return rc;                           \
+  hipLaunchKernelGGL((gdn_chunk_scan16<K, V, HFV>),                                            \
+                     dim3((unsigned)((int64_t)N * HV * (V / kCols16))), dim3(256), 0, s,       \
+                     (const bf16_t*)q, (const bf16_t*)k, ld_qk, (const bf16_t*)v, ld_v,        \
+                     (const uint8_t*)ws, state0, sdt, bps, (bf16_t*)out, ld_out, fin, T, H,    \
+                     HV, nchunks);                                                             \
+  if (const int rc = kad_launch_status("gdn_chunk_scan16")) return rc
+  // 64-column workgroups up to two per CU, where both kernels then hold as many:
+  // 16 sequences x 16 heads of 1,024 tokens 195 us in workgroups of all 128
+  // columns, 178 in two of 64; 24 (three per CU) 140 and 145
+  if ((int64_t)N * HV * (V / kCols16) <= 512) {
+    if (hf_norm) {
+      KAD_CHUNK16(true);
+    } else {
+      KAD_CHUNK16(false);
+    }
+    // a head's columns lie in two workgroups: the gated norm as its own kernel,
+    // the same arithmetic
+    if (gate)
+      return kad_rmsnorm_gated(out, ld_out, gate->z, gate->ldz, gate->w, out, ld_out,
+                               (int64_t)N * T, HV, V, gate->eps, (kad_stream_t)s);
+    return KAD_OK;
+  }
   // the gated output only with the transformers normalisation (the model
   // prefill, whose layer applies the norm)
   if (gate) {
@@ -803,6 +1114,7 @@ int launch_chunk(const void* q, const void* k, const void* v, int64_t ld_qk, int
     KAD_CHUNK(true, false);
   }
   KAD_CHUNK(false, false);
+#undef KAD_CHUNK16
 #undef KAD_CHUNK
 }
 

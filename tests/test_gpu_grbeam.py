@@ -212,6 +212,44 @@ def test_prefill_chunk_gated_equals_chunk_then_norm(device, L, K):
     assert torch.equal(s2.cpu(), s1.cpu()), "gated chunk final state differs"
 
 
+@pytest.mark.parametrize("N,HV", [(1, 2), (70, 4), (140, 4), (300, 4)])
+@pytest.mark.parametrize("K,V,T", [(128, 128, 1), (128, 128, 130), (64, 128, 70), (128, 64, 64),
+                                   (64, 64, 65)])
+def test_chunk_scans_match_oracle(device, N, HV, K, V, T):
+    """Both scans (16 columns a wave while 64-column workgroups number at most
+    two per CU, 32 beyond) against the token-by-token rule, with and without an
+    initial state, chunks whole and partial; the gated form, which the wide scan
+    fuses and the narrow one launches, equals chunk then norm bit for bit."""
+    H = 2
+    q, k, v, g, beta, S = gdn_inputs(N, 1, T, H, HV, K, V, seed=N + T, state_std=0.1)
+    dev = [t.to(device) for t in (q, k, v, g, beta)]
+    ws = _lib.gdn_chunk_workspace(N, T, HV, K, device)
+    o = torch.empty(N, T, HV, V, dtype=torch.bfloat16, device=device)
+    f = torch.empty(N, HV, K, V, device=device)
+    some = sorted({0, N // 2, N - 1})       # the oracle on a few sequences
+    for state in (None, S):
+        sd = None if state is None else state.to(device)
+        args = (*map(_lib.ptr, dev[:3]), H * K, HV * V, 0, _lib.ptr(dev[3]), 2, _lib.ptr(dev[4]),
+                0, HV, _lib.ptr(sd), 2, 1)
+        tail = (_lib.ptr(ws), ws.numel(), N, T, H, HV, K, V, float(K ** -0.5))
+        _lib.call("kad_gdn_chunk", *args, _lib.ptr(o), HV * V, _lib.ptr(f), *tail, 0,
+                  _lib.stream_of(o))
+        eo, ef = ops_ref.gated_delta(*(t[some] for t in (q, k, v, g, beta)),
+                                     (torch.zeros_like(S) if state is None else state)[some],
+                                     return_final_state=True)
+        assert_close_rel(o[some].cpu(), eo, rtol=1e-2, atol_frac=3e-3, name="o")
+        assert_close_rel(f[some].cpu(), ef, rtol=1e-4, atol_frac=1e-5, name="final state")
+    z = torch.randn(N * T, HV * V, generator=torch.Generator().manual_seed(T)).bfloat16().to(device)
+    w = torch.linspace(0.5, 1.5, V).bfloat16().to(device)
+    _lib.call("kad_gdn_chunk", *args, _lib.ptr(o), HV * V, _lib.ptr(f), *tail, 1,
+              _lib.stream_of(o))
+    normed = layers.rmsnorm_gated(o.view(N * T, HV * V), z, w, 1e-6, HV)
+    y, f2 = torch.empty_like(normed), torch.empty_like(f)
+    _lib.call("kad_gdn_chunk_gated", *args, _lib.ptr(y), HV * V, _lib.ptr(f2), *tail, _lib.ptr(z),
+              HV * V, _lib.ptr(w), 1e-6, _lib.stream_of(o))
+    assert torch.equal(y, normed) and torch.equal(f2, f)
+
+
 @pytest.mark.parametrize("L", [1, 3, 50])
 def test_conv_prefill_and_state(device, L):
     B, C = 2, 64
