@@ -300,7 +300,8 @@ int launch_recurrent(const void* q, const void* k, const void* v, int64_t ld_qk,
 // workgroups.  Matrix rate bounds it (a step is 2 x 64 MFMAs of 32 cycles at
 // head dim 256, against 32 KB of K and V from L2 that arrive meanwhile: V
 // during S, the next K during O); 4 requests x 64 beams x 2 tokens, 500 fp32
-// keys: 1,100 us as one wave per row, 44 us here.
+// keys: 1,100 us as one wave per row, 38 us here (46 while each step loaded its
+// mask bytes, behind every load in flight, and scaled to each new maximum).
 //
 // Masked prefix keys have weight 0 and their V is not read as a number; a row
 // with no visible key gives zeros (ops.py:229-240).  The output is rounded to
@@ -441,7 +442,7 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
   const int w_lo = r0 / (a.Tq * G), w_hi = r1 / (a.Tq * G);
   // this lane's query row (rows past the end repeat the last one)
   const int row = min(r0 + c, a.rows - 1);
-  const int qw = row / (a.Tq * G), qt = row / G % a.Tq, qh = hk * G + row % G;
+  const int qw = row / (a.Tq * G), qt = row / G % a.Tq;
   const int qpos = qt + (a.Tk - a.Tq);  // its suffix position
   // suffix tokens that some row of the tile sees
   const int nsuf = w_lo == w_hi ? (r1 / G % a.Tq) + (a.Tk - a.Tq) + 1 : a.Tk;
@@ -475,19 +476,27 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
   // accumulator element r of lane l is C[(l/16)*4 + r][l%16].  The dims of a
   // 16-dim piece i meet in the order 16 i + 4 j + e (step e), so that a lane
   // reads its share of a row as 4-element vectors.
-  float qf[NQ][4];
+  // The 16 query rows come through LDS (where the partial outputs go later), one
+  // load of each for the four waves.
+  float* qs = po[0];
   {
-    const TIN* qp = (const TIN*)a.q + (n0 + qw) * a.sq_n + (int64_t)qt * a.sq_t +
-                    (int64_t)qh * a.sq_h;
+    const int fr = min(r0 + (tid >> 4), a.rows - 1);
+    const TIN* qp = (const TIN*)a.q + (n0 + fr / (a.Tq * G)) * a.sq_n +
+                    (int64_t)(fr / G % a.Tq) * a.sq_t + (int64_t)(hk * G + fr % G) * a.sq_h;
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      const raw4 r = load4(qp, 16 * i + 4 * j);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) qf[i][e] = Elem<TIN>::to_f(r[e]);
+    for (int i = 0; i < NV; ++i) {
+      const int d = 64 * i + (tid & 15) * 4;
+      const raw4 r = load4(qp, d);
+      *(f32x4*)&qs[(tid >> 4) * LDO + d] = f32x4{Elem<TIN>::to_f(r[0]), Elem<TIN>::to_f(r[1]),
+                                                 Elem<TIN>::to_f(r[2]), Elem<TIN>::to_f(r[3])};
     }
   }
   raw4 kf[NQ], vf[4][NV];
+  // lane c's key of the step: its mask byte, loaded ahead with K (a load in the
+  // step itself would wait for every K and V load issued before it)
+  uint8_t mbyte = 1;
   auto load_k = [&](int s) {
+    if (a.mask && s < psteps) mbyte = a.mask[b * a.L + min(s * 16 + c, a.L - 1)];
     const TIN* p = kv_row(false, s, c);
 #pragma unroll
     for (int i = 0; i < NQ; ++i) kf[i] = load4(p, 16 * i + 4 * j);
@@ -498,6 +507,7 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
   float m = -INFINITY, l = 0.f;  // l: this lane's share of the row's sum
 
   if (wave < steps) load_k(wave);
+  __syncthreads();
   for (int s = wave; s < steps; s += 4) {
     // V of key 4 j + r, dims 64 i + 4 c + e
 #pragma unroll
@@ -508,11 +518,12 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
     }
     // which of this lane's 4 keys its row sees; hidden: nobody does
     bool seen[4], hidden[4];
+    const uint32_t visible =
+        (uint32_t)__ballot(s >= psteps || (s * 16 + c < a.L && mbyte != 0)) & 0xffffu;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       if (s < psteps) {
-        const int key = s * 16 + 4 * j + r;
-        seen[r] = key < a.L && !(a.mask && a.mask[b * a.L + key] == 0);
+        seen[r] = (visible >> (4 * j + r)) & 1;
         hidden[r] = !seen[r];
       } else if (a.by_token) {
         const int w = w_lo + 4 * j + r;
@@ -528,11 +539,13 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < NQ; ++i)
+    for (int i = 0; i < NQ; ++i) {
+      const f32x4 qf = *(const f32x4*)&qs[c * LDO + 16 * i + 4 * j];
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(Elem<TIN>::to_f(kf[i][e]), qf[i][e], acc[e],
-                                                      0, 0, 0);
+        acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(Elem<TIN>::to_f(kf[i][e]), qf[e], acc[e], 0,
+                                                      0, 0);
+    }
     if (s + 4 < steps) load_k(s + 4);
     float sc[4], mt = -INFINITY;
 #pragma unroll
@@ -542,16 +555,17 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
       mt = fmaxf(mt, sc[r]);
     }
     mt = max_xor32(max_xor16(mt));
-    const float mn = fmaxf(m, mt);
-    // rows that see a larger score: scale what they have
-    if (__any(mn != m)) {
-      const float alpha = mn == m ? 1.f : (m == -INFINITY ? 0.f : expf(m - mn));
+    // m is the row's reference, not its maximum: a row scales what it has only
+    // when a score exceeds m by 16 (weights up to e^16 lose nothing in fp32)
+    const bool raise = mt > m + 16.f;  // m = -inf: any score
+    if (__any(raise)) {
+      const float alpha = raise ? (m == -INFINITY ? 0.f : expf(m - mt)) : 1.f;
       l *= alpha;
 #pragma unroll
       for (int i = 0; i < NV * 4; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[i][r] *= alpha;
-      m = mn;
+      if (raise) m = mt;
     }
     float p[4];
 #pragma unroll
@@ -575,6 +589,7 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
           o[i * 4 + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(Elem<TIN>::to_f(vf[r][i][e]), p[r],
                                                               o[i * 4 + e], 0, 0, 0);
   }
+  __syncthreads();  // the query rows are read
   // o[4 i + e][r] is dim 64 i + 4 (4 j + r) + e of row c
   l = add_xor32(add_xor16(l));
   if (lane < 16) {
