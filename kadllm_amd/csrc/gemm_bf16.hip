@@ -1866,8 +1866,9 @@ int pick(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, void* 
       // half empty (64 rows 111 against 170 us, 128 rows 124 against 137)
       cfg = CFG_128x128_X16;
     else if (N <= 32)
-      // whole-K waves of 32 rows (the GDN gate projection at M = 32,768),
-      // else 64x32 tiles
+      // more rows than a 128-row ring tile a CU covers (32,768: 16.0 us there
+      // against 16.2 for whole-K waves): whole-K waves of 32 rows, one barrier
+      // in all; 64x32 tiles where K does not suit them
       cfg = n32_ok(A, lda, W, ldw, N, K, EPI) ? CFG_N32 : CFG_64x32;
     else if (tiles256 >= 256 && !vec)
       cfg = CFG_256x256_8W;
