@@ -15,7 +15,7 @@
 // gemm_bf16.hip; the epilogues round as theirs.  Measured with weights from
 // beyond the caches, us a call, the tile that gemm_bf16.hip picks against the
 // one it had: N 1,024, K 3,584: 10 rows 6.6 / 42, 100 rows 8.8 / 62, 400 rows
-// 13.3 / 65, 2,000 rows 25 / 66; N 8,192, K 1,024: 10 rows 6 / 19 (5.3 is what
+// 13.3 / 65, 2,000 rows 23 / 66; N 8,192, K 1,024: 10 rows 6 / 19 (5.3 is what
 // launching costs there), 100 rows 7.7 / 20.
 
 #include <type_traits>
@@ -61,7 +61,7 @@ template <int EPI, class RG>
 __global__ __launch_bounds__(64 * RG::NW) void gemm_ring_kernel(
     const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ Wt, int64_t ldw,
     bf16_t* C, int64_t ldc, const bf16_t* R, int64_t ldr, int M, int N, int K, int mtiles,
-    int vec) {
+    int ntiles, int group, int vec) {
   constexpr int BK = RG::BK, SLOTS = RG::SLOTS, NI = RG::NI, NJ = RG::NJ, NW = RG::NW;
   constexpr int CPR = BK / 8;  // 16-byte chunks per slice row
   constexpr int STEPS = BK / 32;
@@ -69,7 +69,14 @@ __global__ __launch_bounds__(64 * RG::NW) void gemm_ring_kernel(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / RG::WN, wn = wave % RG::WN;
   const int lid = xcd_logical_id(blockIdx.x, gridDim.x);
-  const int mt = lid % mtiles, nt = lid / mtiles;  // a column tile's rows share its W
+  // An XCD's run of tiles walks `group` column tiles a row tile at a time: one,
+  // so that the rows of few row tiles share their W, or eight, which keeps the
+  // run square where a column tile alone would read most of A into each L2
+  // (4,096 x 1,024 x 3,584 in 128x64 tiles: 69.4 us by columns, 43.9 by eights;
+  // 3,419 rows 56.0 and 42.6, 2,000 rows 25 and 23.2).
+  const int g0 = lid / (group * mtiles) * group, in_group = lid - g0 * mtiles;
+  const int gw = min(group, ntiles - g0);
+  const int mt = in_group / gw, nt = g0 + in_group % gw;
   const int m0 = mt * RG::BM;
 
   // Chunk c of slice row r is stored at chunk c ^ swizzle(r), so that the 16
@@ -218,14 +225,16 @@ __global__ __launch_bounds__(64 * RG::NW) void gemm_ring_kernel(
 template <int EPI, class RG>
 int launch(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
            const void* R, int64_t ldr, int M, int N, int K, hipStream_t s) {
-  const int64_t mtiles = kad_cdiv(M, RG::BM), blocks = mtiles * kad_cdiv(N, RG::BN);
+  const int64_t mtiles = kad_cdiv(M, RG::BM), ntiles = kad_cdiv(N, RG::BN);
+  const int64_t blocks = mtiles * ntiles;
   if (blocks > 0x7fffffff) KAD_UNSUPPORTED("gemm grid too large");
   const int n_out = EPI == KAD_EPI_SWIGLU ? N / 2 : N;
   const bool vec = n_out % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C % 8) == 0 &&
                    (EPI != KAD_EPI_RESIDUAL || (ldr % 4 == 0 && ((uintptr_t)R % 8) == 0));
   hipLaunchKernelGGL((gemm_ring_kernel<EPI, RG>), dim3((unsigned)blocks), dim3(64 * RG::NW), 0, s,
                      (const bf16_t*)A, lda, (const bf16_t*)W, ldw, (bf16_t*)C, ldc,
-                     (const bf16_t*)R, ldr, M, N, K, (int)mtiles, (int)vec);
+                     (const bf16_t*)R, ldr, M, N, K, (int)mtiles, (int)ntiles,
+                     mtiles > 8 ? 8 : 1, (int)vec);
   return kad_launch_status("gemm_ring_kernel");
 }
 

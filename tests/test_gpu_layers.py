@@ -368,6 +368,7 @@ def test_gemm_pipelined_tile_rejects_unaligned_output(device):
 @pytest.mark.parametrize("M,N,K", [
     (1, 64, 128), (15, 192, 256), (17, 1088, 384), (33, 320, 512), (65, 448, 640),
     (129, 64, 1152), (64, 128, 64), (130, 192, 320), (100, 1000, 896), (70, 30, 1152),
+    (1200, 1088, 128),   # more than 8 row tiles of every size, 17 = 8 + 8 + 1 column tiles
 ])
 def test_gemm_ring_tiles_agree(device, M, N, K, epi):
     """Configurations 32 .. 37 (K through a ring of LDS slots) and the automatic
