@@ -133,13 +133,7 @@ __device__ __forceinline__ void hf_l2_apply(u32x4& r, float rs) {
 }
 
 // ---------------------------------------------------------------------------
-// N16: T' and In as A fragments of 16x16x32 MFMAs (gdn_chunk_scan16) instead of
-// 32x32x16 ones: fragment f of the 6 is the 16 rows it16(f) against the 32 tokens
-// of step s16(f), lane L holding X[it*16 + L%16][s*32 + (t/4)*16 + (L/16)*4 + t%4].
-__host__ __device__ __forceinline__ constexpr int it16(int f) { return f < 2 ? f : 2 + (f - 2) / 2; }
-__host__ __device__ __forceinline__ constexpr int s16(int f) { return f < 2 ? 0 : (f - 2) % 2; }
-
-template <int K, bool HF, bool N16>
+template <int K, bool HF>
 __global__ __launch_bounds__(kPrepThreads) void gdn_chunk_prep(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, int64_t ld_qk,
     const void* __restrict__ g, int gdt, const void* __restrict__ beta, int bdt, int64_t ld_gate,
@@ -264,57 +258,13 @@ __global__ __launch_bounds__(kPrepThreads) void gdn_chunk_prep(
       const bf16x8 b = as_bf16x8(*(const u32x4*)(kb + (tj * 32 + fr) * LD + s * 16 + fk));
       const bf16x8 bq = as_bf16x8(*(const u32x4*)(qb + (ti * 32 + fr) * LD + s * 16 + fk));
       gram = mfma32x32x16(a, b, gram);
-      if constexpr (!N16) inT = mfma32x32x16(b, bq, inT);
-    }
-  }
-  // N16: In^T in 16 x 16 tiles, two (tokens s*32 and s*32 + 16) to a fragment,
-  // whose accumulators are the fragment's order; wave w forms fragments w, w + 4
-  f32x4 in16[2][2];
-  if constexpr (N16) {
-    const int c16 = lane & 15, k16 = (lane >> 4) * 8;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int f = min(wave + 4 * u, ChunkRec::frags - 1);
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int st = 0; st < K / 32; ++st) {
-          const bf16x8 a = as_bf16x8(*(const u32x4*)(
-              kb + (s16(f) * 32 + half * 16 + c16) * LD + st * 32 + k16));
-          const bf16x8 b =
-              as_bf16x8(*(const u32x4*)(qb + (it16(f) * 16 + c16) * LD + st * 32 + k16));
-          acc = mfma16x16x32(a, b, acc);
-        }
-        in16[u][half] = acc;
-      }
+      inT = mfma32x32x16(b, bq, inT);
     }
   }
   __syncthreads();  // rows no longer needed: the region becomes A / T'
   // In_ij = (q^_i . k^_j) qmul_i kmul_j e^{G_i - G_j} for j <= i, as hi/lo
   // A fragments (it = ti, s = tj * 2 + half) straight from the accumulators
-  if constexpr (N16) {
-    bf16_t* inf = (bf16_t*)(rec + ChunkRec::in);
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int f = wave + 4 * u;
-      if (f >= ChunkRec::frags) break;
-      const int irow = it16(f) * 16 + (lane & 15);
-      const float qmi = qmul[irow], gi = g2s[irow];
-      float x[8];
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int j = s16(f) * 32 + (t / 4) * 16 + (lane >> 4) * 4 + t % 4;
-        x[t] = j <= irow ? (in16[u][t / 4][t % 4] * qmi * kmul[j]) *
-                               __builtin_amdgcn_exp2f(gi - g2s[j])
-                         : 0.f;
-      }
-      bf16x8 ih, il;
-      split8(x, ih, il);
-      *(bf16x8*)(inf + ((f * 2 + 0) * 64 + lane) * 8) = ih;
-      *(bf16x8*)(inf + ((f * 2 + 1) * 64 + lane) * 8) = il;
-    }
-  } else if (wave < 3) {
+  if (wave < 3) {
     const int irow = ti * 32 + (lane & 31);
     const float qmi = qmul[irow], gi = g2s[irow];
 #pragma unroll
@@ -425,11 +375,10 @@ __global__ __launch_bounds__(kPrepThreads) void gdn_chunk_prep(
       if (fl_ >= ChunkRec::frags * 64) break;
       const int f = fl_ >> 6, L = fl_ & 63;
       const int it = f < 2 ? 0 : 1, s = f < 2 ? f : f - 2;
-      const int i = N16 ? it16(f) * 16 + (L & 15) : it * 32 + (L & 31);
-      const int jb = N16 ? s16(f) * 32 + (L >> 4) * 4 : s * 16 + (L >> 5) * 4;
+      const int i = it * 32 + (L & 31), jb = s * 16 + (L >> 5) * 4;
       float x[8];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) x[t] = Tm[i][jb + (t / 4) * (N16 ? 16 : 8) + t % 4];
+      for (int t = 0; t < 8; ++t) x[t] = Tm[i][jb + (t / 4) * 8 + t % 4];
       bf16x8 fh, fl;
       split8(x, fh, fl);
       *(bf16x8*)(tf + ((f * 2 + 0) * 64 + L) * 8) = fh;
@@ -825,18 +774,57 @@ __global__ __launch_bounds__(V * 2, V == 128 ? 2 : 1) void gdn_chunk_scan(
 }
 
 // The scan with 16 value columns per wave, 64 per workgroup, on 16x16x32 MFMAs:
-// half the MFMAs, splits and LDS reads a wave's chunk takes in gdn_chunk_scan.
-// A chunk is one dependent step, so where the (sequence, head) pairs leave the
-// chip idle the step's length is the whole time, and halving it over twice the
-// workgroups is worth reading q, k, T' and In twice: 4 x 16 heads of 1,000
-// tokens 111 -> 77 us (with the prep, 128.6 -> 95.3; loading a chunk ahead in
-// registers made either kernel 5% slower).
+// half the MFMA time and splits a wave's chunk takes in gdn_chunk_scan.  A chunk
+// is one dependent step, so where the (sequence, head) pairs leave the chip idle
+// the step's length is the whole time, and shortening it over twice the
+// workgroups is worth reading q, k, T' and In twice (times at launch_chunk).
 //
-// S[kt][e] is row kt*16 + 4 (lane/16) + e, column lane%16 of the wave's 16.
-// Every product's K runs in the order of the accumulators: slot t of lane group
-// j = lane/16 is entry (t/4)*16 + 4 j + t%4 of a 32-deep step, so that two 16-row
-// accumulator tiles are a B fragment as they stand.
+// Both scans give the same bits, so a sequence's results do not depend on how
+// many others come with it.  A 32-deep MFMA sums its first 16 slots and then the
+// other 16, as two 16-deep ones do, so each instruction here takes two of
+// gdn_chunk_scan's consecutive ones: mostly a step's hi plane against the lower
+// half of the lanes and its lo plane against the upper.  A 16x16 accumulator
+// tile holds rows 4 (lane/16) + e of its 16; a half-wave swap of two planes'
+// words puts the first plane, rows {0-3, 8-11 | 4-7, 12-15}, into the lower 32
+// lanes and the second into the upper, which is the slot order of acc_frags.
 constexpr int kCols16 = 64;
+
+// hi and lo planes of a lane's 4 accumulator entries
+struct Planes {
+  uint32_t hi[2], lo[2];
+};
+__device__ __forceinline__ Planes planes4(const f32x4& x) {
+  Planes p;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    p.hi[i] = pack_bf16x2(x[2 * i], x[2 * i + 1]);
+    p.lo[i] = pack_bf16x2(x[2 * i] - __uint_as_float(p.hi[i] << 16),
+                          x[2 * i + 1] - __uint_as_float(p.hi[i] & 0xffff0000u));
+  }
+  return p;
+}
+// B fragment of plane a in the lower half of the lanes and plane b in the upper
+__device__ __forceinline__ bf16x8 plane_pair(const uint32_t (&a)[2], const uint32_t (&b)[2]) {
+  const auto x = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+  const auto y = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+  return as_bf16x8(u32x4{x[0], y[0], x[1], y[1]});
+}
+
+// an A fragment of one step in the lower half of the lanes and of the next in the
+// upper -> each in both halves (both planes of a step meet the same A); half the
+// LDS reads of loading them so
+__device__ __forceinline__ void both_halves(const bf16x8& f, bf16x8 (&out)[2]) {
+  const u32x4 w = __builtin_bit_cast(u32x4, f);
+  u32x4 a, b;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const auto r = __builtin_amdgcn_permlane32_swap(w[i], w[i], false, false);
+    a[i] = r[0];
+    b[i] = r[1];
+  }
+  out[0] = as_bf16x8(a);
+  out[1] = as_bf16x8(b);
+}
 
 template <int K, int V, bool HF>
 __global__ __launch_bounds__(256, 2) void gdn_chunk_scan16(
@@ -844,7 +832,7 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk_scan16(
     const bf16_t* __restrict__ v, int64_t ld_v, const uint8_t* __restrict__ ws,
     const void* __restrict__ state0, int sdt, int beams_per_state, bf16_t* __restrict__ out,
     int64_t ld_out, float* __restrict__ final_state, int T, int H, int HV, int nchunks) {
-  constexpr int KT = K / 16, KS = K / 32, LDK = K + 8, LDV = kCols16 + 8, CPR = K / 8;
+  constexpr int KT = K / 16, LDK = K + 8, LDV = kCols16 + 8, CPR = K / 8;
   constexpr int NTH = 256, NVB = V / kCols16;
   __shared__ __attribute__((aligned(16))) bf16_t kb[kC * LDK];
   __shared__ __attribute__((aligned(16))) bf16_t qb[kC * LDK];
@@ -853,11 +841,13 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk_scan16(
   __shared__ __attribute__((aligned(16))) float sc[kScal][kC];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, j4 = (lane >> 4) * 4;
+  const int half = (lane >> 4) & 1, upper = lane >> 5;  // slot half, plane of a pair
   const int nh = blockIdx.x / NVB, v0 = (blockIdx.x % NVB) * kCols16;
   const int n = nh / HV, hv = nh % HV;
   const int h = hv / (HV / H);
   const int vcol = wave * 16 + c;  // column within the workgroup's 64
 
+  // S[kt][e] is row kt*16 + j4 + e, column vcol
   f32x4 S[KT];
 #pragma unroll
   for (int kt = 0; kt < KT; ++kt)
@@ -930,32 +920,28 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk_scan16(
     }
     __syncthreads();
 
-    // A fragment of rows `row` .. of a [token][feature] tile, step s
-    auto row_frag = [&](const bf16_t* tile, int row, int s) {
-      const bf16_t* p = tile + (row + c) * LDK + s * 32 + j4;
-      const u32x2 lo = *(const u32x2*)p, up = *(const u32x2*)(p + 16);
-      return as_bf16x8(u32x4{lo[0], lo[1], up[0], up[1]});
-    };
-    // B fragments (hi, lo) of two 16-row accumulator tiles
-    auto tile_frags = [&](const f32x4& a, const f32x4& b, bf16x8& hi, bf16x8& lo) {
-      const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-      split8(x, hi, lo);
-    };
-    // ---- k S and q S
+    // ---- k S and q S: a 16-deep step's hi and lo planes to an instruction
     f32x4 KS4[4], QS4[4];
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) KS4[tt] = QS4[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      bf16x8 sh, sl;
-      tile_frags(S[2 * s], S[2 * s + 1], sh, sl);
+    for (int kt = 0; kt < KT; kt += 2) {
+      bf16x8 s[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const Planes p = planes4(S[kt + u]);
+        s[u] = plane_pair(p.hi, p.lo);
+      }
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) {
-        const bf16x8 ak = row_frag(kb, tt * 16, s), aq = row_frag(qb, tt * 16, s);
-        KS4[tt] = mfma16x16x32(ak, sh, KS4[tt]);
-        KS4[tt] = mfma16x16x32(ak, sl, KS4[tt]);
-        QS4[tt] = mfma16x16x32(aq, sh, QS4[tt]);
-        QS4[tt] = mfma16x16x32(aq, sl, QS4[tt]);
+        bf16x8 ak[2], aq[2];
+        both_halves(perm_frag(kb + (tt * 16 + c) * LDK, (kt + upper) * 16, half), ak);
+        both_halves(perm_frag(qb + (tt * 16 + c) * LDK, (kt + upper) * 16, half), aq);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          KS4[tt] = mfma16x16x32(ak[u], s[u], KS4[tt]);
+          QS4[tt] = mfma16x16x32(aq[u], s[u], QS4[tt]);
+        }
       }
     }
     // ---- Z_j = beta_j v_j - ZK_j (k S)_j
@@ -968,52 +954,64 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk_scan16(
       for (int e = 0; e < 4; ++e)
         Z[tt][e] = fmaf(-zk[e], KS4[tt][e], bt[e] * bf2f(vb[(tt * 16 + j4 + e) * LDV + vcol]));
     }
-    // ---- v_new = Z + T' Z, then o = e^G q S + In v_new (fragment f: rows it16,
-    // tokens of step s16)
-    bf16x8 zh[2], zl[2], vh[2], vl[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) tile_frags(Z[2 * s], Z[2 * s + 1], zh[s], zl[s]);
-    auto product = [&](const bf16_t* frags, int f, const bf16x8& bh, const bf16x8& bl, f32x4 acc) {
-      const bf16x8 ah = *(const bf16x8*)(frags + ((f * 2 + 0) * 64 + lane) * 8);
-      const bf16x8 al = *(const bf16x8*)(frags + ((f * 2 + 1) * 64 + lane) * 8);
-      acc = mfma16x16x32(ah, bh, acc);
-      acc = mfma16x16x32(ah, bl, acc);
-      return mfma16x16x32(al, bh, acc);
+    // Products with the record's hi/lo A fragments, X x for the 64-token x whose
+    // planes are p: two 16-deep steps s, s + 1, three terms each, are the pairs
+    // hi_s (hi_s, lo_s), (lo_s, hi_s+1) (hi_s, hi_s+1), (hi_s+1, lo_s+1) (lo_s+1, hi_s+1).
+    struct Pairs {
+      bf16x8 b[3];
     };
-    f32x4 VN[4];
+    auto pairs = [&](const Planes& s0, const Planes& s1) {
+      return Pairs{{plane_pair(s0.hi, s0.lo), plane_pair(s0.hi, s1.hi),
+                    plane_pair(s1.lo, s1.hi)}};
+    };
+    // rows it*16 .. +15 of the fragments at `frags`, added to acc
+    auto product = [&](const bf16_t* frags, int it, const Pairs (&x)[2], f32x4 acc) {
+      // a fragment's 32 rows are lanes 0-15 | 16-31 of each half
+      const bf16_t* p = frags + (half * 32 + (it % 2) * 16 + c) * 8;
 #pragma unroll
-    for (int it = 0; it < 4; ++it) VN[it] = Z[it];
+      for (int u = 0; u < it / 2 + 1; ++u) {
+        const int f = frag_index(it / 2, 2 * u) * 2;  // planes f .. f + 3: hi, lo, hi, lo
+        acc = mfma16x16x32(*(const bf16x8*)(p + f * 512), x[u].b[0], acc);
+        acc = mfma16x16x32(*(const bf16x8*)(p + (f + 1 + upper) * 512), x[u].b[1], acc);
+        acc = mfma16x16x32(*(const bf16x8*)(p + (f + 2 + upper) * 512), x[u].b[2], acc);
+      }
+      return acc;
+    };
+    // ---- v_new = Z + T' Z, then o = e^G q S + In v_new
+    Pairs x[2];
 #pragma unroll
-    for (int f = 0; f < ChunkRec::frags; ++f)
-      VN[it16(f)] = product(tf, f, zh[s16(f)], zl[s16(f)], VN[it16(f)]);
+    for (int u = 0; u < 2; ++u) x[u] = pairs(planes4(Z[2 * u]), planes4(Z[2 * u + 1]));
+    Planes vn[4];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) tile_frags(VN[2 * s], VN[2 * s + 1], vh[s], vl[s]);
+    for (int it = 0; it < 4; ++it) vn[it] = planes4(product(tf, it, x, Z[it]));
+#pragma unroll
+    for (int u = 0; u < 2; ++u) x[u] = pairs(vn[2 * u], vn[2 * u + 1]);
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       const f32x4 eq = *(const f32x4*)&sc[S_EQ][it * 16 + j4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) QS4[it][e] *= eq[e];
+      QS4[it] = product(tf + ChunkRec::frag_elems, it, x, QS4[it]);
     }
-#pragma unroll
-    for (int f = 0; f < ChunkRec::frags; ++f)
-      QS4[it16(f)] = product(tf + ChunkRec::frag_elems, f, vh[s16(f)], vl[s16(f)], QS4[it16(f)]);
     __syncthreads();  // every wave has read the v tile, which takes the output
 #pragma unroll
     for (int it = 0; it < 4; ++it)
 #pragma unroll
       for (int e = 0; e < 4; ++e) vb[(it * 16 + j4 + e) * LDV + vcol] = f2bf(QS4[it][e]);
     // ---- S <- e^{G_last} S + sum_i (kmul_i e^{G_last - G_i}) k_i v_new_i^T
-    bf16x8 wh[2], wl[2];
+    bf16x8 w[4];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      f32x4 w[2];
+    for (int s = 0; s < 4; ++s) {
+      const f32x4 wu = *(const f32x4*)&sc[S_WU][s * 16 + j4];
+      f32x4 ws4;
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const f32x4 wu = *(const f32x4*)&sc[S_WU][(2 * s + u) * 16 + j4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) w[u][e] = VN[2 * s + u][e] * wu[e];
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t hw = vn[s].hi[e / 2], lw = vn[s].lo[e / 2];
+        ws4[e] = (__uint_as_float(e % 2 ? hw & 0xffff0000u : hw << 16) +
+                  __uint_as_float(e % 2 ? lw & 0xffff0000u : lw << 16)) * wu[e];
       }
-      tile_frags(w[0], w[1], wh[s], wl[s]);
+      const Planes p = planes4(ws4);
+      w[s] = plane_pair(p.hi, p.lo);
     }
     const float egl = sc[S_EG][kC - 1];
 #pragma unroll
@@ -1021,21 +1019,23 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk_scan16(
 #pragma unroll
       for (int e = 0; e < 4; ++e) S[kt][e] *= egl;
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        // k^T: lane 4 e + m of a 16-lane group addresses token e of its four,
-        // features 4 m .. +3 of the tile's 16 (see kt_frag)
+      for (int s = 0; s < 4; s += 2) {
+        // k^T of tokens (s + upper)*16 ..: lane 4 e + m of a 16-lane group
+        // addresses token e of its four, features 4 m .. +3 (see kt_frag)
         tr_v4s_t part[2];
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-          const bf16_t* p = kb + (s * 32 + r * 16 + j4 + (c >> 2)) * LDK + kt * 16 + (c & 3) * 4;
+          const bf16_t* p = kb + ((s + upper) * 16 + r * 8 + half * 4 + (c >> 2)) * LDK + kt * 16 +
+                            (c & 3) * 4;
           part[r] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
               (__attribute__((address_space(3))) tr_v4s_t*)p);
         }
         const u32x2 lo = __builtin_bit_cast(u32x2, part[0]);
         const u32x2 up = __builtin_bit_cast(u32x2, part[1]);
-        const bf16x8 a = as_bf16x8(u32x4{lo[0], lo[1], up[0], up[1]});
-        S[kt] = mfma16x16x32(a, wh[s], S[kt]);
-        S[kt] = mfma16x16x32(a, wl[s], S[kt]);
+        bf16x8 a[2];
+        both_halves(as_bf16x8(u32x4{lo[0], lo[1], up[0], up[1]}), a);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) S[kt] = mfma16x16x32(a[u], w[s + u], S[kt]);
       }
     }
     __syncthreads();
@@ -1069,7 +1069,7 @@ int launch_chunk(const void* q, const void* k, const void* v, int64_t ld_qk, int
   // transformers' bf16 l2norm rounding (hf_norm) or the operator's fp32
   // scales: an instantiation each, so the VALU-bound loops carry no test
 #define KAD_CHUNK(HFV, GV)                                                                     \
-  hipLaunchKernelGGL((gdn_chunk_prep<K, HFV, false>), dim3((unsigned)nrec), dim3(kPrepThreads), 0, s, \
+  hipLaunchKernelGGL((gdn_chunk_prep<K, HFV>), dim3((unsigned)nrec), dim3(kPrepThreads), 0, s, \
                      (const bf16_t*)q, (const bf16_t*)k, ld_qk, g, gdt, beta, bdt, ld_gate,    \
                      (uint8_t*)ws, T, H, HV, nchunks, scale);                                  \
   if (const int rc = kad_launch_status("gdn_chunk_prep")) return rc;                           \
@@ -1079,9 +1079,9 @@ int launch_chunk(const void* q, const void* k, const void* v, int64_t ld_qk, int
                      (bf16_t*)out, ld_out, fin, T, H, HV, nchunks, ga);                        \
   return kad_launch_status("gdn_chunk_scan")
 #define KAD_CHUNK16(HFV)                                                                       \
-  hipLaunchKernelGGL((gdn_chunk_prep<K, HFV, true>), dim3((unsigned)nrec), dim3(kPrepThreads), \
-                     0, s, (const bf16_t*)q, (const bf16_t*)k, ld_qk, g, gdt, beta, bdt,       \
-                     ld_gate, (uint8_t*)ws, T, H, HV, nchunks, scale);                         \
+  hipLaunchKernelGGL((gdn_chunk_prep<K, HFV>), dim3((unsigned)nrec), dim3(kPrepThreads), 0, s, \
+                     (const bf16_t*)q, (const bf16_t*)k, ld_qk, g, gdt, beta, bdt, ld_gate,    \
+                     (uint8_t*)ws, T, H, HV, nchunks, scale);                                  \
   if (const int rc = kad_launch_status("gdn_chunk_prep")) return rc;                           \
   hipLaunchKernelGGL((gdn_chunk_scan16<K, V, HFV>),                                            \
                      dim3((unsigned)((int64_t)N * HV * (V / kCols16))), dim3(256), 0, s,       \
@@ -1089,10 +1089,11 @@ int launch_chunk(const void* q, const void* k, const void* v, int64_t ld_qk, int
                      (const uint8_t*)ws, state0, sdt, bps, (bf16_t*)out, ld_out, fin, T, H,    \
                      HV, nchunks);                                                             \
   if (const int rc = kad_launch_status("gdn_chunk_scan16")) return rc
-  // 64-column workgroups up to two per CU, where both kernels then hold as many:
-  // 16 sequences x 16 heads of 1,024 tokens 195 us in workgroups of all 128
-  // columns, 178 in two of 64; 24 (three per CU) 140 and 145
-  if ((int64_t)N * HV * (V / kCols16) <= 512) {
+  // 64-column workgroups while they number at most one per CU, of 64-wide heads
+  // two (16 heads of 1,024 tokens, us with the prep, wide scan against this one:
+  // 128-wide 1 sequence 120 / 100, 4 128 / 109, 8 146 / 129, 12 170 / 180;
+  // 64-wide 16 189 / 162, 32 of 300 tokens 100 / 90)
+  if ((int64_t)N * HV * (V / kCols16) <= (V == 64 ? 512 : 256)) {
     if (hf_norm) {
       KAD_CHUNK16(true);
     } else {

@@ -250,6 +250,39 @@ def test_chunk_scans_match_oracle(device, N, HV, K, V, T):
     assert torch.equal(y, normed) and torch.equal(f2, f)
 
 
+@pytest.mark.parametrize("K,V,T", [(128, 128, 1), (128, 128, 200), (64, 128, 70), (128, 64, 64),
+                                   (64, 64, 129)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_chunk_bits_do_not_depend_on_the_batch(device, K, V, T, gated):
+    """A sequence's outputs and state among a few, which take the 16-column scan,
+    and among as many as take the wide one (more than 512 64-column workgroups):
+    the same bits, with and without an initial state."""
+    H, HV, few = 2, 4, 3
+    N = 512 * 64 // (HV * V) + 1
+    q, k, v, g, beta, S = (t.to(device) for t in gdn_inputs(N, 1, T, H, HV, K, V, seed=T + K,
+                                                            state_std=0.1))
+    z = torch.randn(N * T, HV * V, generator=torch.Generator().manual_seed(T)).bfloat16().to(device)
+    w = torch.linspace(0.5, 1.5, V).bfloat16().to(device)
+
+    def run(n, state):
+        ws = _lib.gdn_chunk_workspace(n, T, HV, K, device)
+        o = torch.empty(n, T, HV, V, dtype=torch.bfloat16, device=device)
+        f = torch.empty(n, HV, K, V, device=device)
+        args = (*map(_lib.ptr, (q, k, v)), H * K, HV * V, 0, _lib.ptr(g), 2, _lib.ptr(beta), 0, HV,
+                _lib.ptr(state), 2, 1, _lib.ptr(o), HV * V, _lib.ptr(f), _lib.ptr(ws), ws.numel(),
+                n, T, H, HV, K, V, float(K ** -0.5))
+        if gated:
+            _lib.call("kad_gdn_chunk_gated", *args, _lib.ptr(z), HV * V, _lib.ptr(w), 1e-6,
+                      _lib.stream_of(o))
+        else:
+            _lib.call("kad_gdn_chunk", *args, 0, _lib.stream_of(o))
+        return o, f
+
+    for state in (None, S):
+        (o, f), (oa, fa) = run(few, state), run(N, state)
+        assert torch.equal(o, oa[:few]) and torch.equal(f, fa[:few])
+
+
 @pytest.mark.parametrize("L", [1, 3, 50])
 def test_conv_prefill_and_state(device, L):
     B, C = 2, 64
