@@ -451,6 +451,14 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
       }
       if (any) u[i] = order_of(best);
     }
+    if (tid == 0 && head > 0) {
+      // the columns before the first word enter the maximum: it may be theirs
+      float v[VE];
+      bool ok[VE];
+      load(head - VE, v, ok);
+#pragma unroll
+      for (int e = 0; e < VE; ++e) smax = fmaxf(smax, v[e]);
+    }
     smax = wave_max(smax);
     if (lane == 0) red_smax[tid >> 6] = smax;
     __syncthreads();
@@ -473,7 +481,8 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
   // ---- 2. max, sum exp, and candidates >= thr in one pass.  The sum is taken
   // against a fixed reference, the sample max (each term one fma and the
   // hardware exp2: exp(v - m) = 2^(v log2 e - m log2 e)); a row whose true max
-  // exceeds it by more than 60 sums again against the true max.
+  // lies more than 60 above it, or below (0 stands for a sample of -inf alone),
+  // sums again against the true max.
   constexpr float kLog2e = 1.4426950408889634f;
   float mref = -INFINITY;
   for (int w = 0; w < NT / 64; ++w) mref = fmaxf(mref, red_smax[w]);
@@ -543,8 +552,7 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
   for (int w = 0; w < NT / 64; ++w) M = fmaxf(M, red_m[w]);
   float SE = 0.f;
   for (int w = 0; w < NT / 64; ++w) SE += red_s[w];
-  if (M > mref + 60.f) {
-    // the sample missed the top by far: sum again against the true max
+  if (M > mref + 60.f || (M < mref - 60.f && M > -INFINITY)) {
     __syncthreads();
     mref = M;
     nb = -mref * kLog2e;

@@ -228,6 +228,36 @@ def test_select_rows_of_any_length(device, dtype, B, Wp, V, width, masked):
     assert_selection_gap_aware(s, p, t, keys, width, 1e-5, name="rows")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("V,where", [(1001, "head"), (60001, "unsampled")])
+def test_select_rows_whose_sample_holds_no_finite_logit(device, dtype, V, where):
+    """Rows whose finite logits, near -120, are all in the columns before the
+    row's first 16-byte boundary, or in lines the sample leaves out (with as many
+    allowed -inf ones in it): the sum's reference is 0 there, against which every
+    term underflows.  Scores 1e-5 from the 64-bit log-softmax."""
+    g = torch.Generator().manual_seed(V)
+    Wp, W = 4, 3
+    logits = torch.full((1, Wp, V), -float("inf"))
+    finite = torch.zeros(V, dtype=torch.bool)
+    allowed = torch.zeros(V, dtype=torch.bool)
+    if where == "head":
+        finite[:3] = True
+        allowed[:] = True
+    else:
+        finite[100:300] = True      # lines 2 .. 4 of every 7
+        allowed = finite.clone()
+        allowed[64 * 7 * torch.arange(1, 121) + 20] = True
+    logits[0, :, finite] = -120 + torch.randn(Wp, int(finite.sum()), generator=g)
+    logits = logits.to(dtype)
+    scores = -torch.rand(1, Wp, generator=g)
+    mask = allowed.expand(1, Wp, V)
+    s, p, t, valid = select_level(logits.to(device), scores.to(device), W, mask.to(device))
+    keys = (logits.double().log_softmax(-1) + scores.double()[..., None])
+    keys = keys.masked_fill(~mask, -float("inf"))
+    assert bool(valid.all())
+    assert_selection_gap_aware(s, p, t, keys, W, 1e-5, name="rows")
+
+
 def test_select_float_rows_with_equal_keys_take_lower_columns(device):
     """fp32 logits that differ by less than their keys' precision tie, and the
     lower columns of all of them are taken, sampled or not."""
