@@ -28,6 +28,7 @@
 #include "kad_common.h"
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <mutex>
 
@@ -330,6 +331,18 @@ __device__ void row_select_exact_float(
 }
 
 
+// e^d for d <= 0 (a NaN stays one) to 1.5 ulp: 2^(d log2 e) by the hardware, and
+// what the rounded product d log2 e lacks as the factor 1 + r ln 2
+__device__ __forceinline__ float exp_of(float d) {
+  constexpr float kL = 1.44269502162933349609375f, kLLow = 1.92596303e-8f;  // log2 e
+  constexpr float kLn2 = 0.693147182f;
+  d = d < -200.f ? -200.f : d;  // also -inf, whose r would be NaN
+  const float t = d * kL;
+  const float r = fmaf(d, kLLow, fmaf(d, kL, -t));
+  const float e = __builtin_amdgcn_exp2f(t);
+  return fmaf(e, r * kLn2, e);
+}
+
 // inverse of order32
 __device__ __forceinline__ float unorder32(uint32_t u) {
   return __uint_as_float((u & 0x80000000u) ? u ^ 0x80000000u : ~u);
@@ -354,7 +367,7 @@ __device__ __forceinline__ float unorder32(uint32_t u) {
 // NT: 1,024 threads where the rows number at most two per CU (one row on a CU
 // is bound by the loads its waves keep in flight: 8 rows of 248,320 bf16
 // logits 96 -> 35 us), else 256 (2,048 rows 272 -> 246 us, 4.1 TB/s; of fp32, by
-// six passes before, 7.3 ms -> 0.43).
+// six passes before, 7.3 ms -> 0.40).
 template <typename T, int CAP, bool MASKED, int NT>
 __global__ __launch_bounds__(NT) void row_select_kernel(
     const T* __restrict__ logits, int64_t ld, const uint8_t* __restrict__ mask, int64_t ld_mask,
@@ -478,28 +491,46 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
   // order key 0 (too few allowed samples): the exact path below
   const float tf = whole ? -INFINITY : (thr ? value_of(thr) : INFINITY);
 
-  // ---- 2. max, sum exp, and candidates >= thr in one pass.  The sum is taken
-  // against a fixed reference, the sample max (each term one fma and the
-  // hardware exp2: exp(v - m) = 2^(v log2 e - m log2 e)); a row whose true max
-  // lies more than 60 above it, or below (0 stands for a sample of -inf alone),
-  // sums again against the true max.
+  // ---- 2. max, sum exp, and candidates >= thr in one pass.  The sum of a bf16
+  // row is taken against a fixed reference, the sample max (each term one fma
+  // and the hardware exp2: exp(v - m) = 2^(v log2 e - m log2 e)); a row whose
+  // true max lies more than 60 above it, or below (0 stands for a sample of
+  // -inf alone), sums again against the true max.  fp32 and fp16 rows, whose
+  // scores keep what the sum loses, take exact differences to a reference that
+  // each thread raises to its own largest logit, and their keys from the row's
+  // max: as bf16 rows do, a score errs by 1.4e-5 under a peak of 60 that the
+  // sample misses, so by 1.9e-6, its last rounding (2,048 rows of 248,320 fp32
+  // logits 380 -> 404 us, fp16 238 -> 293; 8 rows 36 -> 50).
   constexpr float kLog2e = 1.4426950408889634f;
   float mref = -INFINITY;
   for (int w = 0; w < NT / 64; ++w) mref = fmaxf(mref, red_smax[w]);
+  float ref = fmaxf(mref, -FLT_MAX);  // fp32, fp16: at least the thread's largest logit
   if (mref == -INFINITY) mref = 0.f;
   float m = -INFINITY, se = 0.f;
   float nb = -mref * kLog2e;
-  // fp32 and fp16 terms from the exact difference, an instruction more
   auto term = [&](float v) {
-    return __builtin_amdgcn_exp2f(kBf16 ? fmaf(v, kLog2e, nb) : (v - mref) * kLog2e);
+    if constexpr (kBf16) return __builtin_amdgcn_exp2f(fmaf(v, kLog2e, nb));
+    else return exp_of(v - ref);
   };
   auto visit = [&](int c, const float (&v)[VE], const bool (&ok)[VE]) {
     float mx = v[0];
 #pragma unroll
     for (int e = 1; e < VE; ++e) mx = fmaxf(mx, v[e]);
     m = fmaxf(m, mx);
+    if constexpr (!kBf16)
+      if (mx > ref) {
+        se *= expf(ref - mx);
+        ref = mx;
+      }
+    if constexpr (kBf16) {
 #pragma unroll
-    for (int e = 0; e < VE; ++e) se += term(v[e]);
+      for (int e = 0; e < VE; ++e) se += term(v[e]);
+    } else {
+      float s = 0.f;  // beside a peak's 1, single terms would be lost
+#pragma unroll
+      for (int e = 0; e < VE; ++e) s += term(v[e]);
+      se += s;
+    }
     if (mx >= tf) {
 #pragma unroll
       for (int e = 0; e < VE; ++e)
@@ -540,34 +571,36 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
     }
   }
   for (; c0 < V; c0 += kStep) visit_at(c0);
-  {
-    const float mm = wave_max(m), ss = wave_sum(se);
-    if (lane == 0) {
-      red_m[tid >> 6] = mm;
-      red_s[tid >> 6] = ss;
-    }
-  }
+  auto block_sum = [&](float x) {
+    x = wave_sum(x);
+    if (lane == 0) red_s[tid >> 6] = x;
+    __syncthreads();
+    float s = 0.f;
+    for (int w = 0; w < NT / 64; ++w) s += red_s[w];
+    return s;
+  };
+  m = wave_max(m);
+  if (lane == 0) red_m[tid >> 6] = m;
   __syncthreads();
   float M = -INFINITY;
   for (int w = 0; w < NT / 64; ++w) M = fmaxf(M, red_m[w]);
-  float SE = 0.f;
-  for (int w = 0; w < NT / 64; ++w) SE += red_s[w];
-  if (M > mref + 60.f || (M < mref - 60.f && M > -INFINITY)) {
-    __syncthreads();
-    mref = M;
-    nb = -mref * kLog2e;
-    float s2 = 0.f;
-    for (int c = tid; c < V; c += NT) s2 += term(Elem<T>::to_f(x[c]));
-    s2 = wave_sum(s2);
-    if (lane == 0) red_s[tid >> 6] = s2;
-    __syncthreads();
-    SE = 0.f;
-    for (int w = 0; w < NT / 64; ++w) SE += red_s[w];
+  float lse;
+  if constexpr (kBf16) {
+    float SE = block_sum(se);
+    if (M > mref + 60.f || (M < mref - 60.f && M > -INFINITY)) {
+      __syncthreads();
+      mref = M;
+      nb = -mref * kLog2e;
+      float s2 = 0.f;
+      for (int c = tid; c < V; c += NT) s2 += term(Elem<T>::to_f(x[c]));
+      SE = block_sum(s2);
+    }
+    // log sum exp(v - M) = log(sum exp(v - mref)) + (mref - M)
+    lse = logf(SE) + (mref - M);
+  } else {
+    // a thread without a term keeps 0, also where its reference is no logit
+    lse = logf(block_sum(se == 0.f ? 0.f : se * expf(ref - M)));
   }
-  // bf16: log sum exp(v - M) = log(sum exp(v - mref)) + (mref - M); fp32 and fp16
-  // keys are taken from mref, a rounding less
-  if constexpr (!kBf16) M = mref;
-  const float lse = logf(SE) + (mref - M);
   const int count = sh_count;
   const float p = parent[row];
   auto exact = [&] {

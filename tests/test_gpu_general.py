@@ -258,6 +258,29 @@ def test_select_rows_whose_sample_holds_no_finite_logit(device, dtype, V, where)
     assert_selection_gap_aware(s, p, t, keys, W, 1e-5, name="rows")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("peak", [18.0, 30.0, 60.0])
+def test_select_float_scores_under_a_peak_outside_the_sample(device, dtype, peak):
+    """A confident model's rows: Gaussian logits and one far above them, in a line
+    the sample leaves out.  The peak's key is -lse alone: its thread adds some 60
+    words' sums to 1, half an ulp each in either direction (worst case 30 ulps,
+    sqrt(60) / 2 expected, twice that allowed); the others' keys are three
+    roundings more, half an ulp each."""
+    Wp, V, W = 8, 248320, 24
+    logits = torch.randn(1, Wp, V, generator=torch.Generator().manual_seed(int(peak)))
+    logits[0, torch.arange(Wp), 70 + 3 * torch.arange(Wp)] = peak
+    logits = logits.to(dtype)
+    s, p, t, valid = select_level(logits.to(device), torch.zeros(1, Wp, device=device), W)
+    keys = logits.double().log_softmax(-1)
+    true = keys[0, p[0].cpu(), t[0].cpu()]
+    err = (s[0].double().cpu() - true).abs()
+    top = t[0].cpu() == 70 + 3 * p[0].cpu()
+    assert int(top.sum()) == Wp and bool(valid.all())
+    ulp = 2.0 ** (true.abs().clamp_min(1.0).log2().floor() - 23)
+    assert bool((err[top] <= 8 * 2.0 ** -23).all()), err[top]
+    assert bool((err[~top] <= 1.5 * ulp[~top] + 8 * 2.0 ** -23).all()), err[~top]
+
+
 def test_select_float_rows_with_equal_keys_take_lower_columns(device):
     """fp32 logits that differ by less than their keys' precision tie, and the
     lower columns of all of them are taken, sampled or not."""
