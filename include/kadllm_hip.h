@@ -528,9 +528,11 @@ int kad_cache_prefetch(const void* p0, int64_t bytes0, const void* p1, int64_t b
  *   [B*Wp, T-1, kv_heads, head_dim]); next0/1 written with keep.  prefix[i]: a
  *   linear layer's conv state (p0, strides s0..s2, history slots) and state
  *   (p1, dtype); an attention layer's K, V (p0, p1, strides of [B, L, heads],
- *   history = L).  Scratch as above over B*W rows, rows_ws [B*W, gdn_cols],
- *   qkv [B*W, qkv columns], k_ws and v_ws [B*W, T, kv_heads, head_dim], ab
- *   [B*W*T, ab_rows], g and beta [B*W*T, v_heads]. */
+ *   history = L).  Scratch as above over B*W rows, rows_ws [B*W, gdn_cols]
+ *   ([B*W*T, gdn_cols] where T = 2, nothing is kept and ab_rows % 8 != 0: the
+ *   earlier rows are gathered then), qkv [B*W, qkv columns], k_ws and v_ws
+ *   [B*W, T, kv_heads, head_dim], ab [B*W*T, ab_rows], g and beta
+ *   [B*W*T, v_heads]. */
 typedef struct {
   int linear; /* 1: gated delta layer, 0: attention */
   const void *input_norm, *post_norm, *w_gu, *w_down;

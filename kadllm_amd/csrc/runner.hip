@@ -134,9 +134,9 @@ extern "C" int kad_qwen_decode_step(const kad_qwen_model* m, const kad_qwen_step
       KAD_TRY(kad_cache_prefetch(l.w_qkv, (int64_t)(2 * nh + 2 * nkv) * hd * H * 2, nullptr, 0, s));
     KAD_TRY(kad_rmsnorm(a->x, H, l.input_norm, 1.f, a->n, H, BW, H, m->eps, s));
     if (l.linear) {
-      if (T == 2 && !a->keep) {
+      if (T == 2 && !a->keep && nab % 8 == 0) {
         // the earlier token's rows in place in the parents' cache: only its
-        // gate inputs are gathered
+        // gate inputs are gathered, in whole 16-byte pieces
         KAD_TRY(follow(at(a->prev0[i], c), (int64_t)cols * 2, a->ab, nab * 2, nab * 2));
         KAD_TRY(store(a->n, H, l.w_ab, at(a->ab, (T - 1) * nab), T * nab, BW, nab, H, s));
         KAD_TRY(store(a->n, H, l.w_in, a->rows_ws, cols, BW, c, H, s));

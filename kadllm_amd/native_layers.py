@@ -179,7 +179,10 @@ class NativeLayers:
         at = [None if p is None else ctypes.addressof(p) for pair in arrays for p in pair]
         n, h = empty(BW, cfg.hidden_size), empty(BW, self.ffn)
         mixed, q = empty(BW, max(runner.vd, self.att_cols)), empty(BW, self.att_cols)
-        qkv, rows_ws = empty(BW, self.qkv_cols), empty(BW, cols)
+        # a last level reads the earlier token's rows in its parents' cache where
+        # the gate inputs are whole 16-byte pieces, else gathers all T of a beam
+        parent_rows = T == 1 or keep or self.ab_rows % 8 == 0
+        qkv, rows_ws = empty(BW, self.qkv_cols), empty(BW * (1 if parent_rows else T), cols)
         k_ws, v_ws = (None, None) if keep else (empty(BW, T, nkv, hd), empty(BW, T, nkv, hd))
         ab, beta = empty(BW * T, self.ab_rows), empty(BW * T, HV)
         g = empty(BW * T, HV, dtype=torch.float32)

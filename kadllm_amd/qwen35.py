@@ -291,14 +291,16 @@ class Qwen35Runner:
                       dk, dv, float(dk ** -0.5), _lib.stream_of(conv))
 
     def _mixer_fusable(self, lyr):
-        """Whether the fused decode mixer takes this layer's shapes (besides
-        the suffix length and row alignment, checked where it is called)."""
+        """Whether the fused decode mixer with the parents' rows in place takes
+        this layer's shapes (besides the suffix length and row alignment, checked
+        where it is called): the gathered gate inputs are rows of 4 HV bytes, of
+        which kad_gather_beam_rows takes multiples of 16."""
         cfg = self.cfg
         return (cfg.linear_key_head_dim == 128
                 and cfg.linear_value_head_dim == 128 and self.gdn_cols % 8 == 0
                 and lyr.conv_w.is_contiguous() and lyr.conv_w.data_ptr() % 8 == 0
                 and lyr.norm_w.data_ptr() % 8 == 0
-                and cfg.linear_num_value_heads % 2 == 0)
+                and cfg.linear_num_value_heads % 4 == 0)
 
     def _gdn_mix_parents(self, lyr, n, prev, parents, cached, B, W, Wp, T):
         """_gdn_mix for the search's last level (last token only, T = 2) with

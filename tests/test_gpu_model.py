@@ -685,3 +685,38 @@ def test_layers_in_one_call_equal_the_steps(device, last, B, L, W):
         for a, b in zip(passes(ad), steps):
             assert torch.equal(a, b)
     assert adapter._runner._native is not None
+
+
+@pytest.mark.parametrize("HV", [2, 6, 4])
+@pytest.mark.parametrize("W", [10, 16])
+def test_last_level_of_any_value_head_count(device, HV, W):
+    """A last level (no cache kept) whose gate rows, 4 HV bytes, are no whole
+    16-byte pieces: the logits of the level that keeps its cache and of the whole
+    suffix, as one call and step by step."""
+    from dataclasses import replace
+
+    from kadllm_amd import _lib
+    B, L = 2, 9
+    cfg = replace(tiny_hybrid_config(), linear_num_key_heads=2, linear_num_value_heads=HV,
+                  linear_key_head_dim=128, linear_value_head_dim=128)
+    adapter = Qwen35GRBeamAdapter(*native_model(cfg, random_state_dict(
+        cfg, seed=5, dtype=torch.bfloat16, device=device)))
+    g = torch.Generator().manual_seed(HV * W)
+
+    def ints(high, *shape):
+        return torch.randint(0, high, shape, generator=g).to(device)
+
+    ids, first = ints(cfg.vocab_size, B, L), ints(cfg.vocab_size, B, W, 1)
+    parents, token = ints(W, B, W), ints(cfg.vocab_size, B, W, 1)
+    second = torch.cat((first.gather(1, parents[..., None]), token), 2)
+    for hook in (None, lambda name, args, launch: launch()):
+        _lib.set_call_hook(hook)
+        try:
+            state = adapter.prefill(ids).state
+            _, cache = adapter.decode_incremental(first, None, state, None)
+            kept, _ = adapter.decode_incremental(second, parents, state, cache)
+            last, _ = adapter.decode_incremental(second, parents, state, cache, keep_cache=False)
+            whole = adapter.decode(second, state)
+        finally:
+            _lib.set_call_hook(None)
+        assert torch.equal(last, kept) and torch.equal(last, whole)
