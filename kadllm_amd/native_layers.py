@@ -5,6 +5,7 @@ loops, which run where a trace or a call hook wants every step, and for the
 shapes outside ``step_fits``."""
 
 import ctypes
+import operator
 
 import torch
 
@@ -48,6 +49,20 @@ def _pointers(tensors):
     return (_P * len(tensors))(*[None if t is None else t.data_ptr() for t in tensors])
 
 
+_COMMON = ("input_norm", "post_norm", "w_gu", "w_down")
+_LINEAR = _COMMON + ("w_in", "w_ab", "conv_w", "A_log", "dt_bias", "norm_w", "w_out")
+_ATTENTION = _COMMON + ("w_qkv", "q_norm", "k_norm", "w_o")
+_get_linear, _get_attention = operator.attrgetter(*_LINEAR), operator.attrgetter(*_ATTENTION)
+
+
+def _weights(runner):
+    """Every tensor whose address kad_qwen_model holds."""
+    out = [runner.inv_freq]
+    for lyr in runner.layers:
+        out += _get_linear(lyr) if hasattr(lyr, "w_in") else _get_attention(lyr)
+    return out
+
+
 class NativeLayers:
     """The packed weights of a Qwen35Runner as kad_qwen_model, and its passes."""
 
@@ -58,10 +73,14 @@ class NativeLayers:
         for dst, src in zip(layers, runner.layers):
             dst.linear = int(hasattr(src, "w_in"))
             self.linear.append(bool(dst.linear))
-            for name, _ in _Layer._fields_[1:]:
-                if hasattr(src, name):
-                    setattr(dst, name, getattr(src, name).data_ptr())
-        self._keep = (layers, runner.inv_freq, runner.layers)
+            for name in _LINEAR if dst.linear else _ATTENTION:
+                setattr(dst, name, getattr(src, name).data_ptr())
+        # the tensors are held, so that no address outlives its memory
+        self._layers, self._tensors = layers, _weights(runner)
+        self._addresses = list(map(torch.Tensor.data_ptr, self._tensors))
+        # the passes name no strides and no types
+        self.plain = all(t.is_contiguous() and t.dtype == (
+            torch.float32 if t is runner.inv_freq else torch.bfloat16) for t in self._tensors)
         self.ab_rows = 2 * cfg.linear_num_value_heads
         self.ffn = runner.layers[0].w_down.shape[1]
         # one width throughout (the padded packing of every layer's MLP)
@@ -83,6 +102,15 @@ class NativeLayers:
             and all(lyr.conv_w.is_contiguous() and lyr.conv_w.data_ptr() % 8 == 0
                     and lyr.norm_w.data_ptr() % 8 == 0
                     for lyr, lin in zip(runner.layers, self.linear) if lin))
+
+    def describes(self, runner):
+        """Whether the runner's weights are still the tensors, at the addresses,
+        that the struct was built from (a layer's may be rebound or its storage
+        replaced): 25 us for 24 layers."""
+        now = _weights(runner)
+        return (len(now) == len(self._tensors)
+                and all(map(operator.is_, now, self._tensors))
+                and list(map(torch.Tensor.data_ptr, now)) == self._addresses)
 
     def _call(self, name, args, x):
         _lib.call(name, ctypes.addressof(self.model), ctypes.addressof(args), _lib.stream_of(x))

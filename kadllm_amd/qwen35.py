@@ -196,12 +196,13 @@ class Qwen35Runner:
 
     def _native_layers(self):
         """The layers' one-call form, or None while something watches the
-        single steps (a trace, a call hook)."""
+        single steps (a trace, a call hook) and for weights it does not take."""
         if self.trace is not None or _lib.hooked():
             return None
-        if self._native is None:
-            self._native = NativeLayers(self)
-        return self._native
+        native = self._native
+        if native is None or not native.describes(self):
+            native = self._native = NativeLayers(self)
+        return native if native.plain else None
 
     # ------------------------------------------------------------------
     def _mlp(self, lyr, x, rows, prefetch=False):

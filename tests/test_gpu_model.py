@@ -720,3 +720,44 @@ def test_last_level_of_any_value_head_count(device, HV, W):
         finally:
             _lib.set_call_hook(None)
         assert torch.equal(last, kept) and torch.equal(last, whole)
+
+
+@pytest.mark.parametrize("how", ["rebound", "storage", "strided"])
+def test_layers_in_one_call_follow_replaced_weights(device, how):
+    """Weights of a layer replaced after a pass -- the attribute rebound, the
+    tensor's storage exchanged, a tensor with strides of its own -- are those the
+    next passes run with, as the single steps do."""
+    from kadllm_amd import _lib
+    cfg = tiny_hybrid_config()
+    adapter = Qwen35GRBeamAdapter(*native_model(cfg, random_state_dict(
+        cfg, seed=6, dtype=torch.bfloat16, device=device)))
+    g = torch.Generator().manual_seed(6)
+    ids = torch.randint(0, cfg.vocab_size, (2, 20), generator=g).to(device)
+    tok = torch.randint(0, cfg.vocab_size, (2, 6, 1), generator=g).to(device)
+
+    def logits():
+        pre = adapter.prefill(ids)
+        return pre.logits, adapter.decode_incremental(tok, None, pre.state, None)[0]
+
+    before = logits()
+    held = []                     # the old memory stays allocated throughout
+    for lyr in (adapter._runner.layers[1], adapter._runner.layers[3]):
+        for name in ("w_down", "post_norm"):
+            old = getattr(lyr, name)
+            new = old.flip(0).contiguous() * 0.5
+            held.append(old if how != "storage" else old.data)
+            if how == "storage":
+                old.data = new
+            elif how == "strided" and old.ndim == 2:
+                wide = torch.zeros(old.shape[0], old.shape[1] + 64, dtype=old.dtype, device=device)
+                setattr(lyr, name, wide[:, :old.shape[1]].copy_(new))
+            else:
+                setattr(lyr, name, new)
+    got = logits()
+    _lib.set_call_hook(lambda name, args, launch: launch())
+    try:
+        steps = logits()
+    finally:
+        _lib.set_call_hook(None)
+    for b, a, e in zip(before, got, steps):
+        assert torch.equal(a, e) and not torch.equal(a, b)
