@@ -359,9 +359,12 @@ __device__ __forceinline__ float unorder32(uint32_t u) {
 //     and gathers every allowed entry at or above the threshold into LDS;
 //  3. a radix select over the candidates' keys (ties at the K-th key ranked by
 //     column) emits the row's top K, unordered: the merge stage orders them.
-// Rows of at most CAP columns are all candidates.  If fewer than K or more
-// than CAP entries qualify, the exact path runs instead, so the result never
-// depends on the sample.  bf16 rows are ranked by logit; of fp32 and fp16 ones,
+// Rows of at most CAP columns are all candidates, and so are the allowed columns
+// where too few were sampled.  If fewer than K or more than CAP entries qualify,
+// the exact path runs instead, so the result never depends on the sample; a row
+// of fewer than K allowed columns takes them and its first masked ones.  (2,048
+// bf16 rows of 248,320, a block of 2,048 allowed columns: 4,371 us by word
+// maxima, which too few words had, and exact passes; 277 here.)  bf16 rows are ranked by logit; of fp32 and fp16 ones,
 // whose logits may differ and their fp32 keys not, the keys are ranked, and the
 // K-th must exceed the threshold's own key, below which nothing was gathered.
 // NT: 1,024 threads where the rows number at most two per CU (one row on a CU
@@ -372,7 +375,7 @@ template <typename T, int CAP, bool MASKED, int NT>
 __global__ __launch_bounds__(NT) void row_select_kernel(
     const T* __restrict__ logits, int64_t ld, const uint8_t* __restrict__ mask, int64_t ld_mask,
     const float* __restrict__ parent, int Wp, int V, int K, float* __restrict__ cand_key,
-    int* __restrict__ cand_idx, int line_stride, int rank) {
+    int* __restrict__ cand_idx, int line_stride, int rank, int single_rank) {
   constexpr bool kBf16 = Elem<T>::code == KAD_DTYPE_BF16;
   constexpr int VE = 16 / sizeof(T);                     // logits per 16-byte word
   constexpr int kRounds = kBf16 ? 2 : 4;                 // key bytes that differ
@@ -384,7 +387,7 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
   __shared__ __attribute__((aligned(16))) uint64_t cand[CAP];
   __shared__ int bins[256];
   __shared__ float red_m[NT / 64], red_s[NT / 64], red_smax[NT / 64];
-  __shared__ int sh_reach[32];
+  __shared__ int sh_reach[32], scan_tmp[NT / 64];
   __shared__ int sh_count, sh_hi, sh_above, sh_ties;
   const int tid = threadIdx.x, lane = tid & 63;
   const int64_t row = blockIdx.x;
@@ -443,11 +446,13 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
   {
     const int nlines = (V + kLine - 1) / kLine;
     const int ng = ((nlines + line_stride - 1) / line_stride) * kPer;
-    uint32_t u[kGroups];
+    constexpr int kKeys = MASKED ? VE : 1;
+    uint32_t u[kGroups][kKeys];
 #pragma unroll
     for (int i = 0; i < kGroups; ++i) {
       const int g = tid + i * NT;
-      u[i] = 0u;
+#pragma unroll
+      for (int e = 0; e < kKeys; ++e) u[i][e] = 0u;
       if (g >= ng) continue;
       float v[VE];
       bool ok[VE];
@@ -457,12 +462,12 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
 #pragma unroll
       for (int e = 0; e < VE; ++e) {
         smax = fmaxf(smax, v[e]);
-        if (ok[e]) {
-          best = fmaxf(best, v[e]);
-          any = true;
-        }
+        if (!ok[e]) continue;
+        best = fmaxf(best, v[e]);
+        any = true;
+        if constexpr (MASKED) u[i][e] = order_of(fmaxf(v[e], -INFINITY));
       }
-      if (any) u[i] = order_of(best);
+      if (!MASKED && any) u[i][0] = order_of(best);
     }
     if (tid == 0 && head > 0) {
       // the columns before the first word enter the maximum: it may be theirs
@@ -476,20 +481,51 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
     if (lane == 0) red_smax[tid >> 6] = smax;
     __syncthreads();
     if (!whole) {
+      // a masked row whose mask reaches few words (a block of 8,192 allowed
+      // columns, 34 of them) ranks its samples singly: so few maxima tell little
+      bool single = false;
+      if constexpr (MASKED) {
+        int c = 0;
+#pragma unroll
+        for (int i = 0; i < kGroups; ++i) {
+          bool any = false;
+#pragma unroll
+          for (int e = 0; e < kKeys; ++e) any |= u[i][e] != 0;
+          c += (int)__popcll(__ballot(any));
+        }
+        if (lane == 0) atomicAdd(&sh_reach[0], c);
+        __syncthreads();
+        single = sh_reach[0] < 4 * rank;
+        if (!single) {
+#pragma unroll
+          for (int i = 0; i < kGroups; ++i)
+#pragma unroll
+            for (int e = 1; e < kKeys; ++e) u[i][0] = max(u[i][0], u[i][e]);
+        }
+      }
+      const int reach = single ? single_rank : rank;
 #pragma unroll 1
       for (int bit = 31; bit >= (kBf16 ? 16 : 12); --bit) {
         const uint32_t t = thr | (1u << bit);
         int c = 0;
 #pragma unroll
-        for (int i = 0; i < kGroups; ++i) c += (int)__popcll(__ballot(u[i] >= t));
+        for (int i = 0; i < kGroups; ++i) c += (int)__popcll(__ballot(u[i][0] >= t));
+        if (single) {
+#pragma unroll
+          for (int i = 0; i < kGroups; ++i)
+#pragma unroll
+            for (int e = 1; e < kKeys; ++e) c += (int)__popcll(__ballot(u[i][e] >= t));
+        }
         if (lane == 0) atomicAdd(&sh_reach[bit], c);
         __syncthreads();
-        if (sh_reach[bit] >= rank) thr = t;
+        if (sh_reach[bit] >= reach) thr = t;
       }
     }
   }
-  // order key 0 (too few allowed samples): the exact path below
-  const float tf = whole ? -INFINITY : (thr ? value_of(thr) : INFINITY);
+  // order key 0: too few allowed samples, hence few allowed columns, which are
+  // all candidates
+  const bool all = whole || (MASKED && thr == 0);
+  const float tf = all ? -INFINITY : (thr ? value_of(thr) : INFINITY);
 
   // ---- 2. max, sum exp, and candidates >= thr in one pass.  The sum of a bf16
   // row is taken against a fixed reference, the sample max (each term one fma
@@ -612,7 +648,34 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
       row_select_exact_float<NT>(row, logits, Elem<T>::code, ld, mask, ld_mask, parent, Wp, V, K,
                                  cand_key, cand_idx, (int*)cand);
   };
-  if ((!whole && thr == 0) || count < K || count > CAP) return exact();
+  if (count > CAP) return exact();
+  if (count < K) {
+    // every allowed column, and the first masked ones for the rest of the K, as
+    // the exact path ranks them where no allowed column's key is -inf
+    bool lowest = !all || !MASKED || (!kBf16 && !(p > -INFINITY)) || lse != lse;
+    for (int i = tid; i < min(count, CAP); i += NT)
+      lowest |= value_of((uint32_t)(cand[i] >> 32)) == -INFINITY;
+    if (__syncthreads_or(lowest)) return exact();
+    const int64_t o = row * K;
+    const int base = (int)(row % Wp) * V;
+    for (int i = tid; i < count; i += NT) {
+      cand_key[o + i] = ((value_of((uint32_t)(cand[i] >> 32)) - M) - lse) + p;
+      cand_idx[o + i] = base + (int)~(uint32_t)cand[i];
+    }
+    int taken = count;
+    for (int c0 = 0; c0 < V && taken < K; c0 += NT) {
+      const int c = c0 + tid;
+      const bool masked = MASKED && c < V && mk[c] == 0;
+      int tot = 0;
+      const int at = taken + block_exclusive_scan<NT>(masked ? 1 : 0, scan_tmp, &tot);
+      if (masked && at < K) {
+        cand_key[o + at] = -INFINITY;
+        cand_idx[o + at] = base + c;
+      }
+      taken += tot;
+    }
+    return;
+  }
 
   // ---- 3. exact top K of the candidates (the merge stage orders them; the
   // row's output order is free).  Candidate = (order key << 32) | ~column,
@@ -651,7 +714,7 @@ __global__ __launch_bounds__(NT) void row_select_kernel(
     need -= sh_above;
   }
   if constexpr (!kBf16) {
-    if (!whole && ustar <= order32(key_of(tf) + 0.f)) return exact();
+    if (!all && ustar <= order32(key_of(tf) + 0.f)) return exact();
   }
   const int r_local = (int)(row % Wp);
   auto emit = [&](uint64_t e) {
@@ -1254,8 +1317,8 @@ int launch_row_select(const void* logits, int logits_dtype, int64_t ld, const vo
                       int64_t ld_mask, const float* parent_scores, int rows, int Wp, int V,
                       int K, float* cand_key, int* cand_idx, hipStream_t s) {
   // sample ~kTargetLines lines: about rank * line_stride = 2K + 256 entries of
-  // the row are at or above the rank-th largest sample.  Of the n word maxima
-  // about n (1 - e^(-rank / n)) are.
+  // the row are at or above the rank-th largest sample (of the allowed ones in a
+  // masked row).  Of the n word maxima about n (1 - e^(-rank / n)) are.
   const int nlines = (V + kLine - 1) / kLine;
   const int line_stride = nlines > kTargetLines ? nlines / kTargetLines : 1;
   const double samples = (double)kad_cdiv(2 * (int64_t)K + 256, line_stride);
@@ -1267,7 +1330,7 @@ int launch_row_select(const void* logits, int logits_dtype, int64_t ld, const vo
 #define KAD_ROW_SELECT(T, CAP, MASKED, NT)                                                      \
   hipLaunchKernelGGL((row_select_kernel<T, CAP, MASKED, NT>), dim3(rows), dim3(NT), 0, s,       \
                      (const T*)logits, ld, (const uint8_t*)mask, ld_mask, parent_scores, Wp, V, \
-                     K, cand_key, cand_idx, line_stride, rank)
+                     K, cand_key, cand_idx, line_stride, rank, (int)samples)
 #define KAD_ROW_SELECT_NT(T, CAP, MASKED)                \
   if (few) KAD_ROW_SELECT(T, CAP, MASKED, 1024);         \
   else KAD_ROW_SELECT(T, CAP, MASKED, 256)

@@ -281,6 +281,33 @@ def test_select_float_scores_under_a_peak_outside_the_sample(device, dtype, peak
     assert bool((err[~top] <= 1.5 * ulp[~top] + 8 * 2.0 ** -23).all()), err[~top]
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("allowed", [0, 1, 20, 700, 3000, 9000])
+@pytest.mark.parametrize("spread", ["block", "random"])
+def test_select_rows_of_few_allowed_columns(device, dtype, allowed, spread):
+    """Constraint masks that leave a block of columns, or as many anywhere: fewer
+    than the level's width, than the sample's rank, than the candidate buffer,
+    and more.  Unfilled slots take the lowest masked candidates, in order."""
+    Wp, V, W = 5, 60001, 40
+    g = torch.Generator().manual_seed(allowed)
+    logits = (torch.randn(1, Wp, V, generator=g) * 2).to(dtype)
+    scores = -torch.rand(1, Wp, generator=g)
+    mask = torch.zeros(1, Wp, V, dtype=torch.bool)
+    for r in range(Wp):
+        at = torch.randperm(V, generator=g)[:allowed] if spread == "random" else \
+            torch.arange(20000 + 900 * r, 20000 + 900 * r + allowed)
+        mask[0, r, at] = True
+    s, p, t, valid = select_level(logits.to(device), scores.to(device), W, mask.to(device))
+    keys = (logits.double().log_softmax(-1) + scores.double()[..., None])
+    keys = keys.masked_fill(~mask, -float("inf"))
+    n = min(W, Wp * allowed)
+    assert int(valid.sum()) == n and bool(valid[0, :n].all())
+    if n:
+        assert_selection_gap_aware(s[:, :n], p[:, :n], t[:, :n], keys, n, 1e-5, name="few")
+    free = (~mask[0]).reshape(-1).nonzero()[:W - n, 0]
+    assert torch.equal((p * V + t)[0, n:].cpu(), free)
+
+
 def test_select_float_rows_with_equal_keys_take_lower_columns(device):
     """fp32 logits that differ by less than their keys' precision tie, and the
     lower columns of all of them are taken, sampled or not."""
