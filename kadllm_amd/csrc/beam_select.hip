@@ -31,6 +31,7 @@
 #include <cfloat>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 // Scratch of kad_beam_select_noalloc (32 MiB per GPU; see scratch_address).
 static __device__ __align__(256) uint8_t scratch[32ll << 20];
@@ -862,17 +863,18 @@ __device__ void emit_sorted(uint64_t* words, int count, int W, int V, float* sco
   }
 }
 
-// One workgroup per request.  Levels of up to kPruneCap candidates are sorted
-// whole; of more, a sample's order statistic gives a threshold that about
-// 2 W + 256 candidates reach, one pass collects those, and they are sorted --
-// what is collected holds the W best, ties by index included, whenever it
-// numbers at least W.  Otherwise (many equal keys, or W past about 1,400) the
-// radix rounds below.  8 requests x 65,536 candidates, W 256: 85 us by the radix
-// rounds alone, 35 with the sampled threshold.
+// One workgroup per request.  With prune (merge_prunes), levels of up to
+// kPruneCap candidates are sorted whole; of more, a sample's order statistic
+// gives a threshold that about 2 W + 256 candidates reach, one pass collects
+// those, and they are sorted -- what is collected holds the W best, ties by index
+// included, whenever it numbers at least W.  Otherwise (many equal keys, or W
+// past about 1,400) and without prune the radix rounds below.  8 requests x
+// 65,536 candidates, W 256: 85 us by the radix rounds alone, 35 with the sampled
+// threshold.
 __global__ __launch_bounds__(kMergeThreads) void merge_select_kernel(
     const float* __restrict__ cand_key, const int* __restrict__ cand_idx, int ncand, int W,
     int V, float* __restrict__ scores, int64_t* __restrict__ parents,
-    int64_t* __restrict__ tokens, uint8_t* __restrict__ valid, int cap) {
+    int64_t* __restrict__ tokens, uint8_t* __restrict__ valid, int cap, int prune) {
   __shared__ int hist[256];
   __shared__ uint32_t sh_prefix;
   __shared__ int sh_need, sh_count, sh_ties;
@@ -887,17 +889,22 @@ __global__ __launch_bounds__(kMergeThreads) void merge_select_kernel(
   // f(order key, candidate index) over this thread's candidates
   auto for_each = [&](auto&& f) {
     int i0 = tid;
-    for (; i0 + (kMergeBatch - 1) * kMergeThreads < ncand; i0 += kMergeBatch * kMergeThreads) {
-      float kv[kMergeBatch];
+    auto batches = [&](auto size) {
+      constexpr int kB = decltype(size)::value;
+      for (; i0 + (kB - 1) * kMergeThreads < ncand; i0 += kB * kMergeThreads) {
+        float kv[kB];
 #pragma unroll
-      for (int q = 0; q < kMergeBatch; ++q) kv[q] = keys[i0 + q * kMergeThreads];
+        for (int q = 0; q < kB; ++q) kv[q] = keys[i0 + q * kMergeThreads];
 #pragma unroll
-      for (int q = 0; q < kMergeBatch; ++q) f(order32(kv[q]), i0 + q * kMergeThreads);
-    }
-    for (int i = i0; i < ncand; i += kMergeThreads) f(order32(keys[i]), i);
+        for (int q = 0; q < kB; ++q) f(order32(kv[q]), i0 + q * kMergeThreads);
+      }
+    };
+    batches(std::integral_constant<int, kMergeBatch>{});
+    batches(std::integral_constant<int, 4>{});
+    batches(std::integral_constant<int, 1>{});
   };
 
-  if (ncand <= kPruneCap || 2 * W + 256 <= kPruneCap * 3 / 4) {
+  if (prune) {
     __shared__ int sh_reach[32];
     uint64_t* words = (uint64_t*)merge_lds;
     if (tid < 32) sh_reach[tid] = 0;
@@ -1355,11 +1362,29 @@ int launch_row_select(const void* logits, int logits_dtype, int64_t ld, const vo
   return kad_launch_status("row_select_kernel");
 }
 
+// Whether collecting and sorting past a threshold is the shorter way: its sort
+// takes 10, 17 or 35 us for up to 1,024, 2,048 or 4,096 words and the sampling 8;
+// a radix round grows with the candidates and the winners' sort, run in LDS,
+// with lg W (lg W + 1) / 2 (us on one request: 3,200 candidates, W 50: 15 by
+// radix rounds, 35 by sorting; 4,096, W 2,000: 56 and 36; 8,192, W 8: 13 and 20,
+// W 256: 23 and 20).
+bool merge_prunes(int ncand, int W) {
+  const bool sampled = ncand > kPruneCap;
+  const int64_t words = sampled ? 2 * (int64_t)W + 256 : ncand;
+  if (words > (sampled ? kPruneCap * 3 / 4 : kPruneCap)) return false;
+  int lg = 0;
+  while ((1 << lg) < W) ++lg;
+  const double sort = words <= 1024 ? 10 : (words <= 2048 ? 17 : 35);
+  const double radix = 4 + 0.0008 * ncand + 0.35 * lg * (lg + 1) / 2 * (W > 1024 ? 2 : 1);
+  return sort + (sampled ? 8 + 0.00015 * ncand : 0) <= radix;
+}
+
 int launch_merge(const float* cand_key, const int* cand_idx, int B, int ncand, int W, int V,
                  float* scores, int64_t* parents, int64_t* tokens, void* valid, hipStream_t s) {
   int cap = 1;
   while (cap < W) cap <<= 1;
-  const size_t lds = (size_t)std::max(cap, kPruneCap) * 8;
+  const bool prune = merge_prunes(ncand, W);
+  const size_t lds = (size_t)(prune ? std::max(cap, kPruneCap) : cap) * 8;
   if (lds > 64 * 1024) {
     // beyond the default 64 KB of dynamic LDS per workgroup (the CU has 160 KB)
     const hipError_t e = hipFuncSetAttribute((const void*)merge_select_kernel,
@@ -1372,7 +1397,8 @@ int launch_merge(const float* cand_key, const int* cand_idx, int B, int ncand, i
     }
   }
   hipLaunchKernelGGL(merge_select_kernel, dim3(B), dim3(kMergeThreads), lds, s, cand_key, cand_idx,
-                     ncand, W, V, scores, parents, tokens, (uint8_t*)valid, cap);
+                     ncand, W, V, scores, parents, tokens, (uint8_t*)valid, cap,
+                     (int)prune);
   return kad_launch_status("merge_select_kernel");
 }
 
