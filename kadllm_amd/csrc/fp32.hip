@@ -54,6 +54,15 @@ constexpr int kSlots = 4, kSlice = 64 * 32;  // floats of one operand's slice
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t src, float* lds, uint32_t lane_at,
+                                           uint32_t at) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void_t*)lds, 16, lane_at, at, 0, 0);
+}
+__device__ __forceinline__ void load_lds4(__amdgpu_buffer_rsrc_t src, float* lds, uint32_t lane_at,
+                                          uint32_t at) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void_t*)lds, 4, lane_at, at, 0, 0);
+}
+
 // one output element (or gate / up pair) through the epilogue
 __device__ __forceinline__ void gemm_f32_store(int epilogue, float* C, int64_t ldc, const float* R,
                                                int64_t ldr, int64_t row, int col, float v) {
@@ -61,45 +70,56 @@ __device__ __forceinline__ void gemm_f32_store(int epilogue, float* C, int64_t l
   C[row * ldc + col] = v;
 }
 
+// WIDE: 16-byte loads (16-byte rows, K a multiple of 4), else 4-byte ones.  TAIL:
+// the last slice may reach past K.  2,048 x 2,048 x 1,000 180 us as K split over
+// waves (below), 69 here, x 1,001 478 and 90.
+template <bool WIDE, bool TAIL>
 __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ Wt, int64_t ldw,
     float* C, int64_t ldc, const float* R, int64_t ldr, int M, int N, int K, int epilogue,
     int mtiles) {
+  constexpr int kFl = WIDE ? 4 : 1;          // floats a lane loads
+  constexpr int kLPW = 2048 / (64 * kFl * 4);  // loads per wave, operand and slice
+  constexpr int kRows = 2 * kFl;             // slice rows a load covers
   __shared__ __attribute__((aligned(1024))) float ring[kSlots][2 * kSlice];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lid = xcd_logical_id(blockIdx.x, gridDim.x);
   const int m0 = (lid % mtiles) * 64, n0 = (lid / mtiles) * 64;
-  // a direct load writes 64 x 16 bytes in lane order: 8 rows of a slice, lane
-  // l row l / 8, and fetches the chunk that belongs at its place.  The wave
-  // loads row groups wave and wave + 4 of each operand; rows past the end
-  // repeat the last one (their results are not stored).  Buffer loads take a
-  // lane's row as a fixed offset and the slice as a uniform one, which costs
-  // no address arithmetic between the MFMAs (offsets below 2 GB: checked by
-  // the dispatch).
-  const int dr = lane >> 3;
-  const __amdgpu_buffer_rsrc_t ab = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(A + (int64_t)m0 * lda), 0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t wb = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(Wt + (int64_t)n0 * ldw), 0, 0x7fffffff, 0x00020000);
-  uint32_t ao[2], wo[2];
+  // a direct load writes 64 x 16 (or 4) bytes in lane order: 8 (2) rows of a
+  // slice, and fetches what belongs at its place.  The wave loads row groups
+  // wave, wave + 4, ... of each operand; rows past the end repeat the last one
+  // (their results are not stored).  Buffer loads take a lane's row as a fixed
+  // offset and the slice as a uniform one, which costs no address arithmetic
+  // between the MFMAs (offsets below 2 GB: checked by the dispatch), and read
+  // nothing past the last row's end: a slice that reaches there is zeroed below.
+  auto bounded = [&](const float* p, int64_t ld, int rows) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0,
+                                             (int)(((min(rows, 64) - 1) * ld + K) * 4), 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t ab = bounded(A + (int64_t)m0 * lda, lda, M - m0);
+  const __amdgpu_buffer_rsrc_t wb = bounded(Wt + (int64_t)n0 * ldw, ldw, N - n0);
+  uint32_t ao[kLPW], wo[kLPW];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = (wave + 4 * i) * 8 + dr;
-    const int ch = ((lane & 7) ^ ((r >> 1) & 7)) * 4;
+  for (int i = 0; i < kLPW; ++i) {
+    const int r = (wave + 4 * i) * kRows + lane / (32 / kFl), at = lane % (32 / kFl) * kFl;
+    const int ch = ((at / 4) ^ ((r >> 1) & 7)) * 4 + at % 4;
     ao[i] = (uint32_t)(((int64_t)(min(m0 + r, M - 1) - m0) * lda + ch) * 4);
     wo[i] = (uint32_t)(((int64_t)(min(n0 + r, N - 1) - n0) * ldw + ch) * 4);
   }
-  const int KT = K / 32;
+  const int KT = (K + 31) / 32;
   // slice t into slot `at`; past the last slice, that one again (never read)
   auto issue = [&](int t, int at) {
-    float* slot = ring[at] + wave * 8 * 32;
     const uint32_t k = (uint32_t)min(t, KT - 1) * 128;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ab, (lds_void_t*)(slot + i * 4 * 8 * 32), 16, ao[i],
-                                               k, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wb, (lds_void_t*)(slot + kSlice + i * 4 * 8 * 32),
-                                               16, wo[i], k, 0, 0);
+    for (int i = 0; i < kLPW; ++i) {
+      float* slot = ring[at] + (wave + 4 * i) * kRows * 32;
+      if constexpr (WIDE) {
+        load_lds16(ab, slot, ao[i], k);
+        load_lds16(wb, slot + kSlice, wo[i], k);
+      } else {
+        load_lds4(ab, slot, ao[i], k);
+        load_lds4(wb, slot + kSlice, wo[i], k);
+      }
     }
   };
   f32x4_t acc[4];
@@ -128,11 +148,11 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
   // A wave holds slice t in registers when it reaches the barrier between the
   // slice's two halves: after it the slot takes slice t + kSlots, and slice
   // t + 1 (landed by then) is read while the second half multiplies.  The
-  // barrier does not wait for the loads still in flight (4 a slice); the empty
+  // barrier does not wait for the loads still in flight (2 kLPW a slice); the empty
   // asm statements keep LDS accesses on their side of it.
 #pragma unroll
   for (int t = 0; t < kSlots; ++t) issue(t, t);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(4 * (kSlots - 1)) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * kLPW * (kSlots - 1)) : "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   Frags f[2];
@@ -141,13 +161,26 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
   auto step = [&](int t, auto slot) -> bool {
     constexpr int at = decltype(slot)::value;
     Frags &cur = f[at & 1], &next = f[(at + 1) & 1];
+    if constexpr (TAIL) {
+      if (t + 1 == KT) {
+#pragma unroll
+        for (int piece = 0; piece < 2; ++piece)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (t * 32 + piece * 16 + fq * 4 + e >= K) {
+              cur.a[piece][e] = 0.f;
+#pragma unroll
+              for (int g = 0; g < 4; ++g) cur.w[piece][g][e] = 0.f;
+            }
+      }
+    }
     mfmas(cur, 0);
     __builtin_amdgcn_sched_barrier(0);
     if (t + 1 == KT) {
       mfmas(cur, 1);
       return false;
     }
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(4 * (kSlots - 2)) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(2 * kLPW * (kSlots - 2)) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     read(next, (at + 1) % kSlots);
@@ -158,7 +191,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
     for (int i = 0; i < 16; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       if (i < 10) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      if (i >= 10 && i < 14) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      if (!WIDE || (i >= 10 && i < 14)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
     return true;
@@ -192,8 +225,86 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
         gemm_f32_store(epilogue, C, ldc, R, ldr, row0 + r, n0 + g * 16 + fr, acc[g][r]);
 }
 
-// Products whose 64 x 64 tiles would leave CUs idle, and rows the direct loads
-// do not take: 16 MT rows x 16 columns (SwiGLU: 16 gate and their 16 up
+// Short K: 64 x 64 tiles staged through registers and padded LDS rows, few enough
+// of both that several workgroups share a CU and hide one another's load, which
+// is most of a tile's time, and the output leaves as whole rows (8,192 x 8,192 x
+// 32 115 us in the ring tiles, 88 here; x 33 254 and 111).  Sums as the
+// kernels around it: 32-deep slices of K, then their sums in order.
+constexpr int kShortLd = 20, kShortCld = 65;
+
+__global__ __launch_bounds__(256, 6) void gemm_f32_short_kernel(
+    const float* __restrict__ A, int64_t lda, const float* __restrict__ Wt, int64_t ldw,
+    float* C, int64_t ldc, const float* R, int64_t ldr, int M, int N, int K, int epilogue) {
+  // the operands, and then the output
+  __shared__ __attribute__((aligned(16))) float as[64 * kShortCld];
+  static_assert(2 * kShortLd <= kShortCld, "both operands in the output's place");
+  float *ws = as + 64 * kShortLd, *cs = as;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1, fr = lane & 15, fq = lane >> 4;
+  const int64_t m0 = (int64_t)blockIdx.y * 64;
+  const int n0 = blockIdx.x * 64;
+  f32x4_t acc[2][2], sum[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = sum[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < K; k0 += 16) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = tid + u * 256, r = e / 16, c = e % 16;
+      as[r * kShortLd + c] = m0 + r < M && k0 + c < K ? A[(m0 + r) * lda + k0 + c] : 0.f;
+      ws[r * kShortLd + c] =
+          n0 + r < N && k0 + c < K ? Wt[(int64_t)(n0 + r) * ldw + k0 + c] : 0.f;
+    }
+    __syncthreads();
+    f32x4_t a[2], w[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      a[i] = *(const f32x4_t*)&as[(wm * 32 + i * 16 + fr) * kShortLd + fq * 4];
+      w[i] = *(const f32x4_t*)&ws[(wn * 32 + i * 16 + fr) * kShortLd + fq * 4];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = mfma16x16x4f32(a[i][e], w[j][e], acc[i][j]);
+    if (k0 % 32 || k0 + 16 >= K) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          sum[i][j] += acc[i][j];
+          acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        cs[(wm * 32 + i * 16 + fq * 4 + r) * kShortCld + wn * 32 + j * 16 + fr] = sum[i][j][r];
+  __syncthreads();
+  if (epilogue == KAD_EPI_SWIGLU) {
+    for (int e = tid; e < 64 * 32; e += 256) {
+      const int r = e / 32, c = e % 32;
+      if (m0 + r < M)
+        C[(m0 + r) * ldc + n0 / 2 + c] =
+            silu_exact(cs[r * kShortCld + c]) * cs[r * kShortCld + 32 + c];
+    }
+    return;
+  }
+  for (int e = tid; e < 64 * 64; e += 256) {
+    const int r = e / 64, c = e % 64;
+    if (m0 + r < M && n0 + c < N)
+      gemm_f32_store(epilogue, C, ldc, R, ldr, m0 + r, n0 + c, cs[r * kShortCld + c]);
+  }
+}
+
+// Products whose 64 x 64 tiles would leave CUs idle: 16 MT rows x 16 columns (SwiGLU: 16 gate and their 16 up
 // columns) per workgroup, whose 8 waves take the 32-deep K slices in turn,
 // operands straight from memory, the next slice loading during the current
 // one; the partial sums merge through LDS.  With few rows the weight's bytes
@@ -441,12 +552,27 @@ extern "C" int kad_gemm_f32(const float* A, int64_t lda, const float* W, int64_t
   // its tiles there are (one per CU), the split one 36 us at 64 tiles' worth
   // of rows and columns and 70 us at 80.  At most 32 rows leave half a tile
   // empty: 32 rows against 7,168 x 1,024 are 13 us split, 20 us in tiles.
-  if (vec && K % 32 == 0 && M > 32 && tiles >= 72 && (lda > ldw ? lda : ldw) * 64 + K < 0x1fffffff) {
-    hipLaunchKernelGGL(gemm_f32_tile_kernel, dim3((unsigned)tiles), dim3(256), 0, s, A, lda, W,
-                       ldw, C, ldc, R, ldr, M, N, K, epilogue, (int)kad_cdiv(M, 64));
+  // Beyond 2^23 column tiles its workgroups of 512 no longer fit a grid.
+  const int64_t cols = kad_cdiv(N, epilogue == KAD_EPI_SWIGLU ? 32 : 16);
+  if (((M > 32 && tiles >= 72) || cols >= (1 << 23)) &&
+      (lda > ldw ? lda : ldw) * 64 + K < 0x1fffffff) {
+    // 8,192 x 8,192: K 64 137 us against 150 in the ring, 96 equal; rows that are
+    // not 16-byte ones 129 277 and 388
+    if (K <= (vec ? 64 : 256)) {
+      hipLaunchKernelGGL(gemm_f32_short_kernel,
+                         dim3((unsigned)kad_cdiv(N, 64), (unsigned)kad_cdiv(M, 64)), dim3(256), 0,
+                         s, A, lda, W, ldw, C, ldc, R, ldr, M, N, K, epilogue);
+      return kad_launch_status("gemm_f32_short_kernel");
+    }
+#define KAD_TILE(WIDE, TAIL)                                                                    \
+  hipLaunchKernelGGL((gemm_f32_tile_kernel<WIDE, TAIL>), dim3((unsigned)tiles), dim3(256), 0, s, \
+                     A, lda, W, ldw, C, ldc, R, ldr, M, N, K, epilogue, (int)kad_cdiv(M, 64))
+    if (!vec) KAD_TILE(false, true);
+    else if (K % 32) KAD_TILE(true, true);
+    else KAD_TILE(true, false);
+#undef KAD_TILE
     return kad_launch_status("gemm_f32_tile_kernel");
   }
-  const int64_t cols = kad_cdiv(N, epilogue == KAD_EPI_SWIGLU ? 32 : 16);
   if (kad_cdiv(M, 64) * cols >= 256)
     launch_split_epi<4>(vec, A, lda, W, ldw, C, ldc, R, ldr, M, N, K, epilogue, s);
   else if (M > 16 && kad_cdiv(M, 32) * cols >= 64)

@@ -80,6 +80,37 @@ def test_gemm_f32_kernels_at_their_edges(device, M, N, K):
                                    atol=1e-4, rtol=1e-5)
 
 
+@pytest.mark.parametrize("M,N,K,offset,pad", [
+    (300, 1200, 1000, 0, 0), (257, 1088, 68, 0, 4), (130, 2304, 1001, 0, 0), (129, 2304, 1, 0, 0),
+    (700, 640, 4, 0, 0), (300, 1200, 288, 1, 0), (200, 1500, 257, 0, 3), (64, 64 * 80, 31, 0, 33),
+    (300, 1200, 64, 0, 0), (300, 1217, 256, 1, 0), (65, 64 * 37, 131, 0, 1),
+])
+def test_gemm_f32_tiles_take_any_inner_size(device, M, N, K, offset, pad):
+    """The 64 x 64 tiles, in the ring and staged (short K), where K ends inside a
+    slice and where rows are not 16-byte aligned (a start ``offset`` elements in, rows ``pad`` apart): NaNs lie right
+    behind every row and both matrices.  Sums of at most 1,001 products of unit by
+    0.05: 2e-4."""
+    g = torch.Generator().manual_seed(M + N + K)
+
+    def placed(rows, scale):
+        x = torch.randn(rows, K, generator=g) * scale
+        store = torch.full((offset + rows * (K + pad) + 64,), float("nan"), device=device)
+        d = store[offset:offset + rows * (K + pad)].view(rows, K + pad)[:, :K]
+        return x, d.copy_(x)
+
+    (a, ad), (w, wd) = placed(M, 1.0), placed(N, 0.05)
+    r = torch.randn(M, N, generator=g)
+    ref = a.double() @ w.double().T
+    torch.testing.assert_close(gemm(ad, wd).cpu().double(), ref, atol=2e-4, rtol=1e-5)
+    got = gemm(ad, wd, epilogue=EPI_RESIDUAL, residual=r.to(device))
+    torch.testing.assert_close(got.cpu().double(), ref + r.double(), atol=2e-4, rtol=1e-5)
+    if N % 64 == 0:
+        blocks = ref.view(M, N // 64, 2, 32)
+        expected = (F.silu(blocks[:, :, 0]) * blocks[:, :, 1]).reshape(M, N // 2)
+        torch.testing.assert_close(gemm(ad, wd, epilogue=EPI_SWIGLU).cpu().double(), expected,
+                                   atol=2e-4, rtol=1e-5)
+
+
 def test_rmsnorm_f32_matches_oracle(device):
     g = torch.Generator().manual_seed(2)
     x = torch.randn(33, 256, generator=g)
