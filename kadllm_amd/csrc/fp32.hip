@@ -38,7 +38,11 @@ __device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + 
 // GEMM on v_mfma_f32_16x16x4_f32 (lane l holds A[l % 16][l / 16] and
 // B[l / 16][l % 16]; accumulator element r of lane l is C[(l / 16) * 4 + r][l % 16]).
 // K is taken in pieces of 16: lane group q = l / 16 supplies elements 4 q + e
-// in step e, so that a lane's share of a row is one 16-byte word.
+// in step e, so that a lane's share of a row is one 16-byte word.  Every kernel
+// below sums the 32-deep slices of K in the same eight blocks, each from zero,
+// and then the blocks in order: a row's bits do not depend on how many rows
+// there are, which decides the kernel (2,048 x 2,048 x 1,024 67 us as one sum a
+// tile, 70 by blocks).
 //
 // Large products, bound by the matrix rate: 64 x 64 tiles (small enough that
 // 1,000 rows against 1,024 columns give every CU one), a wave's 16 rows x 64
@@ -51,6 +55,8 @@ __device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + 
 // SwiGLU 275 -> 126 us (116 TFLOP/s), 1,000 x 1,024 x 3,584 399 -> 65 us (113);
 // at 4,096 rows 128 TFLOP/s of the 150 that MFMAs alone reach.
 constexpr int kSlots = 4, kSlice = 64 * 32;  // floats of one operand's slice
+
+__device__ __forceinline__ int slices_per_block(int slices) { return (slices + 7) / 8; }
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 
@@ -122,9 +128,9 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
       }
     }
   };
-  f32x4_t acc[4];
+  f32x4_t acc[4], sum[4];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) acc[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int g = 0; g < 4; ++g) acc[g] = sum[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int fr = lane & 15, fq = lane >> 4, sw = fr >> 1;  // rows differ by multiples of 16
   struct Frags {
     f32x4_t a[2], w[2][4];  // [16-deep piece]
@@ -157,10 +163,19 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
   asm volatile("" ::: "memory");
   Frags f[2];
   read(f[0], 0);
+  int block_end = slices_per_block(KT);
   // false after the last slice
   auto step = [&](int t, auto slot) -> bool {
     constexpr int at = decltype(slot)::value;
     Frags &cur = f[at & 1], &next = f[(at + 1) & 1];
+    if (t == block_end) {
+      block_end += slices_per_block(KT);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        sum[g] += acc[g];
+        acc[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+    }
     if constexpr (TAIL) {
       if (t + 1 == KT) {
 #pragma unroll
@@ -206,6 +221,8 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
   // no load may land in LDS that is another workgroup's by then
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
+#pragma unroll
+  for (int g = 0; g < 4; ++g) sum[g] += acc[g];
   const int64_t row0 = m0 + wave * 16 + fq * 4;
   if (epilogue == KAD_EPI_SWIGLU) {
     // the tile's 64 columns are one [gate 32 | up 32] block of W rows
@@ -214,7 +231,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (row0 + r < M)
-          C[(row0 + r) * ldc + n0 / 2 + g * 16 + fr] = silu_exact(acc[g][r]) * acc[g + 2][r];
+          C[(row0 + r) * ldc + n0 / 2 + g * 16 + fr] = silu_exact(sum[g][r]) * sum[g + 2][r];
     return;
   }
 #pragma unroll
@@ -222,14 +239,14 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       if (row0 + r < M && n0 + g * 16 + fr < N)
-        gemm_f32_store(epilogue, C, ldc, R, ldr, row0 + r, n0 + g * 16 + fr, acc[g][r]);
+        gemm_f32_store(epilogue, C, ldc, R, ldr, row0 + r, n0 + g * 16 + fr, sum[g][r]);
 }
 
 // Short K: 64 x 64 tiles staged through registers and padded LDS rows, few enough
 // of both that several workgroups share a CU and hide one another's load, which
 // is most of a tile's time, and the output leaves as whole rows (8,192 x 8,192 x
-// 32 115 us in the ring tiles, 88 here; x 33 254 and 111).  Sums as the
-// kernels around it: 32-deep slices of K, then their sums in order.
+// 32 115 us in the ring tiles, 88 here; x 33 254 and 111).  At most eight
+// slices: each is a block.
 constexpr int kShortLd = 20, kShortCld = 65;
 
 __global__ __launch_bounds__(256, 6) void gemm_f32_short_kernel(
@@ -305,7 +322,7 @@ __global__ __launch_bounds__(256, 6) void gemm_f32_short_kernel(
 }
 
 // Products whose 64 x 64 tiles would leave CUs idle: 16 MT rows x 16 columns (SwiGLU: 16 gate and their 16 up
-// columns) per workgroup, whose 8 waves take the 32-deep K slices in turn,
+// columns) per workgroup, whose 8 waves take a block of K's slices each,
 // operands straight from memory, the next slice loading during the current
 // one; the partial sums merge through LDS.  With few rows the weight's bytes
 // bound it: 8 rows against 7,168 x 1,024 68 -> 9 us, 1,024 x 3,584 227 -> 13 us.
@@ -354,11 +371,12 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
       for (int i = 0; i < MT; ++i) ar[piece][i] = load4(ap[i], k);
     }
   };
-  const int units = (K + 31) / 32;
-  if (wave < units) load(wave, a, w);
-  for (int u = wave; u < units; u += 8) {
+  const int slices = (K + 31) / 32, per = slices_per_block(slices);
+  const int end = min(slices, (wave + 1) * per);
+  if (wave * per < end) load(wave * per, a, w);
+  for (int u = wave * per; u < end; ++u) {
     f32x4_t an[2][MT], wn[2][NG];
-    load(u + 8 < units ? u + 8 : u, an, wn);
+    load(u + 1 < end ? u + 1 : u, an, wn);
 #pragma unroll
     for (int piece = 0; piece < 2; ++piece)
 #pragma unroll
@@ -556,9 +574,9 @@ extern "C" int kad_gemm_f32(const float* A, int64_t lda, const float* W, int64_t
   const int64_t cols = kad_cdiv(N, epilogue == KAD_EPI_SWIGLU ? 32 : 16);
   if (((M > 32 && tiles >= 72) || cols >= (1 << 23)) &&
       (lda > ldw ? lda : ldw) * 64 + K < 0x1fffffff) {
-    // 8,192 x 8,192: K 64 137 us against 150 in the ring, 96 equal; rows that are
-    // not 16-byte ones 129 277 and 388
-    if (K <= (vec ? 64 : 256)) {
+    // 8,192 x 8,192: K 96 193 us against 202 in the ring, 128 244 and 226; rows
+    // that are not 16-byte ones 129 277 and 388
+    if (K <= (vec ? 96 : 256)) {
       hipLaunchKernelGGL(gemm_f32_short_kernel,
                          dim3((unsigned)kad_cdiv(N, 64), (unsigned)kad_cdiv(M, 64)), dim3(256), 0,
                          s, A, lda, W, ldw, C, ldc, R, ldr, M, N, K, epilogue);

@@ -111,6 +111,21 @@ def test_gemm_f32_tiles_take_any_inner_size(device, M, N, K, offset, pad):
                                    atol=2e-4, rtol=1e-5)
 
 
+@pytest.mark.parametrize("N,K,offset", [(1152, 1000, 0), (1152, 1024, 0), (2304, 64, 0),
+                                        (2304, 33, 0), (1152, 300, 1), (3648, 32, 0)])
+@pytest.mark.parametrize("epi", [0, EPI_SWIGLU])
+def test_gemm_f32_rows_do_not_depend_on_the_others(device, N, K, offset, epi):
+    """A row's bits in products of 1 to 1,000 rows: K split over waves for few of
+    them, ring tiles, and staged tiles for short K."""
+    g = torch.Generator().manual_seed(N + K)
+    a = torch.randn(1000, K, generator=g)
+    ad = torch.empty(a.numel() + offset, device=device)[offset:].view(a.shape).copy_(a)
+    w = (torch.randn(N, K, generator=g) * 0.05).to(device)
+    whole = gemm(ad, w, epilogue=epi)
+    for rows in (1, 16, 17, 32, 33, 64, 100, 300):
+        assert torch.equal(gemm(ad[:rows], w, epilogue=epi), whole[:rows]), rows
+
+
 def test_rmsnorm_f32_matches_oracle(device):
     g = torch.Generator().manual_seed(2)
     x = torch.randn(33, 256, generator=g)
