@@ -11,6 +11,7 @@
 // ops.py:152-158 and one softmax over the prefix and causal suffix keys
 // (equal to the two-partition LSE merge of ops.py:229-249,340).
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -26,6 +27,9 @@ __device__ __forceinline__ void store_from_float(void* p, int64_t i, int dtype, 
   else
     ((_Float16*)p)[i] = (_Float16)f;
 }
+
+// workgroups of 256 in one launch: a grid holds fewer than 2^32 work-items
+constexpr int kMaxBlocks = (1 << 24) - 1;
 
 // 1 / (1 + e^-x) with the IEEE exp and divide (torch.sigmoid in fp32)
 __device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + expf(-x)); }
@@ -81,7 +85,7 @@ __global__ __launch_bounds__(256) void gdn_recurrent_kernel(
     int gate_dtype, const void* __restrict__ beta, int beta_dtype, int64_t ld_gate,
     const void* __restrict__ init, int state_dtype, int beams_per_state, TIN* __restrict__ out,
     int64_t ld_out, float* __restrict__ final_state, int T, int H, int HV, int K, int V,
-    float scale, int nvt, int wide) {
+    float scale, int nvt, int wide, int first) {
   constexpr int VW = KV < 4 ? KV : 4, NC = KV / VW, KP = 16 * KV;
   constexpr int kQK = kTile * KP;   // floats of a tile's k (or q) rows
   constexpr int kStage = 2 * kQK > KP * (kCols + 1) ? 2 * kQK : KP * (kCols + 1);
@@ -95,7 +99,7 @@ __global__ __launch_bounds__(256) void gdn_recurrent_kernel(
   const int vt = (int)(blockIdx.x % (unsigned)nvt);
   const int64_t nh = blockIdx.x / (unsigned)nvt;
   const int hv = (int)(nh % HV);
-  const int64_t n = nh / HV;
+  const int64_t n = first + nh / HV;
   const int h = hv / (HV / H);
   const int v0 = vt * kCols, ncol = min(kCols, V - v0);
 
@@ -269,17 +273,21 @@ int launch_recurrent(const void* q, const void* k, const void* v, int64_t ld_qk,
                      int64_t ld_out, float* fin, int N, int T, int H, int HV, int K, int V,
                      float scale, hipStream_t s) {
   const int nvt = (V + kCols - 1) / kCols;
-  const int64_t blocks = (int64_t)N * HV * nvt;
-  if (blocks > 0x7fffffffLL) KAD_UNSUPPORTED("too many (sequence, head) pairs for one launch");
+  if ((int64_t)HV * nvt > kMaxBlocks) KAD_UNSUPPORTED("too many heads for one launch");
   // whole vectors of min(KV, 4) elements: full, aligned rows
   constexpr int VW = KV < 4 ? KV : 4;
   const int wide = K == 16 * KV && ld_qk % VW == 0 && ((uintptr_t)q % (VW * sizeof(TIN))) == 0 &&
                    ((uintptr_t)k % (VW * sizeof(TIN))) == 0;
-  hipLaunchKernelGGL((gdn_recurrent_kernel<TIN, KV>), dim3((unsigned)blocks), dim3(256), 0, s,
-                     (const TIN*)q, (const TIN*)k, (const TIN*)v, ld_qk, ld_v, g, gate_dtype,
-                     beta, beta_dtype, ld_gate, init, state_dtype, bps, (TIN*)out, ld_out, fin, T,
-                     H, HV, K, V, scale, nvt, wide);
-  return kad_launch_status("gdn_recurrent_kernel");
+  const int per = kMaxBlocks / (HV * nvt);  // sequences of a launch
+  for (int first = 0; first < N; first += std::min(per, N - first)) {
+    const int blocks = std::min(per, N - first) * HV * nvt;
+    hipLaunchKernelGGL((gdn_recurrent_kernel<TIN, KV>), dim3((unsigned)blocks), dim3(256), 0, s,
+                       (const TIN*)q, (const TIN*)k, (const TIN*)v, ld_qk, ld_v, g, gate_dtype,
+                       beta, beta_dtype, ld_gate, init, state_dtype, bps, (TIN*)out, ld_out, fin,
+                       T, H, HV, K, V, scale, nvt, wide, first);
+    if (const int rc = kad_launch_status("gdn_recurrent_kernel")) return rc;
+  }
+  return KAD_OK;
 }
 
 // ---------------------------------------------------------------------------

@@ -79,6 +79,24 @@ def test_gated_delta_recurrence_tile_edges(device, T, K, V, offset):
     torch.testing.assert_close(gf.double().cpu(), ef.double(), atol=2e-5, rtol=1e-4)
 
 
+def test_gated_delta_of_more_sequences_than_a_grid_holds(device):
+    """2^24 + 3 one-token sequences of one-dimensional heads: as many workgroups of
+    256, more work-items than one launch takes.  fp32: 1e-5 relative."""
+    N = (1 << 24) + 3
+    gen = torch.Generator(device=device).manual_seed(1)
+    q, k, v, S = (torch.randn(N, 1, 1, 1, generator=gen, device=device) for _ in range(4))
+    g = -torch.rand(N, 1, 1, generator=gen, device=device)
+    beta = torch.rand(N, 1, 1, generator=gen, device=device)
+    out, final = ops.gated_delta(q, k, v, g, beta, S, return_final_state=True)
+    q, k, v, S, g, beta = (t.flatten().double() for t in (q, k, v, S, g, beta))
+    kn = k / (k * k + 1e-6).sqrt()
+    S = S * g.exp()
+    S = S + kn * beta * (v - S * kn)
+    torch.testing.assert_close(final.flatten().double(), S, atol=1e-5, rtol=1e-5)
+    torch.testing.assert_close(out.flatten().double(), S * q / (q * q + 1e-6).sqrt(), atol=1e-5,
+                               rtol=1e-5)
+
+
 def _attn_inputs(B, W, T, H, HK, L, D, dtype, seed, Tk=None):
     g = torch.Generator().manual_seed(seed)
     Tk = T if Tk is None else Tk
