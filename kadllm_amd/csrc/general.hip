@@ -333,6 +333,7 @@ struct AttnArgs {
   int by_token;      // suffix order, see attention_general_kernel
   int beams;         // beams that share a group of rows: W, or 1
   int rows, tiles;   // rows of a group, and its 16-row tiles
+  int first;         // the launch's first tile
   float scale;
 };
 
@@ -441,7 +442,7 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, j = lane >> 4;
   const int G = a.H / a.HK;
-  const int lid = xcd_logical_id(blockIdx.x, gridDim.x);
+  const int lid = a.first + xcd_logical_id(blockIdx.x, gridDim.x);
   const int tile = lid % a.tiles;
   const int hk = (lid / a.tiles) % a.HK;
   const int64_t n0 = (int64_t)(lid / a.tiles / a.HK) * a.beams;  // the group's first beam
@@ -654,24 +655,27 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
 }
 
 template <typename TIN, int DMAX>
-int launch_attention(const AttnArgs& a, unsigned blocks, hipStream_t s) {
+int launch_attention(AttnArgs a, int blocks, hipStream_t s) {
   const int64_t strides[] = {a.sq_n, a.sq_t, a.sq_h, a.sp_b, a.sp_l, a.sp_h, a.ssk_n,
                              a.ssk_t, a.ssk_h, a.ssv_n, a.ssv_t, a.ssv_h};
   bool full = a.D == DMAX;
   for (int64_t x : strides) full = full && x % 4 == 0;
   for (const void* p : {a.q, a.pk, a.pv, a.sk, a.sv})
     full = full && ((uintptr_t)p % (4 * sizeof(TIN))) == 0;
-  if (full)
-    hipLaunchKernelGGL((attention_general_kernel<TIN, DMAX, true>), dim3(blocks), dim3(256), 0, s,
-                       a);
-  else
-    hipLaunchKernelGGL((attention_general_kernel<TIN, DMAX, false>), dim3(blocks), dim3(256), 0, s,
-                       a);
-  return kad_launch_status("attention_general_kernel");
+  while (a.first < blocks) {
+    const int n = std::min(kMaxBlocks, blocks - a.first);
+    if (full)
+      hipLaunchKernelGGL((attention_general_kernel<TIN, DMAX, true>), dim3(n), dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL((attention_general_kernel<TIN, DMAX, false>), dim3(n), dim3(256), 0, s, a);
+    if (const int rc = kad_launch_status("attention_general_kernel")) return rc;
+    a.first += n;
+  }
+  return KAD_OK;
 }
 
 template <typename TIN>
-int launch_attention_dim(const AttnArgs& a, unsigned blocks, hipStream_t s) {
+int launch_attention_dim(const AttnArgs& a, int blocks, hipStream_t s) {
   if (a.D <= 64) return launch_attention<TIN, 64>(a, blocks, s);
   if (a.D <= 128) return launch_attention<TIN, 128>(a, blocks, s);
   return launch_attention<TIN, 256>(a, blocks, s);
@@ -752,9 +756,9 @@ extern "C" int kad_attention_general(
   const AttnArgs a{q, prefix_k, prefix_v, suffix_k, suffix_v, gate, (const uint8_t*)prefix_mask,
                    out, sq_n, sq_t, sq_h, sp_b, sp_l, sp_h, ssk_n, ssk_t, ssk_h, ssv_n, ssv_t,
                    ssv_h, sg_n, sg_t, sg_h, so_n, so_t, so_h, W, Tq, Tk, H, HK, L, D, by_token,
-                   beams, (int)grows, (int)tiles, scale};
+                   beams, (int)grows, (int)tiles, 0, scale};
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == KAD_DTYPE_F32) return launch_attention_dim<float>(a, (unsigned)blocks, s);
-  if (dtype == KAD_DTYPE_BF16) return launch_attention_dim<bf16_t>(a, (unsigned)blocks, s);
-  return launch_attention_dim<_Float16>(a, (unsigned)blocks, s);
+  if (dtype == KAD_DTYPE_F32) return launch_attention_dim<float>(a, (int)blocks, s);
+  if (dtype == KAD_DTYPE_BF16) return launch_attention_dim<bf16_t>(a, (int)blocks, s);
+  return launch_attention_dim<_Float16>(a, (int)blocks, s);
 }

@@ -178,6 +178,16 @@ def test_prefix_attention_general_nonfinite_values_stay_with_their_rows(device, 
     torch.testing.assert_close(got, expected, atol=2e-5, rtol=1e-4)
 
 
+def test_prefix_attention_of_more_rows_than_a_grid_holds(device):
+    """2^20 + 1 requests of 16 heads and one token: 2^24 + 16 workgroups of 256,
+    more work-items than one launch takes.  A row that sees one key is its V."""
+    B, H, D = (1 << 20) + 1, 16, 4
+    gen = torch.Generator(device=device).manual_seed(1)
+    q, sk, sv = (torch.randn(B, 1, H, D, generator=gen, device=device) for _ in range(3))
+    none = torch.empty(B, 0, H, D, device=device)
+    assert torch.equal(ops.prefix_attention(q, none, none, sk, sv), sv)
+
+
 def test_prefix_attention_general_query_offset_and_gate(device):
     """Queries that are the last Tq of Tk suffix tokens equal the last rows of
     the full Tk-token attention; a gate multiplies by its rounded sigmoid."""
