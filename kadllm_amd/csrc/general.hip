@@ -299,8 +299,8 @@ int launch_recurrent(const void* q, const void* k, const void* v, int64_t ld_qk,
 // the request's prefix keys, then the suffix.  Suffixes of up to 8 tokens go
 // one token a step, its 16 keys the tile's beams (a row sees its own); longer
 // ones, whole prompts among them, keep to one beam per tile and go 16 tokens a
-// step.  Either way a row's keys come in steps that do not depend on which
-// rows share its tile or on how many tokens follow, nor do its bits.  Each wave folds
+// step.  Within either order a row's keys come in steps that do not depend on
+// which rows share its tile or on how many tokens follow, nor do its bits.  Each wave folds
 // its steps with an online softmax into O^T = V^T P^T -- the accumulator of
 // S^T is P^T's operand as it stands -- and the four partial results merge
 // through LDS.  Splitting the keys over the waves rather than the rows fills
@@ -319,7 +319,7 @@ int launch_recurrent(const void* q, const void* k, const void* v, int64_t ld_qk,
 // A product with weight 0 is not left out of an MFMA, so an infinite or NaN V
 // entry that a row must not see would reach it.  Rows whose result is not
 // finite are therefore computed again one by one (attention_row), skipping
-// the keys of weight 0.
+// the keys of weight 0; their sums then run in another order.
 struct AttnArgs {
   const void *q, *pk, *pv, *sk, *sv, *gate;
   const uint8_t* mask;
@@ -439,6 +439,7 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
   typedef TIN raw4 __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(16))) float po[4][16 * LDO];
   __shared__ float pm[4][16], pl[4][16];
+  __shared__ int again[16];  // rows whose result is not finite
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, j = lane >> 4;
   const int G = a.H / a.HK;
@@ -515,6 +516,7 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
   for (int i = 0; i < NV * 4; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;  // l: this lane's share of the row's sum
 
+  if (tid < 16) again[tid] = 0;
   if (wave < steps) load_k(wave);
   __syncthreads();
   for (int s = wave; s < steps; s += 4) {
@@ -641,17 +643,17 @@ __global__ __launch_bounds__(256, 1) void attention_general_kernel(AttnArgs a) {
       finite = finite && fabsf(y[i][e]) < INFINITY;
     }
   }
-  if (__syncthreads_or(!finite)) {
-    for (int r = r0 + wave; r <= r1; r += 4)
-      attention_row<TIN, DMAX>(a, po[wave], n0 + r / (a.Tq * G), r / G % a.Tq, hk * G + r % G);
-    return;
-  }
-  if (r0 + mr < a.rows)
+  if (!finite) again[mr] = 1;
+  __syncthreads();  // and every partial output is read
+  if (r0 + mr < a.rows && !again[mr])
 #pragma unroll
     for (int i = 0; i < NV; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (64 * i + md + e < a.D) attention_store<TIN>(a, on, ot, oh, 64 * i + md + e, y[i][e]);
+  for (int r = r0 + wave; r <= r1; r += 4)
+    if (again[r - r0])
+      attention_row<TIN, DMAX>(a, po[wave], n0 + r / (a.Tq * G), r / G % a.Tq, hk * G + r % G);
 }
 
 template <typename TIN, int DMAX>

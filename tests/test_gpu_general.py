@@ -188,6 +188,21 @@ def test_prefix_attention_of_more_rows_than_a_grid_holds(device):
     assert torch.equal(ops.prefix_attention(q, none, none, sk, sv), sv)
 
 
+@pytest.mark.parametrize("Tk", [2, 20])
+def test_prefix_attention_general_rows_beside_nonfinite_ones_keep_their_bits(device, Tk):
+    """A row whose result is not finite is computed again; the rows that share its
+    tile are not: the bits of the same call without it."""
+    B, W, H, HK, L, D = 1, 4, 4, 2, 40, 64
+    dev = _on(device, *_attn_inputs(B, W, Tk, H, HK, L, D, torch.float32, seed=Tk))
+    clean = ops.prefix_attention(*dev, beam_width=W)
+    dev[0][1, -1] = 0.0
+    dev[0][1, -1, :, 0] = float("inf")      # beam 1's last query: its scores and no others
+    got = ops.prefix_attention(*dev, beam_width=W)
+    assert not torch.isfinite(got[1, -1]).any()
+    got[1, -1] = clean[1, -1]
+    assert torch.equal(got, clean)
+
+
 def test_prefix_attention_general_query_offset_and_gate(device):
     """Queries that are the last Tq of Tk suffix tokens equal the last rows of
     the full Tk-token attention; a gate multiplies by its rounded sigmoid."""
