@@ -15,6 +15,8 @@
 // reference's contiguous [BW, C, T] layout, both in 16-byte words of any of the
 // three types, and a scalar one for any other strides and widths.
 
+#include <algorithm>
+
 #include "kad_common.h"
 
 namespace {
@@ -162,7 +164,7 @@ struct ConvVec {
 // taps are loaded once); width 4 (3 taps), any T.  Grid: x = request x beam
 // group, y = channel groups of 256 threads, z = runs of kConvRun tokens of
 // suffixes longer than 4 (an fp32 model's whole prompts, which one thread per
-// channel would walk).  The next (beam, token) row is loaded before the current
+// channel would walk; longer runs where a grid does not hold as many).  The next (beam, token) row is loaded before the current
 // one is computed so that every thread keeps one 16-byte load in flight.
 constexpr int kConvBeams = 8, kConvRun = 16;
 
@@ -173,10 +175,10 @@ __global__ __launch_bounds__(256) void conv_suffix_vec(
     const T* __restrict__ x, int64_t sx_n, int64_t sx_t, const T* __restrict__ state,
     int64_t ss_b, int64_t ss_c, int64_t ss_t, int history, const T* __restrict__ w,
     T* __restrict__ out, int64_t so_n, int64_t so_t, int W, int C, int T_rt, int nbg, int beams,
-    int silu) {
+    int run, int silu) {
   constexpr int VE = ConvVec<T>::VE;
-  const int t0 = TT > 0 ? 0 : blockIdx.z * kConvRun;
-  const int T_ = TT > 0 ? TT : min(kConvRun, T_rt - t0);
+  const int t0 = TT > 0 ? 0 : blockIdx.z * run;
+  const int T_ = TT > 0 ? TT : min(run, T_rt - t0);
   const int cv = blockIdx.y * 256 + threadIdx.x;
   if (cv >= C / VE) return;
   const int c0 = cv * VE;
@@ -477,13 +479,13 @@ int launch_typed(const void* x, int64_t sx_n, int64_t sx_c, int64_t sx_t, const 
   const int nbg = (int)kad_cdiv(W, beams);
   if (vec) {
     KAD_REQUIRE((int64_t)B * nbg < 2147483647, "too many beams for the grid");
-    const int64_t runs = T_ > 4 ? kad_cdiv(T_, kConvRun) : 1;
-    KAD_REQUIRE(runs < 65536, "too many tokens for the grid");
+    const int run = (int)std::max<int64_t>(kConvRun, kad_cdiv(T_, 65535));
+    const int64_t runs = T_ > 4 ? kad_cdiv(T_, run) : 1;
     const dim3 grid((unsigned)(B * nbg), (unsigned)groups, (unsigned)runs);
 #define KAD_CONV_VEC(TTV)                                                                       \
   hipLaunchKernelGGL((conv_suffix_vec<T, TTV>), grid, dim3(256), 0, s, (const T*)x, sx_n, sx_t, \
                      (const T*)state, ss_b, ss_c, ss_t, history, (const T*)w, (T*)out, so_n,    \
-                     so_t, W, C, T_, nbg, beams, silu)
+                     so_t, W, C, T_, nbg, beams, run, silu)
     switch (T_) {
       case 1: KAD_CONV_VEC(1); break;
       case 2: KAD_CONV_VEC(2); break;

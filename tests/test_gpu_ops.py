@@ -261,6 +261,26 @@ def test_conv_word_kernels_equal_the_scalar_one(device, dtype, B, W, C, T, histo
     assert torch.equal(ops.causal_conv1d(x, st, w, beam_width=W, activation=None), linear)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_conv_of_more_runs_than_a_grid_holds(device, dtype):
+    """A token-major suffix past 65,535 runs of 16 tokens: its first and last
+    thousand tokens are those of calls over them alone (the last with the three
+    before as its prefix taps)."""
+    C, T, n = 8, 65535 * 16 + 17, 1000
+    g = torch.Generator(device=device).manual_seed(2)
+    x = torch.randn(1, T, C, generator=g, device=device).to(dtype).transpose(1, 2)
+    st = torch.randn(1, C, 3, generator=g, device=device).to(dtype)
+    w = torch.randn(C, 4, generator=g, device=device).to(dtype)
+    got = ops.causal_conv1d(x, st, w)
+
+    def rows(t):
+        return t.transpose(1, 2).contiguous().transpose(1, 2)
+
+    assert torch.equal(got[..., :n], ops.causal_conv1d(rows(x[..., :n]), st, w))
+    taps = x[..., T - n - 3:T - n].contiguous()
+    assert torch.equal(got[..., T - n:], ops.causal_conv1d(rows(x[..., T - n:]), taps, w))
+
+
 def test_conv_golden_fixture(device):
     f = load_npz("ops_bf16.npz")
     x, st, w = (bf16_from_bits(f[n]) for n in ("conv_x", "conv_state", "conv_w"))
