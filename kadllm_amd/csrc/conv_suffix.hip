@@ -467,9 +467,14 @@ int launch_typed(const void* x, int64_t sx_n, int64_t sx_c, int64_t sx_t, const 
   const bool words = width == 4 && bias == nullptr && C % VE == 0 && sx_n % VE == 0 &&
                      so_n % VE == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
                      ((uintptr_t)w % 16) == 0;
+  // fp16's IEEE SiLU eight times a thread is its time, so below 8 M elements of
+  // token-major rows more threads of one channel each take less (8 x 50 beams of
+  // 6,144 channels, 1 / 2 tokens 17.4 / 19.0 us in words, 14.9 / 16.6; 4 22.2 both)
+  const bool scalar16 = Elem<T>::code == KAD_DTYPE_F16 && T_ <= 4 &&
+                        (int64_t)B * W * C * T_ < (8 << 20);
   // token-major rows (of one token both layouts are that)
   const bool vec = words && sx_c == 1 && so_c == 1 &&
-                   (T_ == 1 || (sx_t % VE == 0 && so_t % VE == 0));
+                   (T_ == 1 || (sx_t % VE == 0 && so_t % VE == 0)) && !scalar16;
   // [BW, C, T] with each beam's C * T block contiguous (the reference's layout)
   const bool ct = words && T_ <= 4 && sx_t == 1 && sx_c == T_ && so_t == 1 && so_c == T_;
   const int groups = (int)kad_cdiv(C / VE, 256);

@@ -241,6 +241,7 @@ def test_conv_reference_layout_equals_token_major(device, T, history):
 @pytest.mark.parametrize("B,W,C,T,history", [
     (2, 1, 8, 1, 4), (3, 13, 776, 2, 3), (1, 9, 2056, 3, 4), (2, 17, 520, 4, 6),
     (2, 3, 512, 5, 4), (1, 2, 264, 16, 3), (2, 1, 768, 33, 4), (1, 1, 6144, 50, 3),
+    (1, 350, 6144, 4, 4),   # fp16 token-major rows past the scalar kernel's range
 ])
 def test_conv_word_kernels_equal_the_scalar_one(device, dtype, B, W, C, T, history):
     """Both 16-byte-word kernels, in both layouts and of every type, against the
