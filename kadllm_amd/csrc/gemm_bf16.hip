@@ -1865,6 +1865,11 @@ int pick(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, void* 
       // many columns and few rows (the vocabulary head): 256-row tiles would be
       // half empty (64 rows 111 against 170 us, 128 rows 124 against 137)
       cfg = CFG_128x128_X16;
+    else if (M <= 128)
+      // the same for outputs of no whole 16-byte words (a head of odd size), in
+      // tiles with element stores (70,001 x 1,024: 17 rows 67 us in 256-row
+      // tiles, 26 here, 64 rows 69 and 31; 100 rows 70 and 39)
+      cfg = M <= 64 ? CFG_RING + RING_64x64 : CFG_128x128;
     else if (N <= 32)
       // more rows than a 128-row ring tile a CU covers (32,768: 16.0 us there
       // against 16.2 for whole-K waves): whole-K waves of 32 rows, one barrier

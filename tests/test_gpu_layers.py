@@ -400,6 +400,28 @@ def test_gemm_ring_tiles_agree(device, M, N, K, epi):
             assert torch.equal(cv, outs[2]), f"config {cfg} differs from config 2"
 
 
+@pytest.mark.parametrize("epi", [layers.EPI_STORE, layers.EPI_RESIDUAL])
+@pytest.mark.parametrize("M", [17, 64, 65, 128, 129])
+@pytest.mark.parametrize("N", [33001, 66003])
+def test_gemm_few_rows_to_an_odd_number_of_columns(device, M, N, epi):
+    """The automatic choice for outputs that no 16-byte store suits (a vocabulary
+    head of odd size) equals configuration 2 bit for bit."""
+    from kadllm_amd import _lib
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.randn(M, 192, generator=g).bfloat16().to(device)
+    w = (torch.randn(N, 192, generator=g) * 0.05).bfloat16().to(device)
+    x = torch.randn(M, N, generator=g).bfloat16().to(device)
+    outs = []
+    for cfg in (2, 0):
+        c = x.clone()
+        res = epi == layers.EPI_RESIDUAL
+        _lib.call("kad_gemm_bf16_tiled", _lib.ptr(a), 192, _lib.ptr(w), 192, _lib.ptr(c), N,
+                  _lib.ptr(c) if res else None, N if res else 0, M, N, 192, epi, cfg,
+                  _lib.stream_of(a))
+        outs.append(c)
+    assert torch.equal(*outs)
+
+
 @pytest.mark.parametrize("cfg,K,epi", [(32, 64, layers.EPI_STORE), (35, 192, layers.EPI_STORE),
                                        (32, 128, layers.EPI_SWIGLU)])
 def test_gemm_ring_tiles_reject(device, cfg, K, epi):
