@@ -368,9 +368,10 @@ __device__ __forceinline__ float unorder32(uint32_t u) {
 // maxima, which too few words had, and exact passes; 277 here.)  bf16 rows are ranked by logit; of fp32 and fp16 ones,
 // whose logits may differ and their fp32 keys not, the keys are ranked, and the
 // K-th must exceed the threshold's own key, below which nothing was gathered.
-// NT: 1,024 threads where the rows number at most two per CU (one row on a CU
-// is bound by the loads its waves keep in flight: 8 rows of 248,320 bf16
-// logits 96 -> 35 us), else 256 (2,048 rows 272 -> 246 us, 4.1 TB/s; of fp32, by
+// NT: 1,024 threads where the rows number at most one per CU, of long rows two
+// (one row on a CU is bound by the loads its waves keep in flight: 8 rows of
+// 248,320 bf16 logits 96 -> 35 us; 512 rows of 30,000 26 us with 256 threads and
+// 31 with 1,024, of 248,320 77 and 61), else 256 (2,048 rows 272 -> 246 us, 4.1 TB/s; of fp32, by
 // six passes before, 7.3 ms -> 0.40).
 template <typename T, int CAP, bool MASKED, int NT>
 __global__ __launch_bounds__(NT) void row_select_kernel(
@@ -1333,7 +1334,7 @@ int launch_row_select(const void* logits, int logits_dtype, int64_t ld, const vo
                        (logits_dtype == KAD_DTYPE_F32 ? 4 : 8);
   const int rank = (int)std::ceil(words * (1.0 - std::exp(-samples / words)));
   const bool small = 2 * (int64_t)K + 256 <= kCandCapSmall / 2;
-  const bool few = rows <= 512;
+  const bool few = rows <= 256 || (rows <= 512 && V > 65536);
 #define KAD_ROW_SELECT(T, CAP, MASKED, NT)                                                      \
   hipLaunchKernelGGL((row_select_kernel<T, CAP, MASKED, NT>), dim3(rows), dim3(NT), 0, s,       \
                      (const T*)logits, ld, (const uint8_t*)mask, ld_mask, parent_scores, Wp, V, \
