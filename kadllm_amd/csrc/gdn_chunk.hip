@@ -811,8 +811,9 @@ __device__ __forceinline__ bf16x8 plane_pair(const uint32_t (&a)[2], const uint3
 }
 
 // an A fragment of one step in the lower half of the lanes and of the next in the
-// upper -> each in both halves (both planes of a step meet the same A); half the
-// LDS reads of loading them so
+// upper -> each in both halves (both planes of a step meet the same A).  For q and
+// k that is quicker than reading each so from LDS (4 x 16 heads of 1,000 tokens
+// 108 us against 111), for the k^T of the state update it is not (110).
 __device__ __forceinline__ void both_halves(const bf16x8& f, bf16x8 (&out)[2]) {
   const u32x4 w = __builtin_bit_cast(u32x4, f);
   u32x4 a, b;
@@ -1019,23 +1020,20 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk_scan16(
 #pragma unroll
       for (int e = 0; e < 4; ++e) S[kt][e] *= egl;
 #pragma unroll
-      for (int s = 0; s < 4; s += 2) {
-        // k^T of tokens (s + upper)*16 ..: lane 4 e + m of a 16-lane group
-        // addresses token e of its four, features 4 m .. +3 (see kt_frag)
+      for (int s = 0; s < 4; ++s) {
+        // k^T, both planes against the same 16 tokens: lane 4 e + m of a 16-lane
+        // group addresses token e of its four, features 4 m .. +3 (see kt_frag)
         tr_v4s_t part[2];
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-          const bf16_t* p = kb + ((s + upper) * 16 + r * 8 + half * 4 + (c >> 2)) * LDK + kt * 16 +
-                            (c & 3) * 4;
+          const bf16_t* p =
+              kb + (s * 16 + r * 8 + half * 4 + (c >> 2)) * LDK + kt * 16 + (c & 3) * 4;
           part[r] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
               (__attribute__((address_space(3))) tr_v4s_t*)p);
         }
         const u32x2 lo = __builtin_bit_cast(u32x2, part[0]);
         const u32x2 up = __builtin_bit_cast(u32x2, part[1]);
-        bf16x8 a[2];
-        both_halves(as_bf16x8(u32x4{lo[0], lo[1], up[0], up[1]}), a);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) S[kt] = mfma16x16x32(a[u], w[s + u], S[kt]);
+        S[kt] = mfma16x16x32(as_bf16x8(u32x4{lo[0], lo[1], up[0], up[1]}), w[s], S[kt]);
       }
     }
     __syncthreads();
@@ -1091,8 +1089,8 @@ int launch_chunk(const void* q, const void* k, const void* v, int64_t ld_qk, int
   if (const int rc = kad_launch_status("gdn_chunk_scan16")) return rc
   // 64-column workgroups while they number at most one per CU, of 64-wide heads
   // two (16 heads of 1,024 tokens, us with the prep, wide scan against this one:
-  // 128-wide 1 sequence 120 / 100, 4 128 / 109, 8 146 / 129, 12 170 / 180;
-  // 64-wide 16 189 / 162, 32 of 300 tokens 100 / 90)
+  // 128-wide 1 sequence 120 / 98, 4 128 / 108, 8 146 / 128, 12 170 / 180;
+  // 64-wide 16 189 / 161, 32 of 300 tokens 100 / 89)
   if ((int64_t)N * HV * (V / kCols16) <= (V == 64 ? 512 : 256)) {
     if (hf_norm) {
       KAD_CHUNK16(true);
