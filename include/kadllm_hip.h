@@ -178,7 +178,8 @@ int kad_gemm_bf16_conv(const void* A, int64_t lda, const void* W, int64_t ldw, v
                        kad_stream_t stream);
 
 /* Same with an explicit tile configuration, the forms the automatic choice
- * picks from (0 = automatic choice as kad_gemm_bf16; 1 = 32x256 with 4 waves;
+ * picks from (0 = automatic choice as kad_gemm_bf16, which does not reach 1 and
+ * 12; 1 = 32x256 with 4 waves;
  * 2 = 128x128 with 4 waves; 5 = 256x256 with 8 waves; 11 = 64x32 with 2
  * waves, no SwiGLU epilogue; 12 = 32x64 with 2 waves, no SwiGLU epilogue;
  * 13 = outputs of at most 32 columns, one wave per 32 rows over the whole

@@ -16,7 +16,7 @@
 //
 // Stage 2, kad_beam_merge_select (one workgroup per request): a sampled
 // threshold keeps a few times W of the request's Wp*K candidates, which are
-// sorted by (key desc, index asc); wide or heavily tied levels take an 8-bit
+// sorted by (key desc, index asc); small, wide or heavily tied levels take an 8-bit
 // radix select over the keys for the W-th key, a second over flat indices for
 // its ties (lower flat index first), and a bitonic sort of the W winners in
 // LDS, for W up to 16384.  kad_beam_merge_select_wide serves wider levels (the reference's

@@ -52,8 +52,9 @@ __device__ __forceinline__ float sigmoid_exact(float x) { return 1.0f / (1.0f + 
 // distinct bank groups.  One wave per SIMD has nothing to hide its other
 // instructions behind but its own MFMAs, so LDS reads and loads are spread
 // between them and slot indexes are constants.  1,000 x 7,168 x 1,024 with
-// SwiGLU 275 -> 126 us (116 TFLOP/s), 1,000 x 1,024 x 3,584 399 -> 65 us (113);
-// at 4,096 rows 128 TFLOP/s of the 150 that MFMAs alone reach.
+// SwiGLU 275 -> 117 us (126 TFLOP/s, inputs in the caches), 1,000 x 1,024 x 3,584
+// 399 -> 60 us (123); at 4,096 rows 128 to 139 TFLOP/s of the 150 that MFMAs alone
+// reach.
 constexpr int kSlots = 4, kSlice = 64 * 32;  // floats of one operand's slice
 
 __device__ __forceinline__ int slices_per_block(int slices) { return (slices + 7) / 8; }

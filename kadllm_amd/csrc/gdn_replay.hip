@@ -885,8 +885,9 @@ void gdn_replay_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restric
 // Beams per workgroup, whole groups of 16, at most `most`: a request's beams in
 // one workgroup pay the state prologue once per (request, head) -- two-token
 // suffixes of 32 requests x 256 beams ran 7% faster so than in two of 128 --
-// unless that leaves the CUs with fewer than two workgroups each (16 heads: 8
-// requests x 50 beams, two tokens 17.6 -> 9.9 us; 1 x 256, one token 21 -> 7.4).
+// unless that leaves the CUs with fewer than two workgroups each (kernel times
+// with inputs in the caches, 16 heads: 8 requests x 50 beams, two tokens, by the
+// register kernel 18.0, here 10.5 us; 1 x 256, one token 20.8 -> 5.1).
 int beams_per_block(int64_t heads, int W, int most) {
   int bpb = W < most ? (W + 15) / 16 * 16 : (W > most ? 128 : most);
   while (bpb > 16 && heads * kad_cdiv(W, bpb) < 512) bpb = (bpb / 2 + 15) / 16 * 16;

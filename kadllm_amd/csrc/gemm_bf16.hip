@@ -1871,9 +1871,10 @@ int pick(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, void* 
       // tiles, 26 here, 64 rows 69 and 31; 100 rows 70 and 39)
       cfg = M <= 64 ? CFG_RING + RING_64x64 : CFG_128x128;
     else if (N <= 32)
-      // more rows than a 128-row ring tile a CU covers (32,768: 16.0 us there
-      // against 16.2 for whole-K waves): whole-K waves of 32 rows, one barrier
-      // in all; 64x32 tiles where K does not suit them
+      // more rows than a 128-row ring tile a CU covers (32 columns, K 1,024: at
+      // 8,192 rows 5.0 us there against 8.0 for whole-K waves, 16,384 6.9 and
+      // 11.8, 32,768 12.4 and 13.7): whole-K waves of 32 rows, one barrier in
+      // all; 64x32 tiles where K does not suit them
       cfg = n32_ok(A, lda, W, ldw, N, K, EPI) ? CFG_N32 : CFG_64x32;
     else if (tiles256 >= 256 && !vec)
       cfg = CFG_256x256_8W;
@@ -1929,6 +1930,7 @@ int pick(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, void* 
     }
   }
   switch (cfg) {
+    // 32x256 and 32x64 by their numbers only
     case CFG_32x256: return launch<32, 256, 1, 4, EPI>(A, lda, W, ldw, C, ldc, R, ldr, M, N, K, s);
     case CFG_32x64:
       if (EPI == KAD_EPI_SWIGLU) KAD_UNSUPPORTED("tile configuration 12 has no SwiGLU epilogue");

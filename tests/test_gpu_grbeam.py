@@ -216,8 +216,8 @@ def test_prefill_chunk_gated_equals_chunk_then_norm(device, L, K):
 @pytest.mark.parametrize("K,V,T", [(128, 128, 1), (128, 128, 130), (64, 128, 70), (128, 64, 64),
                                    (64, 64, 65)])
 def test_chunk_scans_match_oracle(device, N, HV, K, V, T):
-    """Both scans (16 columns a wave while 64-column workgroups number at most
-    two per CU, 32 beyond) against the token-by-token rule, with and without an
+    """Both scans (16 columns a wave while 64-column workgroups number at most one
+    per CU, two of 64-wide heads, 32 beyond) against the token-by-token rule, with and without an
     initial state, chunks whole and partial; the gated form, which the wide scan
     fuses and the narrow one launches, equals chunk then norm bit for bit."""
     H = 2
