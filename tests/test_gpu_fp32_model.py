@@ -54,13 +54,12 @@ def test_gemm_f32_matches_torch(device, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [
     (33, 64 * 72, 32), (100, 64 * 36 + 4, 64), (64, 64 * 80, 96), (257, 1088, 128),
-    (1000, 1024, 160), (129, 2304, 288),                     # 64 x 64 tiles, 1 .. 9 slices
+    (1000, 1024, 160), (129, 2304, 288),            # 64 x 64 tiles, staged and in the ring
     (256, 1024, 64), (300, 200, 36), (17, 96, 260), (16, 128, 31), (5, 33, 1), (700, 640, 33),
 ])
 def test_gemm_f32_kernels_at_their_edges(device, M, N, K):
-    """Tile and split kernels: partial tiles, every remainder of the slice ring,
-    K short of a slice and rows that are not 16-byte aligned.  Sums of at most
-    288 products of unit by 0.05: 1e-4."""
+    """Tile and split kernels: partial tiles, K short of a slice and rows that are
+    not 16-byte aligned.  Sums of at most 288 products of unit by 0.05: 1e-4."""
     g = torch.Generator().manual_seed(M + N + K)
     a = torch.randn(M, K + 3, generator=g)[:, :K] if K % 2 else torch.randn(M, K, generator=g)
     w = torch.randn(N, K, generator=g) * 0.05
@@ -84,11 +83,13 @@ def test_gemm_f32_kernels_at_their_edges(device, M, N, K):
     (300, 1200, 1000, 0, 0), (257, 1088, 68, 0, 4), (130, 2304, 1001, 0, 0), (129, 2304, 1, 0, 0),
     (700, 640, 4, 0, 0), (300, 1200, 288, 1, 0), (200, 1500, 257, 0, 3), (64, 64 * 80, 31, 0, 33),
     (300, 1200, 64, 0, 0), (300, 1217, 256, 1, 0), (65, 64 * 37, 131, 0, 1),
+    (300, 1200, 192, 0, 0), (300, 1200, 224, 0, 0), (300, 1200, 180, 0, 0), (300, 1200, 200, 0, 0),
+    (300, 1200, 300, 0, 1), (300, 1200, 333, 0, 0),
 ])
 def test_gemm_f32_tiles_take_any_inner_size(device, M, N, K, offset, pad):
     """The 64 x 64 tiles, in the ring and staged (short K), where K ends inside a
-    slice and where rows are not 16-byte aligned (a start ``offset`` elements in, rows ``pad`` apart): NaNs lie right
-    behind every row and both matrices.  Sums of at most 1,001 products of unit by
+    slice and where rows are not 16-byte aligned (a start ``offset`` elements in, rows ``pad`` apart), over every
+    remainder of the ring: NaNs lie right behind every row and both matrices.  Sums of at most 1,001 products of unit by
     0.05: 2e-4."""
     g = torch.Generator().manual_seed(M + N + K)
 
